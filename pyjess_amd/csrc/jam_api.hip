@@ -131,7 +131,7 @@ struct jam_context {
     int64_t front_cap = 0, done_cap = 0;
     int front_stride = 0, done_stride = 0;
     int join_grid[4] = {0, 0, 0, 0};   // resident workgroups of the join kernel <8/16/24/32>
-    int kd_grid[14] = {};           // resident workgroups of the kd kernels
+    int kd_grid[13] = {};           // resident workgroups of the kd kernels
     // the exact kd pass of each size tier runs on a stream of its own, from
     // the moment the tier's fast pass has listed its tied sets, beside the
     // fast passes of the other tiers (all streams at the default priority)
@@ -142,6 +142,7 @@ struct jam_context {
     hipStream_t kd_lds = nullptr;
     hipEvent_t kd_lds_done = nullptr;
     bool kd_pending = false;    // side-stream work of the last kd launch may still run
+    unsigned kd_used = 0;       // bit k: the last kd launch uses side stream k
     // sort of the complete matches
     DBuf s_key[2], s_perm[2], s_pkey[2];
     DBuf s_starts;   // per template size: complete matches of at most that many atoms
@@ -1188,11 +1189,10 @@ int32_t grow_events(jam_context *c, int64_t cap, int stride)
     return JAM_OK;
 }
 
-// clears the kd passes' per-tier counts and their error word
-__global__ void k_kd_setup(unsigned int *counts, int n, unsigned int *err)
+// clears the kd passes' per-tier counts
+__global__ void k_kd_setup(unsigned int *counts, int n)
 {
     if ((int)threadIdx.x < n) counts[threadIdx.x] = 0u;
-    if (threadIdx.x == 0) *err = 0u;
 }
 
 __global__ void k_items_any(DevPairs pr)
@@ -1263,24 +1263,34 @@ void launch_join(jam_context *c, int stride, hipStream_t s, const DevMols &dm, c
 }
 
 
-// Launches the kd passes over the candidate sets of `st`: the sets are
-// bucketed by size tier, then every tier gets its fast pass on `s` (every
-// set: <= 64 entries in one wave's registers, up to KD_BIG with one position
-// per thread, above KD_LDS_MAX in global scratch; a set with a tie at a split
-// point is listed instead of written) and, on the tier's side stream from the
-// end of that fast pass, the exact QuickSelect pass over the listed sets. Sets
-// of KD_BIG+1 ... KD_LDS_MAX entries skip the fast pass (at library sizes
-// 25-100% of them have a tie) and all go to the exact pass in LDS. With one
-// molecule (few sets, latency-bound) the 513-1024 and 257-512 tiers skip the
-// fast pass and run the exact pass on all their sets from the start: for a
-// handful of big sets it is the kd phase's longest chain, and the fast pass
-// would mostly give up on them (with 0.001 A coordinates a big set nearly
-// always has equal values at one of its n-1 split points). kd_joined[k] is
-// recorded at the end of tier k's passes; every set is written once all are.
-// Grids are upper bounds (the counts stay on the device); every kernel loops
-// over its own list.
+// Launches the kd passes over the candidate sets of `st`. Sets of up to
+// KD_LDS_MAX entries are mostly left to the exact QuickSelect pass alone: on
+// 0.001 A coordinates a set of a few hundred entries often has equal values at
+// one of its n-1 split points, and the exact pass costs no more than the sorts
+// of the fast pass (2,000 sets of 800 entries: 0.35 ms against 0.46 ms).
+//
+// One molecule (a few hundred sets, bound by the latency of the longest chain
+// of rounds and by launches): every set of up to KD_BIG entries in one launch
+// of 1,024-thread workgroups, one position per thread -- two of them per CU,
+// so all sets run at once -- and the larger ones beside it on side streams:
+// one of them where the molecule is too small for more than an odd set of
+// that size (KD_ONE_STREAM_ATOMS), three, by size, in larger ones.
+//
+// Several molecules: the sets are bucketed by size tier, and every tier gets
+// a stream of its own. Tiers 0 and 1 (<= 128 entries, mostly without ties)
+// get a fast pass on `s` and the exact pass over the sets that it lists;
+// tiers 2-4 the exact pass alone, two positions per thread above 256 entries
+// (throughput: 0.35 ms for 2,000 sets of 800 entries against 0.51 ms with one
+// position per thread, which is the faster form for a single set); tier 5 the
+// exact pass in LDS up to KD_LDS_MAX entries, and above that a fast and an
+// exact pass in global scratch.
+//
+// The passes of tier k end before kd_joined[k]; every set is written once
+// all are. Grids are upper bounds (the counts stay on the device); every
+// kernel loops over its own list. The caller has cleared *st.kd_err.
+constexpr int64_t KD_ONE_STREAM_ATOMS = 16384;
 int32_t launch_kd(jam_context *c, const DevMols &dm, const DevTpls &dt, const DevSets &st, hipStream_t s,
-                  bool one_molecule)
+                  bool one_molecule, int64_t n_atoms)
 {
     const int n_sets = st.n_sets;
     unsigned char *scr = c->kscr.as<unsigned char>();
@@ -1289,116 +1299,126 @@ int32_t launch_kd(jam_context *c, const DevMols &dm, const DevTpls &dt, const De
     unsigned int *nb = c->kd_count.as<unsigned int>();
     unsigned int *nt = nb + KD_TIERS;
     const size_t ns = (size_t)n_sets;
-    hipLaunchKernelGGL(k_kd_setup, dim3(1), dim3(64), 0, s, nb, 2 * KD_TIERS, st.kd_err);
-    hipLaunchKernelGGL(jam::k_kdbucket,
-                       dim3(std::max(1, std::min((n_sets + KD_BUCKET_SPAN - 1) / KD_BUCKET_SPAN, 1024))), dim3(256),
-                       0, s, st, bucket, nb);
-    HIP_TRY(hipGetLastError());
     if (c->kd_grid[0] == 0) {
         const int d = c->device;
         c->kd_grid[0] = resident_grid(jam::k_kdwave, JAM_WAVE, d);
         c->kd_grid[1] = resident_grid(jam::k_kdblock<128>, 128, d);
-        c->kd_grid[2] = resident_grid(jam::k_kdblock<256>, 256, d);
-        c->kd_grid[3] = resident_grid(jam::k_kdblock<512>, 512, d);
-        c->kd_grid[4] = resident_grid(jam::k_kdblock<1024>, 1024, d);
-        c->kd_grid[5] = resident_grid(jam::k_kdbig, KD_THREADS, d);
-        c->kd_grid[6] = resident_grid(jam::k_kdexact<64>, 64, d);
-        c->kd_grid[7] = resident_grid(jam::k_kdexact<128>, 128, d);
-        c->kd_grid[8] = resident_grid(jam::k_kdexact<256>, 256, d);
-        c->kd_grid[9] = resident_grid(jam::k_kdexact<512>, 512, d);
-        c->kd_grid[10] = resident_grid(jam::k_kdexact<1024>, 1024, d);
-        c->kd_grid[11] = resident_grid(jam::k_kdbig_exact, KD_EXACT_THREADS, d);
-        c->kd_grid[12] = resident_grid(jam::k_kdexact_lds<KD_LDS_SMALL_THREADS, 8>, KD_LDS_SMALL_THREADS, d);
-        c->kd_grid[13] = resident_grid(jam::k_kdexact_lds<KD_LDS_MAX / 8, 8>, KD_LDS_MAX / 8, d);
+        c->kd_grid[2] = resident_grid(jam::k_kdbig, KD_THREADS, d);
+        c->kd_grid[3] = resident_grid(jam::k_kdexact<64>, 64, d);
+        c->kd_grid[4] = resident_grid(jam::k_kdexact<128>, 128, d);
+        c->kd_grid[5] = resident_grid(jam::k_kdexact<256>, 256, d);
+        c->kd_grid[6] = resident_grid(jam::k_kdexact_lds<256, 2>, 256, d);
+        c->kd_grid[7] = resident_grid(jam::k_kdexact_lds<512, 2>, 512, d);
+        c->kd_grid[8] = resident_grid(jam::k_kdexact_lds<KD_BIG, 1>, KD_BIG, d);
+        c->kd_grid[9] = resident_grid(jam::k_kdexact_lds<1024, 2>, 1024, d);
+        c->kd_grid[10] = resident_grid(jam::k_kdexact_lds<1024, 4>, 1024, d);
+        c->kd_grid[11] = resident_grid(jam::k_kdexact_lds<KD_LDS_MAX / 8, 8>, KD_LDS_MAX / 8, d);
+        c->kd_grid[12] = resident_grid(jam::k_kdbig_exact, KD_EXACT_THREADS, d);
     }
     auto grid = [&](int k) { return dim3((unsigned)std::min(n_sets, c->kd_grid[k])); };
-    auto launch_fast = [&](int k, hipStream_t x) {
-        const size_t o = (size_t)k * ns;
-        switch (k) {
-        case 0:
-            hipLaunchKernelGGL(jam::k_kdwave, grid(0), dim3(JAM_WAVE), 0, x, dm, dt, st, bucket, nb, tied, nt);
-            break;
-        case 1:
-            hipLaunchKernelGGL((jam::k_kdblock<128>), grid(1), dim3(128), 0, x, dm, dt, st, bucket + o, nb + 1,
-                               tied + o, nt + 1);
-            break;
-        case 2:
-            hipLaunchKernelGGL((jam::k_kdblock<256>), grid(2), dim3(256), 0, x, dm, dt, st, bucket + o, nb + 2,
-                               tied + o, nt + 2);
-            break;
-        case 3:
-            hipLaunchKernelGGL((jam::k_kdblock<512>), grid(3), dim3(512), 0, x, dm, dt, st, bucket + o, nb + 3,
-                               tied + o, nt + 3);
-            break;
-        case 4:
-            hipLaunchKernelGGL((jam::k_kdblock<1024>), grid(4), dim3(1024), 0, x, dm, dt, st, bucket + o, nb + 4,
-                               tied + o, nt + 4);
-            break;
-        default:
-            hipLaunchKernelGGL(jam::k_kdbig, grid(5), dim3(KD_THREADS), 0, x, dm, dt, st, scr, bucket + o, nb + 5,
-                               tied + o, nt + 5, KD_LDS_MAX);
-            break;
-        }
+    // the LDS exact passes of tier 5 over `lst` (every set where there is none)
+    auto lds2 = [&](hipStream_t x, const int *lst, const unsigned int *lc) {
+        hipLaunchKernelGGL((jam::k_kdexact_lds<1024, 2>), grid(9), dim3(1024), 0, x, dm, dt, st, lst, lc, KD_BIG);
     };
-    // the exact pass of tier k over the sets its fast pass listed, or
-    // (`all`) over every set of the tier
-    auto launch_exact = [&](int k, hipStream_t x, bool all) {
-        const size_t o = (size_t)k * ns;
-        const int *lst = all ? bucket + o : tied + o;
-        const unsigned int *lc = all ? nb + k : nt + k;
-        switch (k) {
-        case 0:
-            hipLaunchKernelGGL((jam::k_kdexact<64>), grid(6), dim3(64), 0, x, dm, dt, st, lst, lc);
-            break;
-        case 1:
-            hipLaunchKernelGGL((jam::k_kdexact<128>), grid(7), dim3(128), 0, x, dm, dt, st, lst, lc);
-            break;
-        case 2:
-            hipLaunchKernelGGL((jam::k_kdexact<256>), grid(8), dim3(256), 0, x, dm, dt, st, lst, lc);
-            break;
-        case 3:
-            hipLaunchKernelGGL((jam::k_kdexact<512>), grid(9), dim3(512), 0, x, dm, dt, st, lst, lc);
-            break;
-        case 4:
-            hipLaunchKernelGGL((jam::k_kdexact<1024>), grid(10), dim3(1024), 0, x, dm, dt, st, lst, lc);
-            break;
-        default:
-            // every set of the tier of 8 * KD_LDS_SMALL_THREADS + 1 ...
-            // KD_LDS_MAX entries (most of them have a tie) in LDS (the
-            // smaller ones run on kd_lds), then the larger sets the fast
-            // pass listed in global scratch
-            hipLaunchKernelGGL((jam::k_kdexact_lds<KD_LDS_MAX / 8, 8>), grid(13), dim3(KD_LDS_MAX / 8), 0, x, dm, dt,
-                               st, bucket + o, nb + 5, KD_LDS_SMALL_THREADS * 8);
-            hipLaunchKernelGGL(jam::k_kdbig_exact, grid(11), dim3(KD_EXACT_THREADS), 0, x, dm, dt, st, scr, lst, lc,
-                               KD_LDS_MAX);
-            break;
-        }
+    auto lds4 = [&](hipStream_t x, const int *lst, const unsigned int *lc) {
+        hipLaunchKernelGGL((jam::k_kdexact_lds<1024, 4>), grid(10), dim3(1024), 0, x, dm, dt, st, lst, lc,
+                           KD_LDS_MAX / 4);
+    };
+    auto lds8 = [&](hipStream_t x, const int *lst, const unsigned int *lc) {
+        hipLaunchKernelGGL((jam::k_kdexact_lds<KD_LDS_MAX / 8, 8>), grid(11), dim3(KD_LDS_MAX / 8), 0, x, dm, dt, st,
+                           lst, lc, KD_LDS_MAX / 2);
+    };
+    auto big_exact = [&](hipStream_t x, const int *lst, const unsigned int *lc) {
+        hipLaunchKernelGGL(jam::k_kdbig_exact, grid(12), dim3(KD_EXACT_THREADS), 0, x, dm, dt, st, scr, lst, lc,
+                           KD_LDS_MAX);
     };
     c->kd_pending = true;
-    // largest tier first: its exact pass, the longest, starts earliest (with
-    // one molecule the exact-only tiers first: sets above 1,024 entries are
-    // rare there)
-    static const int by_size[KD_TIERS] = {5, 4, 3, 2, 1, 0};
-    static const int one_mol[KD_TIERS] = {4, 3, 5, 2, 1, 0};
-    static_assert(KD_TIERS == 6, "tier orders list six tiers");
-    for (int i = 0; i < KD_TIERS; i++) {
-        const int k = one_molecule ? one_mol[i] : by_size[i];
-        const bool all = one_molecule && (k == 3 || k == 4);
-        if (!all) launch_fast(k, s);
-        HIP_TRY(hipEventRecord(c->kd_fast[k], s));
-        HIP_TRY(hipStreamWaitEvent(c->kd_side[k], c->kd_fast[k], 0));
-        if (k == 5) {
-            HIP_TRY(hipStreamWaitEvent(c->kd_lds, c->kd_fast[k], 0));
-            hipLaunchKernelGGL((jam::k_kdexact_lds<KD_LDS_SMALL_THREADS, 8>), grid(12), dim3(KD_LDS_SMALL_THREADS), 0,
-                               c->kd_lds, dm, dt, st, bucket + (size_t)k * ns, nb + k, KD_BIG);
-            HIP_TRY(hipEventRecord(c->kd_lds_done, c->kd_lds));
+    c->kd_used = 0u;
+    // side stream k starts from here on `s`, and is waited for by kd_join
+    auto fork = [&](int k) -> hipError_t {
+        hipError_t e = hipEventRecord(c->kd_fast[k], s);
+        return e == hipSuccess ? hipStreamWaitEvent(c->kd_side[k], c->kd_fast[k], 0) : e;
+    };
+    auto joined = [&](int k) -> hipError_t {
+        c->kd_used |= 1u << k;
+        return hipEventRecord(c->kd_joined[k], c->kd_side[k]);
+    };
+    if (one_molecule) {
+        if (n_atoms > KD_BIG) {
+            const bool spread = n_atoms > KD_ONE_STREAM_ATOMS;
+            HIP_TRY(fork(5));
+            lds8(c->kd_side[5], nullptr, nullptr);
+            big_exact(c->kd_side[5], nullptr, nullptr);
+            if (spread) HIP_TRY(hipStreamWaitEvent(c->kd_side[4], c->kd_fast[5], 0));
+            lds4(c->kd_side[spread ? 4 : 5], nullptr, nullptr);
+            if (spread) HIP_TRY(hipStreamWaitEvent(c->kd_side[3], c->kd_fast[5], 0));
+            lds2(c->kd_side[spread ? 3 : 5], nullptr, nullptr);
+            HIP_TRY(joined(5));
+            if (spread) HIP_TRY(joined(4));
+            if (spread) HIP_TRY(joined(3));
         }
-        launch_exact(k, c->kd_side[k], all);
-        if (k == 5) HIP_TRY(hipStreamWaitEvent(c->kd_side[k], c->kd_lds_done, 0));
-        HIP_TRY(hipEventRecord(c->kd_joined[k], c->kd_side[k]));
+        hipLaunchKernelGGL((jam::k_kdexact_lds<KD_BIG, 1>), grid(8), dim3(KD_BIG), 0, s, dm, dt, st,
+                           (const int *)nullptr, (const unsigned int *)nullptr, 0);
+        HIP_TRY(hipGetLastError());
+        return JAM_OK;
+    }
+    hipLaunchKernelGGL(k_kd_setup, dim3(1), dim3(64), 0, s, nb, 2 * KD_TIERS);
+    hipLaunchKernelGGL(jam::k_kdbucket,
+                       dim3(std::max(1, std::min((n_sets + KD_BUCKET_SPAN - 1) / KD_BUCKET_SPAN, 1024))), dim3(256),
+                       0, s, st, bucket, nb);
+    HIP_TRY(hipGetLastError());
+    // largest tier first: its exact passes, the longest, start earliest
+    for (int k = KD_TIERS - 1; k >= 0; k--) {
+        const int *all = bucket + (size_t)k * ns;
+        int *lst = tied + (size_t)k * ns;
+        const unsigned int *na = nb + k;
+        unsigned int *nl = nt + k;
+        hipStream_t x = c->kd_side[k];
+        if (k == 5) {
+            // the smallest of the tier on kd_lds, beside the larger ones
+            hipLaunchKernelGGL(jam::k_kdbig, grid(2), dim3(KD_THREADS), 0, s, dm, dt, st, scr, all, na, lst, nl,
+                               KD_LDS_MAX);
+            HIP_TRY(fork(k));
+            HIP_TRY(hipStreamWaitEvent(c->kd_lds, c->kd_fast[k], 0));
+            lds2(c->kd_lds, all, na);
+            HIP_TRY(hipEventRecord(c->kd_lds_done, c->kd_lds));
+            lds8(x, all, na);
+            lds4(x, all, na);
+            big_exact(x, lst, nl);
+            HIP_TRY(hipStreamWaitEvent(x, c->kd_lds_done, 0));
+        } else if (k == 4) {
+            HIP_TRY(fork(k));
+            hipLaunchKernelGGL((jam::k_kdexact_lds<512, 2>), grid(7), dim3(512), 0, x, dm, dt, st, all, na, 0);
+        } else if (k == 3) {
+            HIP_TRY(fork(k));
+            hipLaunchKernelGGL((jam::k_kdexact_lds<256, 2>), grid(6), dim3(256), 0, x, dm, dt, st, all, na, 0);
+        } else if (k == 2) {
+            HIP_TRY(fork(k));
+            hipLaunchKernelGGL((jam::k_kdexact<256>), grid(5), dim3(256), 0, x, dm, dt, st, all, na);
+        } else if (k == 1) {
+            hipLaunchKernelGGL((jam::k_kdblock<128>), grid(1), dim3(128), 0, s, dm, dt, st, all, na, lst, nl);
+            HIP_TRY(fork(k));
+            hipLaunchKernelGGL((jam::k_kdexact<128>), grid(4), dim3(128), 0, x, dm, dt, st, lst, nl);
+        } else {
+            hipLaunchKernelGGL(jam::k_kdwave, grid(0), dim3(JAM_WAVE), 0, s, dm, dt, st, all, na, lst, nl);
+            HIP_TRY(fork(k));
+            hipLaunchKernelGGL((jam::k_kdexact<64>), grid(3), dim3(64), 0, x, dm, dt, st, lst, nl);
+        }
+        HIP_TRY(joined(k));
     }
     HIP_TRY(hipGetLastError());
     return JAM_OK;
+}
+
+// `s` waits for the side streams of the last launch_kd
+hipError_t kd_join(jam_context *c, hipStream_t s)
+{
+    for (int k = 0; k < KD_TIERS; k++) {
+        if (!((c->kd_used >> k) & 1u)) continue;
+        const hipError_t e = hipStreamWaitEvent(s, c->kd_joined[k], 0);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace
@@ -1511,7 +1531,7 @@ extern "C" int32_t jam_query(jam_context *c, const jam_templates *tp, const jam_
                            (long long *)(cnts + CNT_ITEMS));
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipEventRecord(c->ev[1], s));
-        if ((rc = launch_kd(c, dm, dt, st, s, M == 1)) != JAM_OK) {
+        if ((rc = launch_kd(c, dm, dt, st, s, M == 1, ms->n_atoms)) != JAM_OK) {
             drain_kd(c);
             return rc;
         }
@@ -1519,7 +1539,7 @@ extern "C" int32_t jam_query(jam_context *c, const jam_templates *tp, const jam_
         // order: set them up while the exact passes still run
         hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, cnts, (long long)CNT_TOTAL);
         hipLaunchKernelGGL(k_items_any, dim3(pair_blocks), dim3(256), 0, s, pr);
-        for (int k = 0; k < KD_TIERS; k++) HIP_TRY(hipStreamWaitEvent(s, c->kd_joined[k], 0));
+        HIP_TRY(kd_join(c, s));
         c->kd_pending = false;   // the rest of the query is ordered after every kd pass
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipEventRecord(c->ev[2], s));
@@ -2187,11 +2207,12 @@ extern "C" int32_t jam_kd_order(jam_context *c, const double *xyz, const int64_t
     st.total = (int64_t *)(cnts + CNT_TOTAL);
     st.maxcnt = (int *)(cnts + CNT_MAXCNT);
     st.kd_err = c->kd_count.as<unsigned int>() + 2 * KD_TIERS;
-    if ((rc = launch_kd(c, dm, dt, st, s, n_sets == 1)) != JAM_OK) {
+    hipLaunchKernelGGL(k_kd_setup, dim3(1), dim3(64), 0, s, st.kd_err, 1);
+    if ((rc = launch_kd(c, dm, dt, st, s, n_sets == 1, total)) != JAM_OK) {
         drain_kd(c);
         return rc;
     }
-    for (int k = 0; k < KD_TIERS; k++) HIP_TRY(hipStreamWaitEvent(s, c->kd_joined[k], 0));
+    HIP_TRY(kd_join(c, s));
     std::vector<int> kidx((size_t)total);
     unsigned int err = 0;
     HIP_TRY(hipMemcpyAsync(kidx.data(), st.kidx, sizeof(int) * (size_t)total, hipMemcpyDeviceToHost, s));

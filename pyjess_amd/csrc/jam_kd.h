@@ -20,26 +20,23 @@
 //          memberships alone: sort every axis once, then at level d cut each
 //          range of axis d%3 in half and stably partition the two other axes
 //          by side. Detects a tie across a split point and then gives up.
-//   exact  for the sets the fast path gave up on: all ranges of a tree level
-//          run their QuickSelect together, one partition round at a time,
-//          and each Lomuto partition is computed without its serial scan:
-//            * the "<= pivot" elements keep their order: a stable compaction;
-//            * the others move as a FIFO queue: each is pushed when scanned,
-//              and each "<=" element scanned after the first ">" one pops the
-//              front and pushes it back; push number t of such a re-push is
-//              the q-th pop, i.e. push number q < t. Pointer jumping resolves
-//              every push to its element. The final queue fills
-//              [l+k+1, r-1] from its second element on, its front goes to r,
-//              the pivot to l+k.
+//   exact  all ranges of a tree level run their QuickSelect together, one
+//          partition round at a time, and each Lomuto partition is computed
+//          without its serial scan: the "<= pivot" elements keep their order
+//          (a stable compaction), the others move as a FIFO queue (each is
+//          pushed when scanned, and each "<=" element scanned after the first
+//          ">" one pops the front and pushes it back), whose final contents
+//          are found by following each push back to the element it started
+//          as. Nearly as fast as the fast path's sorts, so only sets that
+//          seldom have a tie (up to 128 entries of many molecules, and those
+//          too large for LDS) try the fast path first.
 //
-// Sets are bucketed by size; sets of up to 64 entries run in one wave's
-// registers, up to KD_BIG entries with one position per thread (shuffles,
-// ballots and LDS exchanges), up to KD_LDS_MAX entries straight to the exact
-// pass with 8 positions per thread in LDS (most sets that large have a tie),
-// larger ones in global scratch. Every loop of the
-// exact pass whose length depends on the data has a bound that a correct
-// chain never reaches; a pass that reaches it sets st.kd_err and leaves the
-// set unwritten, and the query reports an error.
+// Fast path: sets of up to 64 entries in one wave's registers, up to KD_BIG
+// with one position per thread, above KD_LDS_MAX in global scratch. Exact
+// path: up to KD_LDS_MAX entries in LDS, larger ones in global scratch. Every
+// loop of an exact pass whose length depends on the data has a bound that a
+// correct run never reaches; a pass that reaches it sets st.kd_err, and the
+// query reports an error.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -457,512 +454,474 @@ __global__ void __launch_bounds__(NT) k_kdblock(DevMols ms, DevTpls tp, DevSets 
 }
 
 // ---------------------------------------------------------------------------
-// exact path, sets of at most NT entries (NT = 64 ... KD_BIG): one position
-// per thread. The arrangement, prefix counts and pushes live in LDS; every
-// thread keeps its own element, its range and the QuickSelect window of that
-// range in registers, and computes the window updates itself, so one
-// partition step costs three barriers plus the pointer-jumping rounds.
+// exact path, sets of at most KD_LDS_MAX entries
 //
-// One partition step of a window [lw, rw] (pivot moved to rw) in the
-// reference's order: the "<=" elements keep their order at the front; every
-// position from the first ">" element f on pushes once onto a queue, a ">"
-// element itself, a "<=" element the element it pops from the queue's front
-// (the ">" block rotating by one); the pivot follows the "<=" elements and the
-// queue's final contents fill the rest, its front at rw.
+// One partition step of a window [l, r] (pivot moved to r) in the reference's
+// order: the k "<=" elements keep their order at the front, the pivot goes to
+// pos = l + k. The ">" elements are a queue that lies in place behind the
+// "<=" ones and rotates by one whenever a "<=" element is scanned: after the
+// scan position q > pos holds what was pushed when q was scanned -- its own
+// element if that is a ">" one, else the queue's front of that moment, which
+// is what lies s positions earlier, s being the number of ">" elements before
+// q (the queue's length). Following q -> q - s until a ">" element is met
+// names the source of every position behind pos; the queue's front (position
+// pos) goes to r in the pivot's swap. Inside a run of "<=" elements s does not
+// change, so a run is left in one hop of a multiple of s; every hop then
+// passes a ">" element, s shrinks by at least one and a hop is at least s
+// long: at most about sqrt(2 * width) hops (and one per 64 positions, as runs
+// are looked at one flag word at a time).
+//
+// Windows of more than 64 positions take rounds of the whole workgroup: the
+// "<=" flags as one 64-bit word per 64 positions in LDS, prefix counts by
+// popcounts, two barriers a round. Windows of at most 64 positions, and from
+// the depth on where every range has at most 64 positions whole subtrees, are
+// finished by one wave each with its positions in lanes: no barrier, flags
+// and queue chains in one ballot word. What bounds it is the chain of
+// dependent rounds (18 of the workgroup and 50 of a wave for 1,000 entries, 40
+// and 70 for 4,000), each a few thousand cycles of dependent LDS reads and of
+// the VALU work of up to 16 waves. Against one round of the whole workgroup
+// per partition at all sizes, with the queues resolved by pointer jumping
+// through LDS (a barrier per jump): a set of 1,000 entries 224 -> 94 us, 4,000
+// entries 891 -> 442 us, 8,000 entries 1,370 -> 928 us; 2,000 sets of 800
+// entries 1,191 -> 353 us, 1,000 sets of 2,000 entries 1,606 -> 885 us.
 // ---------------------------------------------------------------------------
-
-// links of a pop chain followed per thread before the pointer jumping
-#ifndef KD_CHASE
-#define KD_CHASE 8
-#endif
 
 // ceil(log2(n)) for n >= 1
 __host__ __device__ constexpr int kd_log2_ceil(int n) { return n <= 1 ? 0 : 1 + kd_log2_ceil((n + 1) / 2); }
 
-// Bounds of the exact pass's data-dependent loops. A window of w elements
+// Bounds of the exact passes' data-dependent loops. A window of w elements
 // needs at most w partition rounds, a tree of n elements fewer than
-// n * (ceil(log2 n) + 1) in all; a pop chain has at most n links, so pointer
-// jumping (each round halves every open chain) ends within ceil(log2 n) + 1
-// rounds. Reaching a bound means a broken invariant: the pass stops and
-// reports it instead of looping.
+// n * (ceil(log2 n) + 1) in all; a chain of the queue has at most n links, and
+// pointer jumping (each round halves every open chain) ends within
+// ceil(log2 n) + 1 rounds. Reaching a bound means a broken invariant: the pass
+// stops and reports it instead of looping.
 #define KD_JUMP_BOUND(n) (kd_log2_ceil(n) + 2)
 #define KD_ROUND_BOUND(n) ((long long)(n) * (kd_log2_ceil(n) + 2) + 64)
 
-template <int NT>
-__global__ void __launch_bounds__(NT) k_kdexact(DevMols ms, DevTpls tp, DevSets st, const int *list,
-                                                const unsigned int *count)
+#if defined(__HIP_DEVICE_COMPILE__)
+#define KD_RCP(x) __builtin_amdgcn_rcpf(x)
+#else
+#define KD_RCP(x) (1.0f / (x))
+#endif
+
+// bits [0, x) of a word, x < 64
+__device__ static inline unsigned long long kd_below(int x) { return (1ull << x) - 1ull; }
+
+// Range i (of 2^d, in position order) of depth d of a tree of n elements: [lo, hi).
+__device__ static inline void kd_range(int n, int d, int i, int &lo, int &hi)
 {
-    constexpr int NW = NT / JAM_WAVE;
-    constexpr int JUMPS = KD_JUMP_BOUND(NT);
-    __shared__ double cc[3][NT];  // coordinates by element
-    __shared__ int xa[NT];        // arrangement: element at each position
-    __shared__ int xp1[NT];       // exclusive prefix counts of the "<=" flags
-    __shared__ int src[NT];       // queue pushes of the window starting at lw, from lw on
-    __shared__ int wf[NT];        // first ">" position of the window of the range starting here
-    __shared__ int wsum[NW], wact[NW];
-    const int t = threadIdx.x;
-    const int lane = lane_id();
-    const int wv = t / JAM_WAVE;
-    if (*st.total > st.cap) return;
-    const int cnt = (int)*count;
-    for (int q = blockIdx.x; q < cnt; q += gridDim.x) {
-        const int s = list[q];
-        const int n = st.cnt[s];
-        const int64_t off = st.off[s];
-        const int abase = ms.atom_off[s / tp.n_types];
-        const bool live = t < n;
-        if (live) {
-            const size_t g = (size_t)(abase + st.list[off + t]);
-            cc[0][t] = ms.xyz[3 * g + 0];
-            cc[1][t] = ms.xyz[3 * g + 1];
-            cc[2][t] = ms.xyz[3 * g + 2];
-            xa[t] = t;
-        }
-        __syncthreads();
-        int a = t;                          // element at position t
-        int R = 0, H = n;                   // range of position t
-        int lw = 0, rw = n >= 2 ? n - 1 : -1;  // its window; rw < 0: none
-        int hmax = n;                       // largest range at this depth
-        bool broken = false;                // a loop bound was reached (block-uniform)
-        const long long round_bound = KD_ROUND_BOUND(n);
-        long long rounds = 0;
-        for (int d = 0; hmax >= 2;) {
-            if (++rounds > round_bound) {
-                broken = true;
-                break;
-            }
-            const double *c = cc[d % 3];
-            const bool active = live && rw >= 0;
-            double pv = 0.0;
-            int piv = -1, er = 0;   // pivot position, and the element it takes in the swap
-            if (active) {
-                // pivot: median of three, swapped with the window's right end
-                const int mid = (lw + rw + 1) / 2;
-                const int el = xa[lw], em = xa[mid];
-                er = xa[rw];
-                const double kl = c[el], km = c[em], kr = c[er];
-                if ((kl > km) != (kl > kr)) piv = lw;
-                else if ((km < kl) != (km < kr)) piv = mid;
-                else piv = rw;
-                const int ep = piv == lw ? el : (piv == mid ? em : er);
-                pv = c[ep];
-                if (t == piv) a = er;
-                if (t == rw) a = ep;
-                if (t == R) wf[R] = rw;
-            }
-            const bool inwin = active && t >= lw && t < rw;
-            const bool le = inwin && c[a] <= pv;
-            const bool gt = inwin && !le;
-            const unsigned long long bal = ballot(le);
-            const unsigned long long gball = ballot(gt);
-            const unsigned long long aball = ballot(active);
-            if (lane == 0) {
-                wsum[wv] = __popcll(bal);
-                wact[wv] = aball != 0ull;
-            }
-            __syncthreads();
-            bool any = false;
-            for (int w = 0; w < NW; w++) any |= wact[w] != 0;
-            if (!any) {
-                // every selection of this depth is done: split the ranges at
-                // their medians and open the windows of the next depth
-                hmax -= hmax / 2;
-                if (live && H - R >= 2) {
-                    const int m = R + (H - R) / 2;
-                    if (t < m) H = m;
-                    else R = m;
-                }
-                lw = R;
-                rw = (live && H - R >= 2) ? H - 1 : -1;
-                d++;
-                __syncthreads();
-                continue;
-            }
-            int p1 = rank_below(bal);
-            for (int w = 0; w < wv; w++) p1 += wsum[w];
-            xp1[t] = p1;
-            if (gt) {
-                // the first ">" of its window among this wave's lanes
-                const int lo = max(lw - (t - lane), 0);
-                const unsigned long long below = gball & ((1ull << lane) - 1ull) & ~((1ull << lo) - 1ull);
-                if (below == 0ull) atomicMin(&wf[R], t);
-            }
-            __syncthreads();
-            int p1l = 0, p1r = 0, f = 0;
-            if (active) {
-                p1l = xp1[lw];
-                p1r = xp1[rw];
-                f = wf[R];
-            }
-            const int ones = p1 - p1l;        // "<=" elements before t in the window
-            const int k1 = p1r - p1l;         // "<=" elements of the window
-            const int m = (rw - lw) - k1;     // ">" elements
-            const int nrot = k1 - (f - lw);   // pops: "<=" elements after f
-            const int pushes = rw - f;
-            bool again = false;
-            if (inwin && t >= f) {
-                // push t - f; a "<=" element pushes what pop number
-                // r = ones - (f - lw) takes, which is push number r, made at
-                // position f + r: that position's element if it is a ">" one
-                // (its "<=" flag, read off the prefix counts, is 0), else
-                // what that position's own pop took, up to KD_CHASE links;
-                // a chain still open then is a link for the pointer jumping
-                if (!le) {
-                    src[lw + (t - f)] = a;
-                } else {
-                    int r = ones - (f - lw), q = f + r;
-                    bool found = xp1[q + 1] == xp1[q];
-                    for (int hop = 1; hop < KD_CHASE && !found; hop++) {
-                        r = (xp1[q] - p1l) - (f - lw);
-                        q = f + r;
-                        found = xp1[q + 1] == xp1[q];
-                    }
-                    if (found) {
-                        src[lw + (t - f)] = q == piv ? er : xa[q];
-                    } else {
-                        src[lw + (t - f)] = -(lw + r) - 1;
-                        again = true;
-                    }
-                }
-            }
-            // pointer jumping until every push names an element; each pop
-            // names a lower push, so the chains end within JUMPS rounds
-            for (int jumps = 0; __syncthreads_or(again); jumps++) {
-                if (jumps >= JUMPS) {
-                    broken = true;
-                    break;
-                }
-                again = false;
-                if (inwin && t - lw < pushes) {
-                    const int v = src[t];
-                    if (v < 0) {
-                        const int u = src[-v - 1];
-                        src[t] = u;
-                        again = u < 0;
-                    }
-                }
-            }
-            if (broken) break;
-            // scatter: "<=" elements in order, the pivot after them, the
-            // queue from its second element on, its front at the right end
-            if (active) {
-                if (t == rw) {
-                    xa[lw + k1] = a;
-                } else if (inwin) {
-                    if (le) xa[lw + ones] = a;
-                    const int j = t - lw;
-                    if (j < m) xa[j == 0 ? rw : lw + k1 + j] = src[lw + nrot + j];
-                }
-            }
-            __syncthreads();
-            if (live) a = xa[t];
-            if (active) {
-                // next window of the range's QuickSelect
-                const int pos = lw + k1;
-                const int k = R + (H - R) / 2;
-                int nl = lw, nr = rw;
-                if (pos == k) nr = -1;
-                else if (k < pos) nr = pos - 1;
-                else nl = pos + 1;
-                if (nr >= 0 && nl == nr) nr = -1;
-                lw = nl;
-                rw = nr;
-            }
-        }
-        __syncthreads();
-        if (broken) {
-            if (t == 0) atomicOr(st.kd_err, 1u);
-        } else {
-            // DFS order: position p holds element arrangement[n-1-p]
-            const int e = live ? xa[n - 1 - t] : 0;
-            kd_emit_lane(ms, st, s, n, off, abase, t, e);
-        }
-        __syncthreads();
+    lo = 0;
+    hi = n;
+    for (int b = d - 1; b >= 0; b--) {
+        const int m = lo + (hi - lo) / 2;
+        if ((i >> b) & 1) lo = m;
+        else hi = m;
     }
 }
 
-// ---------------------------------------------------------------------------
-// exact path, sets of (min_n, NT * P] entries: the partition step of
-// k_kdexact with P positions per thread, so that a set of a few thousand
-// entries stays in LDS. Wave w holds positions w * 64P ... (w + 1) * 64P - 1,
-// its lane l positions w * 64P + k * 64 + l (k < P): P slices of 64
-// consecutive positions, so that the lanes of a wave touch consecutive LDS
-// entries, and prefix counts within a wave come from ballots. Positions,
-// elements and prefix counts are 16-bit, and only the coordinate of the
-// current depth's axis is kept (reloaded from HBM at every depth): 18 bytes
-// per entry, 144 KB for 8,192 entries. A thread keeps the element, range and
-// window of each of its positions in registers; its positions in one range
-// share the range's pivot and prefix reads.
-// ---------------------------------------------------------------------------
+// The range of depth d that position p lies in.
+__device__ static inline int kd_range_of(int n, int d, int p)
+{
+    int lo = 0, hi = n, i = 0;
+    for (; d > 0; d--) {
+        const int m = lo + (hi - lo) / 2;
+        i = 2 * i + (p < m ? 0 : 1);
+        if (p < m) hi = m;
+        else lo = m;
+    }
+    return i;
+}
+
+// Hops out of the run of "<=" positions that ends at position q, given the
+// "<=" flags of q's word shifted up so that q's is the top bit (t) and the
+// number s > 0 of ">" positions before q: as many hops of s as the run's part
+// in this word takes. run / s by reciprocal: run < 64, and the half keeps the
+// quotient further from the integers than the reciprocal's error reaches.
+__device__ static inline int kd_hop(int q, unsigned long long t, int s)
+{
+    const int run = __clzll((long long)~t) - 1;
+    return q - s * (1 + (int)(((float)run + 0.5f) * KD_RCP((float)s)));
+}
+
+// The QuickSelects of the windows [lw, rw] of a wave, lane = position (rw < 0:
+// no window; lanes of one window agree on lw, rw and K, and are all there),
+// until each has its element K in place. id and v (the key) move along.
+__device__ static inline void kd_wave_select(int &id, double &v, int lw, int rw, int K)
+{
+    const int lane = lane_id();
+    // every round shortens every open window
+    for (int round = 0; round < JAM_WAVE; round++) {
+        const bool open = rw >= 0;
+        if (ballot(open) == 0ull) break;
+        const int l = open ? lw : lane, r = open ? rw : lane;
+        const int mid = (l + r + 1) >> 1;
+        // pivot: median of three, swapped with the window's right end
+        const double vl = __shfl(v, l, JAM_WAVE), vm = __shfl(v, mid, JAM_WAVE), vr = __shfl(v, r, JAM_WAVE);
+        int piv = r;
+        double pv = vr;
+        if ((vl > vm) != (vl > vr)) {
+            piv = l;
+            pv = vl;
+        } else if ((vm < vl) != (vm < vr)) {
+            piv = mid;
+            pv = vm;
+        }
+        const bool in = lane >= l && lane < r;
+        const bool le = in && (lane == piv ? vr : v) <= pv;
+        const unsigned long long bl = kd_below(l);
+        const unsigned long long L = ballot(le) & kd_below(r) & ~bl;
+        const unsigned long long G = ~(L | bl);   // ">" from l on
+        const int pos = l + __popcll(L);
+        const int ones = __popcll(L & kd_below(lane));
+        // the stable partition is a permutation of the lanes: every "<="
+        // lane tells its new place
+        const int part = push_int(lane, in ? (le ? l + ones : pos + (lane - l - ones)) : lane);
+        // the queue: one hop of every "<=" lane behind the first ">" one,
+        // then pointer doubling until every lane from pos on names a ">" one;
+        // lane r takes what pos names
+        const int before = lane - l - ones;       // ">" before this lane
+        int from = le && before > 0 ? kd_hop(lane, L << (JAM_WAVE - 1 - lane), before) : lane;
+        if (lane == r && open) from = pos;
+        for (int jump = 0; jump < KD_JUMP_BOUND(JAM_WAVE); jump++) {
+            from = __shfl(from, from, JAM_WAVE);
+            from = __shfl(from, from, JAM_WAVE);
+            if (ballot(open && lane > pos && lane <= r && ((G >> from) & 1ull) == 0ull) == 0ull) break;
+        }
+        int src = lane < pos ? part : (lane == pos ? r : from);
+        src = src == piv ? r : (src == r ? piv : src);
+        if (!(open && lane >= l && lane <= r)) src = lane;
+        id = __shfl(id, src, JAM_WAVE);
+        v = __shfl(v, src, JAM_WAVE);
+        if (open) {
+            // the next window of the QuickSelect
+            if (pos == K) rw = -1;
+            else if (K < pos) rw = pos - 1;
+            else lw = pos + 1;
+            if (rw >= 0 && lw == rw) rw = -1;
+        }
+    }
+}
+
+// The whole subtree of n <= 64 elements whose root splits axis d % 3: lane k
+// holds the element at position k (coordinates c0, c1, c2) and returns the
+// lane that held the element which ends there.
+__device__ static inline int kd_wave_tree(int n, int d, double c0, double c1, double c2)
+{
+    const int lane = lane_id();
+    int id = lane, R = 0, H = n;
+    for (int h = n; h >= 2; h -= h / 2, d++) {
+        const int ax = d % 3;
+        double v = __shfl(ax == 0 ? c0 : (ax == 1 ? c1 : c2), id, JAM_WAVE);
+        const bool open = lane < n && H - R >= 2;
+        const int K = R + (H - R) / 2;
+        kd_wave_select(id, v, R, open ? H - 1 : -1, K);
+        if (open) {
+            if (lane < K) H = K;
+            else R = K;
+        }
+    }
+    return id;
+}
 
 // largest set of the LDS exact pass (1,024 threads); larger ones run in
 // global scratch. Sets up to 8 * KD_LDS_SMALL_THREADS entries run with fewer
-// threads and half the LDS, two workgroups per CU.
+// threads and half the LDS, three workgroups per CU.
 #define KD_LDS_MAX 8192
 #define KD_LDS_SMALL_THREADS 512
-// a queue push that still names another push (src entries are 16-bit)
-#define KD_LINK 0x8000u
 
 template <int NT, int P>
-__global__ void __launch_bounds__(NT, 4) k_kdexact_lds(DevMols ms, DevTpls tp, DevSets st, const int *list,
-                                                    const unsigned int *count, int min_n)
+struct KdExactLds {
+    static constexpr int N = NT * P;
+    static constexpr int NW = NT / JAM_WAVE;
+    static constexpr int NWORDS = N / JAM_WAVE;
+    // all three axes of small sets; of larger ones the axis of the depth
+    // (loaded again at every depth)
+    static constexpr int AXES = N <= KD_BIG ? 3 : 1;
+    double cc[AXES][N];                   // coordinates by element
+    unsigned long long le[N / JAM_WAVE];  // "<=" flags by position
+    int pre[2][N / JAM_WAVE];             // "<=" flags of the words before (rounds take turns)
+    int wbig[NW];                         // whether a wave has a window of more than 64 positions
+    int winl[N / JAM_WAVE], winr[N / JAM_WAVE];   // windows of a depth's ranges
+    unsigned short xa[2][N];              // arrangement: element at each position (rounds take turns)
+};
+
+// Arranges set s (n <= NT * P entries) in the reference's leaf order; the
+// index of the xa buffer that holds it, or -1 when a loop bound was reached.
+// P positions per thread: wave w holds positions w * 64P ... (w + 1) * 64P - 1,
+// its lane l positions w * 64P + k * 64 + l (k < P), so that the lanes of a
+// wave touch consecutive LDS entries. A thread keeps the element, range and
+// window of each of its positions in registers; its positions in one range
+// share the range's pivot and prefix reads.
+template <int NT, int P>
+__device__ static inline int kd_exact_set(const DevMols &ms, const DevSets &st, KdExactLds<NT, P> &S, int n,
+                                          int64_t off, int abase)
 {
-    constexpr int N = NT * P;
-    constexpr int NW = NT / JAM_WAVE;
-    static_assert(N <= KD_LDS_MAX && N < (int)KD_LINK, "16-bit positions with a link flag");
-    __shared__ double cc[N];             // coordinate on the current axis, by element
-    __shared__ unsigned short xa[N];     // arrangement: element at each position
-    __shared__ unsigned short xp1[N];    // exclusive prefix counts of the "<=" flags
-    __shared__ unsigned short src[N];    // queue pushes: element, or KD_LINK | push slot
-    __shared__ int wf[N];                // first ">" position of the window of the range starting here
-    __shared__ int wsum[NW], wact[NW];
+    using Lds = KdExactLds<NT, P>;
+    constexpr int N = Lds::N, NW = Lds::NW;
     const int t = threadIdx.x;
     const int lane = lane_id();
     const int wv = t / JAM_WAVE;
     const int p0 = wv * JAM_WAVE * P + lane;   // position of slice k: p0 + k * JAM_WAVE
-    if (*st.total > st.cap) return;
-    const int cnt = (int)*count;
-    for (int qs = blockIdx.x; qs < cnt; qs += gridDim.x) {
-        const int s = list[qs];
-        const int n = st.cnt[s];
-        if (n <= min_n || n > N) continue;
-        const int64_t off = st.off[s];
-        const int abase = ms.atom_off[s / tp.n_types];
-        for (int e = t; e < n; e += NT) {
-            cc[e] = ms.xyz[3 * (size_t)(abase + st.list[off + e])];
-            xa[e] = (unsigned short)e;
+#pragma unroll
+    for (int k = 0; k < P; k++) {
+        const int e = t + k * NT;
+        if (e < n) {
+            const size_t g = (size_t)(abase + st.list[off + e]);
+#pragma unroll
+            for (int q = 0; q < Lds::AXES; q++) S.cc[q][e] = ms.xyz[3 * g + q];
+            S.xa[0][e] = (unsigned short)e;
         }
-        // per position: element, range [R, H), window [lw, rw] (rw < 0: none)
-        int a[P], R[P], H[P], lw[P], rw[P];
+    }
+    for (int i = t; i < 2 * Lds::NWORDS; i += NT) S.pre[i / Lds::NWORDS][i % Lds::NWORDS] = 0;
+    __syncthreads();
+    int cur = 0, par = 0, d = 0, hmax = n;   // hmax: the largest range of this depth
+    if (n > JAM_WAVE) {
+        // per position: element, range [R, H), window [lw, rw] (pairs of
+        // 16-bit halves; rw < 0: no window)
+        int a[P], range[P], win[P];
 #pragma unroll
         for (int k = 0; k < P; k++) {
             a[k] = p0 + k * JAM_WAVE;
-            R[k] = 0;
-            H[k] = n;
-            lw[k] = 0;
-            rw[k] = (n >= 2 && p0 + k * JAM_WAVE < n) ? n - 1 : -1;
+            range[k] = p0 + k * JAM_WAVE < n ? n << 16 : 0;
         }
-        __syncthreads();
-        int hmax = n;                      // largest range at this depth
-        bool broken = false;               // a loop bound was reached (block-uniform)
         const long long round_bound = KD_ROUND_BOUND(n);
-        const int jump_bound = KD_JUMP_BOUND(n);
         long long rounds = 0;
-        for (int d = 0; hmax >= 2;) {
-            if (++rounds > round_bound) {
-                broken = true;
-                break;
-            }
-            // pivot of each window: median of three, swapped with its right end
-            int piv[P], er[P];
-            unsigned lem = 0u, gtm = 0u;   // bit k: position k is "<=" / ">" in its window
-            bool act = false;
-            {
-                int cR = -1, c_piv = 0, c_er = 0;
-                double c_pv = 0.0;
+        for (; hmax > JAM_WAVE; d++, hmax -= hmax / 2) {
+            const double *c = S.cc[Lds::AXES == 3 ? d % 3 : 0];
 #pragma unroll
-                for (int k = 0; k < P; k++) {
-                    const int p = p0 + k * JAM_WAVE;
-                    piv[k] = -1;
-                    er[k] = 0;
-                    if (rw[k] < 0) continue;
-                    act = true;
-                    if (R[k] != cR) {
-                        const int l = lw[k], r = rw[k], mid = (l + r + 1) / 2;
-                        const int el = xa[l], em = xa[mid], e_r = xa[r];
-                        const double kl = cc[el], km = cc[em], kr = cc[e_r];
-                        if ((kl > km) != (kl > kr)) c_piv = l;
-                        else if ((km < kl) != (km < kr)) c_piv = mid;
-                        else c_piv = r;
-                        c_er = e_r;
-                        c_pv = c_piv == l ? kl : (c_piv == mid ? km : kr);
-                        cR = R[k];
-                    }
-                    piv[k] = c_piv;
-                    er[k] = c_er;
-                    if (p == c_piv) a[k] = c_er;
-                    if (p == rw[k]) a[k] = xa[c_piv];
-                    if (p == R[k]) wf[p] = rw[k];
-                    if (p >= lw[k] && p < rw[k]) {
-                        if (cc[a[k]] <= c_pv) lem |= 1u << k;
-                        else gtm |= 1u << k;
+            for (int k = 0; k < P; k++) win[k] = range[k] - (1 << 16);
+            // rounds of the workgroup while a window has more than 64 positions
+            for (;;) {
+                if (++rounds > round_bound) return -1;   // the same for every thread
+                const unsigned short *xc = S.xa[cur];
+                unsigned short *xn = S.xa[cur ^ 1];
+                // per position: the pivot of its window, the "<=" lanes before it
+                int pp[P];
+                unsigned lem = 0u;                       // bit k: position k is "<=" in its window
+                unsigned long long word = 0ull;
+                int wtot = 0, before = 0;
+                {
+                    int cR = -1, c_piv = 0, c_er = 0, c_ep = 0;
+                    double c_pv = 0.0;
+#pragma unroll
+                    for (int k = 0; k < P; k++) {
+                        const int p = p0 + k * JAM_WAVE;
+                        const int l = win[k] & 0xFFFF, r = win[k] >> 16;
+                        const bool big = r - l >= JAM_WAVE;
+                        pp[k] = 0;
+                        if (ballot(big) == 0ull) continue;   // no large window in this slice
+                        if (big && range[k] != cR) {
+                            // pivot: median of three, swapped with the window's right end
+                            const int mid = (l + r + 1) / 2;
+                            const int el = xc[l], em = xc[mid];
+                            c_er = xc[r];
+                            const double kl = c[el], km = c[em], kr = c[c_er];
+                            const bool at_l = (kl > km) != (kl > kr), at_m = (km < kl) != (km < kr);
+                            c_piv = at_l ? l : (at_m ? mid : r);
+                            c_ep = at_l ? el : (at_m ? em : c_er);
+                            c_pv = at_l ? kl : (at_m ? km : kr);
+                            cR = range[k];
+                        }
+                        if (big) a[k] = p == c_piv ? c_er : (p == r ? c_ep : a[k]);
+                        const bool le = big && p >= l && p < r && c[a[k]] <= c_pv;
+                        const unsigned long long bal = ballot(le);
+                        if (le) lem |= 1u << k;
+                        pp[k] = c_piv | rank_below(bal) << 16;
+                        if (lane == (wv * P + k) % JAM_WAVE) word = bal;
+                        if (lane > (wv * P + k) % JAM_WAVE) before += __popcll(bal);
+                        wtot += __popcll(bal);
                     }
                 }
-            }
-            // prefix counts of the "<=" flags: within the wave by slice
-            // ballots, across waves through LDS; whether any window is open
-            int p1[P];
-            int wtot = 0;
+                // the wave's flag words, and its counts added to the prefix
+                // counts of every later word
 #pragma unroll
-            for (int k = 0; k < P; k++) {
-                const unsigned long long bal = ballot((lem >> k) & 1u);
-                p1[k] = wtot + rank_below(bal);
-                wtot += __popcll(bal);
-            }
-            const unsigned long long aball = ballot(act);
-            if (lane == 0) {
-                wsum[wv] = wtot;
-                wact[wv] = aball != 0ull;
-            }
-            __syncthreads();
-            bool any = false;
-            int base = 0;
-            for (int w = 0; w < NW; w++) {
-                any |= wact[w] != 0;
-                if (w < wv) base += wsum[w];
-            }
-            if (!any) {
-                // every selection of this depth is done: split the ranges at
-                // their medians, open the windows of the next depth and load
-                // its axis (every read of cc at this depth came before the
-                // barrier above)
-                hmax -= hmax / 2;
-#pragma unroll
-                for (int k = 0; k < P; k++) {
-                    const bool live = p0 + k * JAM_WAVE < n;
-                    if (live && H[k] - R[k] >= 2) {
-                        const int m = R[k] + (H[k] - R[k]) / 2;
-                        if (p0 + k * JAM_WAVE < m) H[k] = m;
-                        else R[k] = m;
-                    }
-                    lw[k] = R[k];
-                    rw[k] = (live && H[k] - R[k] >= 2) ? H[k] - 1 : -1;
-                }
-                d++;
-                if (hmax >= 2) {
-                    const int ax = d % 3;
-                    for (int e = t; e < n; e += NT) cc[e] = ms.xyz[3 * (size_t)(abase + st.list[off + e]) + ax];
+                for (int i = lane; i < Lds::NWORDS; i += JAM_WAVE) {
+                    const bool own = i >= wv * P && i < wv * P + P;
+                    if (own) S.le[i] = word;
+                    const int add = own ? before : wtot;
+                    if (i >= wv * P && add != 0) atomicAdd(&S.pre[par][i], add);
                 }
                 __syncthreads();
-                continue;
-            }
-            // prefix counts; the first ">" of each window: per slice, the
-            // lowest ">" lane of the window among this wave's lanes
-            int ones[P];
+                for (int i = t; i < Lds::NWORDS; i += NT) S.pre[par ^ 1][i] = 0;
+                const int *pre = S.pre[par];
+                // "<=" flags before position q
+                auto prefix = [&](int q) {
+                    const int w = q / JAM_WAVE;
+                    return pre[w] + __popcll(S.le[w] & kd_below(q % JAM_WAVE));
+                };
+                bool big = false;
+                {
+                    int cR = -1, c_pl = 0, c_pos = 0;
 #pragma unroll
-            for (int k = 0; k < P; k++) {
-                const int p = p0 + k * JAM_WAVE;
-                ones[k] = base + p1[k];
-                if (p < n) xp1[p] = (unsigned short)ones[k];
-                const bool g = (gtm >> k) & 1u;
-                const unsigned long long gball = ballot(g);
-                if (g) {
-                    const int lo = max(lw[k] - (p - lane), 0);
-                    const unsigned long long below = gball & ((1ull << lane) - 1ull) & ~((1ull << lo) - 1ull);
-                    if (below == 0ull) atomicMin(&wf[R[k]], p);
-                }
-            }
-            __syncthreads();
-            // queue pushes (as in k_kdexact); ones[k] becomes the "<="
-            // elements before the position in its window
-            int k1v[P], fv[P];
-            bool again = false;
-            {
-                int cR = -1, c_p1l = 0, c_p1r = 0, c_f = 0;
-#pragma unroll
-                for (int k = 0; k < P; k++) {
-                    const int p = p0 + k * JAM_WAVE;
-                    k1v[k] = 0;
-                    fv[k] = 0;
-                    if (rw[k] < 0) continue;
-                    if (R[k] != cR) {
-                        c_p1l = xp1[lw[k]];
-                        c_p1r = xp1[rw[k]];
-                        c_f = wf[R[k]];
-                        cR = R[k];
-                    }
-                    const int l = lw[k], r = rw[k], f = c_f;
-                    ones[k] -= c_p1l;
-                    k1v[k] = c_p1r - c_p1l;
-                    fv[k] = f;
-                    if (p >= l && p < r && p >= f) {
-                        if (!((lem >> k) & 1u)) {
-                            src[l + (p - f)] = (unsigned short)a[k];
-                        } else {
-                            // pop number rr takes push number rr, made at f + rr
-                            int rr = ones[k] - (f - l), q = f + rr;
-                            bool found = xp1[q + 1] == xp1[q];
-                            for (int hop = 1; hop < KD_CHASE && !found; hop++) {
-                                rr = (xp1[q] - c_p1l) - (f - l);
-                                q = f + rr;
-                                found = xp1[q + 1] == xp1[q];
-                            }
-                            if (found) {
-                                src[l + (p - f)] = (unsigned short)(q == piv[k] ? er[k] : xa[q]);
-                            } else {
-                                src[l + (p - f)] = (unsigned short)(KD_LINK | (unsigned)(l + rr));
-                                again = true;
-                            }
+                    for (int k = 0; k < P; k++) {
+                        const int p = p0 + k * JAM_WAVE;
+                        int l = win[k] & 0xFFFF, r = win[k] >> 16;
+                        const bool mine = r - l >= JAM_WAVE;
+                        if (ballot(mine) == 0ull) {
+                            if (p < n) xn[p] = (unsigned short)a[k];
+                            continue;
                         }
+                        if (mine && range[k] != cR) {
+                            c_pl = prefix(l);
+                            c_pos = l + prefix(r) - c_pl;
+                            cR = range[k];
+                        }
+                        // "<=" elements in order, the pivot after them; the
+                        // places behind pos look for what the queue leaves there
+                        const bool in = mine && p >= l && p <= r, le = (lem >> k) & 1u;
+                        const int to = !in ? p : (p == r ? c_pos : l + pre[wv * P + k] + (pp[k] >> 16) - c_pl);
+                        if (in ? (le || p == r) : p < n) xn[to] = (unsigned short)a[k];
+                        const bool behind = in && p > c_pos;
+                        int q = behind && p == r ? c_pos : p;
+                        for (int hops = 0;; hops++) {
+                            const int w = q / JAM_WAVE;
+                            const unsigned long long t = S.le[w] << (JAM_WAVE - 1 - q % JAM_WAVE);
+                            const bool hop = behind && (long long)t < 0;
+                            if (ballot(hop) == 0ull) break;
+                            if (hops > N) {   // cannot happen: every hop goes towards the first ">" position
+                                atomicOr(st.kd_err, 1u);
+                                break;
+                            }
+                            const int s = q - (l - c_pl - 1) - (pre[w] + __popcll(t));   // ">" before q
+                            const int next = kd_hop(q, t, max(s, 1));
+                            q = hop ? next : q;
+                        }
+                        if (behind) xn[p] = xc[q == (pp[k] & 0xFFFF) ? r : q];
+                        if (!mine) continue;
+                        // the next window of the range's QuickSelect
+                        const int lo = range[k] & 0xFFFF, hi = range[k] >> 16, kk = lo + (hi - lo) / 2;
+                        if (c_pos == kk) r = -1;
+                        else if (kk < c_pos) r = c_pos - 1;
+                        else l = c_pos + 1;
+                        if (l == r) r = -1;
+                        win[k] = l | r << 16;
+                        big |= r - l >= JAM_WAVE;
                     }
                 }
-            }
-            // pointer jumping until every push names an element; each pop
-            // names a lower push, so the chains end within jump_bound rounds
-            for (int jumps = 0; __syncthreads_or(again); jumps++) {
-                if (jumps >= jump_bound) {
-                    broken = true;
-                    break;
-                }
-                again = false;
+                const unsigned long long bigs = ballot(big);
+                if (lane == 0) S.wbig[wv] = bigs != 0ull;
+                __syncthreads();
+                cur ^= 1;
+                par ^= 1;
 #pragma unroll
-                for (int k = 0; k < P; k++) {
-                    const int p = p0 + k * JAM_WAVE;
-                    if (rw[k] < 0 || p < lw[k] || p - lw[k] >= rw[k] - fv[k]) continue;
-                    const unsigned v = src[p];
-                    if (v & KD_LINK) {
-                        const unsigned u = src[v & (KD_LINK - 1u)];
-                        src[p] = (unsigned short)u;
-                        again |= (u & KD_LINK) != 0u;
-                    }
-                }
+                for (int k = 0; k < P; k++)
+                    if (p0 + k * JAM_WAVE < n) a[k] = xn[p0 + k * JAM_WAVE];
+                if (ballot(lane < NW && S.wbig[lane] != 0) == 0ull) break;
             }
-            if (broken) break;
-            // scatter: "<=" elements in order, the pivot after them, the
-            // queue from its second element on, its front at the right end
+            // the windows left, of at most 64 positions, one wave each
 #pragma unroll
-            for (int k = 0; k < P; k++) {
-                const int p = p0 + k * JAM_WAVE;
-                if (rw[k] < 0) continue;
-                const int l = lw[k], r = rw[k], k1 = k1v[k];
-                if (p == r) {
-                    xa[l + k1] = (unsigned short)a[k];
-                } else if (p >= l && p < r) {
-                    if ((lem >> k) & 1u) xa[l + ones[k]] = (unsigned short)a[k];
-                    const int j = p - l;
-                    const int m = (r - l) - k1;            // ">" elements
-                    const int nrot = k1 - (fv[k] - l);     // pops
-                    if (j < m) xa[j == 0 ? r : l + k1 + j] = src[l + nrot + j];
+            for (int k = 0; k < P; k++)
+                if (p0 + k * JAM_WAVE < n && p0 + k * JAM_WAVE == (range[k] & 0xFFFF)) {
+                    const int i = kd_range_of(n, d, range[k] & 0xFFFF);
+                    S.winl[i] = win[k] & 0xFFFF;
+                    S.winr[i] = win[k] >> 16;
                 }
+            __syncthreads();
+            for (int i = wv; i < (1 << d); i += NW) {
+                const int l = S.winl[i], r = S.winr[i];
+                if (r < 0) continue;   // the same for the whole wave
+                int lo, hi;
+                kd_range(n, d, i, lo, hi);
+                const int K = lo + (hi - lo) / 2;
+                const int p = l + lane;
+                const bool in = p <= r;
+                int e = in ? (int)S.xa[cur][p] : 0;
+                double v = in ? c[e] : 0.0;
+                kd_wave_select(e, v, 0, in ? r - l : -1, K - l);
+                if (in) S.xa[cur][p] = (unsigned short)e;
             }
             __syncthreads();
 #pragma unroll
             for (int k = 0; k < P; k++) {
-                if (p0 + k * JAM_WAVE < n) a[k] = xa[p0 + k * JAM_WAVE];
-                if (rw[k] < 0) continue;
-                // next window of the range's QuickSelect
-                const int pos = lw[k] + k1v[k];
-                const int kk = R[k] + (H[k] - R[k]) / 2;
-                int nl = lw[k], nr = rw[k];
-                if (pos == kk) nr = -1;
-                else if (kk < pos) nr = pos - 1;
-                else nl = pos + 1;
-                if (nr >= 0 && nl == nr) nr = -1;
-                lw[k] = nl;
-                rw[k] = nr;
+                const int p = p0 + k * JAM_WAVE;
+                if (p >= n) continue;
+                a[k] = S.xa[cur][p];
+                const int lo = range[k] & 0xFFFF, hi = range[k] >> 16, m = lo + (hi - lo) / 2;
+                range[k] = p < m ? (lo | m << 16) : (m | hi << 16);
+            }
+            if (Lds::AXES == 1 && hmax - hmax / 2 > JAM_WAVE) {
+                const int ax = (d + 1) % 3;
+#pragma unroll
+                for (int k = 0; k < P; k++)
+                    if (t + k * NT < n)
+                        S.cc[0][t + k * NT] = ms.xyz[3 * (size_t)(abase + st.list[off + t + k * NT]) + ax];
+                __syncthreads();
             }
         }
-        __syncthreads();
-        if (broken) {
-            if (t == 0) atomicOr(st.kd_err, 1u);
-        } else {
-            // DFS order: position p holds element arrangement[n-1-p]
-            for (int b0 = wv * JAM_WAVE; b0 < n; b0 += NT) {
-                const int p = b0 + lane;
-                kd_emit_lane(ms, st, s, n, off, abase, p, p < n ? (int)xa[n - 1 - p] : 0);
+    }
+    // ranges of at most 64 positions: one wave each
+    for (int i = wv; i < (1 << d); i += NW) {
+        int lo, hi;
+        kd_range(n, d, i, lo, hi);
+        const int m = hi - lo;
+        int e = 0;
+        double x[3] = {0.0, 0.0, 0.0};
+        if (lane < m) {
+            e = S.xa[cur][lo + lane];
+            if (Lds::AXES == 3) {
+#pragma unroll
+                for (int q = 0; q < 3; q++) x[q] = S.cc[q % Lds::AXES][e];
+            } else {
+                const size_t g = (size_t)(abase + st.list[off + e]);
+#pragma unroll
+                for (int q = 0; q < 3; q++) x[q] = ms.xyz[3 * g + q];
             }
         }
-        __syncthreads();
+        const int id = kd_wave_tree(m, d, x[0], x[1], x[2]);
+        e = shfl_int(e, id);
+        if (lane < m) S.xa[cur][lo + lane] = (unsigned short)e;
+    }
+    __syncthreads();
+    return cur;
+}
+
+template <int NT, int P>
+__device__ static inline void kd_exact_emit(const DevMols &ms, const DevSets &st, KdExactLds<NT, P> &S, int s, int n,
+                                            int64_t off, int abase)
+{
+    const int lane = lane_id();
+    const int cur = kd_exact_set<NT, P>(ms, st, S, n, off, abase);
+    if (cur < 0) {
+        if (threadIdx.x == 0) atomicOr(st.kd_err, 1u);
+    } else {
+        // DFS order: position p holds element arrangement[n-1-p]
+        for (int b0 = (threadIdx.x / JAM_WAVE) * JAM_WAVE; b0 < n; b0 += NT) {
+            const int p = b0 + lane;
+            kd_emit_lane(ms, st, s, n, off, abase, p, p < n ? (int)S.xa[cur][n - 1 - p] : 0);
+        }
+    }
+    __syncthreads();
+}
+
+// every set of `list` (at most NT entries each), one position per thread
+template <int NT>
+__global__ void __launch_bounds__(NT, 8) k_kdexact(DevMols ms, DevTpls tp, DevSets st, const int *list,
+                                                const unsigned int *count)
+{
+    __shared__ KdExactLds<NT, 1> S;
+    if (*st.total > st.cap) return;
+    const int cnt = (int)*count;
+    for (int q = blockIdx.x; q < cnt; q += gridDim.x) {
+        const int s = list[q];
+        kd_exact_emit<NT, 1>(ms, st, S, s, st.cnt[s], st.off[s], ms.atom_off[s / tp.n_types]);
+    }
+}
+
+// the sets of `list` (every set of the query where there is none) of min_n + 1
+// ... NT * P entries, P positions per thread
+template <int NT, int P>
+__global__ void __launch_bounds__(NT, 4) k_kdexact_lds(DevMols ms, DevTpls tp, DevSets st, const int *list,
+                                                    const unsigned int *count, int min_n)
+{
+    static_assert(NT * P <= KD_LDS_MAX && KD_LDS_MAX <= 65536, "16-bit elements");
+    __shared__ KdExactLds<NT, P> S;
+    if (*st.total > st.cap) return;
+    const int cnt = list ? (int)*count : st.n_sets;
+    for (int q = blockIdx.x; q < cnt; q += gridDim.x) {
+        const int s = list ? list[q] : q;
+        const int n = st.cnt[s];
+        if (n <= min_n || n > NT * P) continue;
+        kd_exact_emit<NT, P>(ms, st, S, s, n, st.off[s], ms.atom_off[s / tp.n_types]);
     }
 }
 
@@ -1369,7 +1328,8 @@ __global__ void __launch_bounds__(KD_THREADS) k_kdbig(DevMols ms, DevTpls tp, De
     }
 }
 
-// exact path of the sets of `list` larger than min_n
+// exact path of the sets of `list` (every set of the query where there is none)
+// larger than min_n
 __global__ void __launch_bounds__(KD_EXACT_THREADS) k_kdbig_exact(DevMols ms, DevTpls tp, DevSets st,
                                                                   unsigned char *scr, const int *list,
                                                                   const unsigned int *count, int min_n)
@@ -1377,9 +1337,9 @@ __global__ void __launch_bounds__(KD_EXACT_THREADS) k_kdbig_exact(DevMols ms, De
     __shared__ int partial[KD_EXACT_THREADS];
     __shared__ int flag[2];
     if (*st.total > st.cap) return;
-    const int cnt = (int)*count;
+    const int cnt = list ? (int)*count : st.n_sets;
     for (int q = blockIdx.x; q < cnt; q += gridDim.x) {
-        const int s = list[q];
+        const int s = list ? list[q] : q;
         const int n = st.cnt[s];
         if (n <= min_n) continue;
         const int64_t off = st.off[s];

@@ -85,6 +85,7 @@ __global__ void __launch_bounds__(256) k_candidates(DevMols ms, DevTpls tp, DevS
     if (FILL && blockIdx.x == 0 && threadIdx.x == 0) {
         // level-0 items of all pairs: the end of the scan of the pair chunks
         const int np = pr.n_pairs;
+        *st.kd_err = 0u;   // the kd passes come after this
         *n_items = np > 0 ? pr.item_base[np - 1] + pr.nchunk[np - 1] : 0;
     }
     const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) / JAM_WAVE);
