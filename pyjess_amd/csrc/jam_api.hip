@@ -47,19 +47,29 @@ int32_t fail(int32_t code, const std::string &msg)
             return fail(JAM_EDEVICE, std::string(#expr) + ": " + hipGetErrorString(_e)); \
     } while (0)
 
-// A device allocation that grows (never shrinks) and frees itself.
+// A device allocation that grows (never shrinks) and frees itself; or a view
+// of a part of another one, which must outlive it.
 struct DBuf {
     void *ptr = nullptr;
     size_t bytes = 0;
+    bool owned = true;
     DBuf() = default;
     DBuf(const DBuf &) = delete;
     DBuf &operator=(const DBuf &) = delete;
     ~DBuf() { release(); }
     void release()
     {
-        if (ptr) (void)hipFree(ptr);
+        if (ptr && owned) (void)hipFree(ptr);
         ptr = nullptr;
         bytes = 0;
+        owned = true;
+    }
+    void view(void *p, size_t n)
+    {
+        release();
+        ptr = p;
+        bytes = n;
+        owned = false;
     }
     hipError_t reserve(size_t n)
     {
@@ -176,6 +186,15 @@ struct jam_context {
     DBuf g_buf, g_toff, g_nl, g_blk, g_blkoff, g_starts, g_kind, g_textof, g_first, g_lineatom, g_atomline, g_textrng;
     DBuf g_err, g_firsterr, g_keys, g_nnames, g_resoff64, g_bucket, g_bcount, g_bstart, g_skey, g_sval;
     std::vector<std::unique_ptr<DBuf>> g_scan;
+    // jam_molecules_create: two pinned halves of up_half bytes, one packed
+    // while the other is on its way to the device, and the index's temporary
+    // buffers; one call at a time uses them
+    std::mutex up_mutex;
+    void *up_stage = nullptr;
+    size_t up_half = 0;
+    hipEvent_t up_ev[2] = {};
+    DBuf u_keys, u_starts, u_nnames;
+    std::vector<std::unique_ptr<DBuf>> u_scan;
 };
 
 struct jam_templates {
@@ -211,6 +230,7 @@ struct jam_molecules {
     int n_mols = 0;
     int64_t n_atoms = 0;
     int64_t n_buckets = 0;
+    DBuf block;   // holds the arrays of a batch made by jam_molecules_create
     DBuf atom_off, xyz, name, resname, chain, resseq, perm, res_off, res_key, res_begin, res_end;
     // the other atom fields, kept by jam_molecules_parse_pdb for the host's copy
     bool parsed = false;
@@ -363,6 +383,9 @@ extern "C" void jam_context_free(jam_context *ctx)
         if (ev) (void)hipEventDestroy(ev);
     if (ctx->hstage) (void)hipHostFree(ctx->hstage);
     if (ctx->hsmall) (void)hipHostFree(ctx->hsmall);
+    if (ctx->up_stage) (void)hipHostFree(ctx->up_stage);
+    for (auto &ev : ctx->up_ev)
+        if (ev) (void)hipEventDestroy(ev);
     for (auto &ev : ctx->stage_ev)
         if (ev) (void)hipEventDestroy(ev);
     for (int k = 0; k < KD_TIERS; k++) {
@@ -483,40 +506,103 @@ extern "C" void jam_templates_free(jam_templates *t)
 // molecules
 // ---------------------------------------------------------------------------
 
-extern "C" int32_t jam_molecules_create(jam_context *ctx, const jam_molecule_desc *mols, int32_t n,
-                                        jam_molecules **out)
+namespace {
+int32_t residue_index(jam_context *c, jam_molecules *M, const int *order, void *perm, void *res_off, hipStream_t s,
+                      bool &done);
+}
+
+// ---------------------------------------------------------------------------
+// molecules from host arrays
+// ---------------------------------------------------------------------------
+
+namespace {
+
+// a stretch of host memory and where it goes in the device block
+struct UploadPart {
+    size_t at;
+    const void *src;
+    size_t bytes;
+};
+
+// bytes [lo, hi) of the image that `parts` (ascending, disjoint) make up, to dst
+void pack_range(const std::vector<UploadPart> &parts, size_t lo, size_t hi, char *dst)
 {
-    if (!ctx || !out || (n > 0 && !mols)) return fail(JAM_EINVAL, "NULL argument");
-    if (n < 0) return fail(JAM_EINVAL, "negative molecule count");
-    *out = nullptr;
-    std::vector<int> atom_off{0}, chain, resseq, perm, res_off{0}, res_begin, res_end;
-    std::vector<double> xyz;
-    std::vector<uint32_t> name, resname, res_key;
-    for (int m = 0; m < n; m++) {
-        const jam_molecule_desc &M = mols[m];
-        if (M.n_atoms < 0) return fail(JAM_EINVAL, "negative atom count");
-        const int N = M.n_atoms;
-        if ((int64_t)atom_off.back() + N > INT32_MAX) return fail(JAM_ETOOBIG, "too many atoms in one batch");
-        xyz.insert(xyz.end(), M.xyz, M.xyz + 3 * (size_t)N);
-        std::vector<uint32_t> upkey(N);
-        for (int i = 0; i < N; i++) {
-            name.push_back(pack4(M.names + 4 * i));
-            uint32_t rn = pack4(M.resnames + 4 * i);
-            resname.push_back(rn);
-            upkey[i] = jam_upper4(rn);
-            chain.push_back((int)(signed char)M.chain2[i]);
-            resseq.push_back(M.resseq[i]);
+    auto it = std::upper_bound(parts.begin(), parts.end(), lo, [](size_t x, const UploadPart &p) { return x < p.at; });
+    if (it != parts.begin()) --it;
+    for (; it != parts.end() && it->at < hi; ++it) {
+        const size_t a = std::max(lo, it->at), b = std::min(hi, it->at + it->bytes);
+        if (a < b) std::memcpy(dst + (a - lo), (const char *)it->src + (a - it->at), b - a);
+    }
+}
+
+// The same by up to 8 host threads, each at least 1 MB of it.
+void pack_range_mt(const std::vector<UploadPart> &parts, size_t lo, size_t hi, char *dst)
+{
+    const size_t nt = std::min<size_t>(8, (hi - lo) >> 20);
+    std::vector<std::thread> th;
+    size_t done = lo;
+    if (nt > 1) {
+        const size_t per = ((hi - lo) / nt) & ~(size_t)63;
+        try {
+            th.reserve(nt);
+            for (size_t k = 0; k + 1 < nt; k++, done += per)
+                th.emplace_back([&parts, done, per, lo, dst] { pack_range(parts, done, done + per, dst + (done - lo)); });
+        } catch (...) {
+            // no more threads: the rest is done here
         }
-        // residue-name index (ResIndex_create, patches/ResIndex.c.patch:34-119):
-        // atoms grouped by case-insensitive residue name, each group by serial,
-        // ties in input order. Groups are ordered by their packed key value,
-        // the order the device binary search expects; the order of groups has
-        // no effect on candidate lists, only the order inside a group does.
+    }
+    pack_range(parts, done, hi, dst + (done - lo));
+    for (auto &x : th) x.join();
+}
+
+constexpr size_t UP_HALF_MAX = size_t(16) << 20;
+
+// Sends the image of `bytes` bytes to dev on stream s through the pinned
+// halves (the caller holds up_mutex). Pinned halves because a copy from
+// pageable memory moves at 10 GB/s here, a pinned one at 50, and its packing
+// runs beside the transfer before it.
+int32_t upload_parts(jam_context *c, const std::vector<UploadPart> &parts, size_t bytes, char *dev, hipStream_t s)
+{
+    const size_t want = std::min(UP_HALF_MAX, std::max<size_t>(bytes, size_t(1) << 18));
+    if (want > c->up_half) {
+        if (c->up_stage) HIP_TRY(hipHostFree(c->up_stage));
+        c->up_stage = nullptr;
+        c->up_half = 0;
+        HIP_TRY(hipHostMalloc(&c->up_stage, 2 * want, hipHostMallocDefault));
+        c->up_half = want;
+    }
+    for (auto &ev : c->up_ev)
+        if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    size_t k = 0;
+    for (size_t lo = 0; lo < bytes; lo += c->up_half, k++) {
+        const size_t hi = std::min(bytes, lo + c->up_half);
+        char *h = (char *)c->up_stage + (k & 1) * c->up_half;
+        if (k >= 2) HIP_TRY(hipEventSynchronize(c->up_ev[k & 1]));
+        pack_range_mt(parts, lo, hi, h);
+        HIP_TRY(hipMemcpyAsync(dev + lo, h, hi - lo, hipMemcpyHostToDevice, s));
+        HIP_TRY(hipEventRecord(c->up_ev[k & 1], s));
+    }
+    return JAM_OK;
+}
+
+// The residue-name index of a batch on the host, for molecules with more
+// names than the device kernel holds (ResIndex_create,
+// patches/ResIndex.c.patch:34-119): atoms grouped by case-insensitive residue
+// name, each group by serial, ties in input order, groups by key value.
+int32_t host_residue_index(const jam_molecule_desc *mols, int32_t n, jam_molecules *M, hipStream_t s)
+{
+    std::vector<int> perm, res_off{0}, res_begin, res_end;
+    std::vector<uint32_t> res_key;
+    for (int m = 0; m < n; m++) {
+        const jam_molecule_desc &D = mols[m];
+        const int N = D.n_atoms;
+        std::vector<uint32_t> upkey(N);
+        for (int i = 0; i < N; i++) upkey[i] = jam_upper4(pack4(D.resnames + 4 * (size_t)i));
         std::vector<int> p(N);
         std::iota(p.begin(), p.end(), 0);
         std::stable_sort(p.begin(), p.end(), [&](int a, int b) {
             if (upkey[a] != upkey[b]) return upkey[a] < upkey[b];
-            return M.serial[a] < M.serial[b];
+            return D.serial[a] < D.serial[b];
         });
         perm.insert(perm.end(), p.begin(), p.end());
         for (int i = 0; i < N; i++) {
@@ -528,28 +614,125 @@ extern "C" int32_t jam_molecules_create(jam_context *ctx, const jam_molecule_des
         }
         if (N > 0) res_end.push_back(N);
         res_off.push_back((int)res_key.size());
-        atom_off.push_back(atom_off.back() + N);
     }
-    HIP_TRY(hipSetDevice(ctx->device));
-    std::unique_ptr<jam_molecules> M(new jam_molecules());
-    M->ctx = ctx;
-    M->n_mols = n;
-    M->n_atoms = atom_off.back();
-    hipStream_t s = ctx->stream;
-    HIP_TRY(upload(M->atom_off, atom_off, s));
-    HIP_TRY(upload(M->xyz, xyz, s));
-    HIP_TRY(upload(M->name, name, s));
-    HIP_TRY(upload(M->resname, resname, s));
-    HIP_TRY(upload(M->chain, chain, s));
-    HIP_TRY(upload(M->resseq, resseq, s));
     HIP_TRY(upload(M->perm, perm, s));
     HIP_TRY(upload(M->res_off, res_off, s));
     HIP_TRY(upload(M->res_key, res_key, s));
     HIP_TRY(upload(M->res_begin, res_begin, s));
     HIP_TRY(upload(M->res_end, res_end, s));
     M->n_buckets = (int64_t)res_key.size();
+    return JAM_OK;
+}
+
+// serial numbers that never descend
+bool ascending(const int32_t *v, int n)
+{
+    int down = 0;
+    for (int i = 1; i < n; i++) down |= v[i] < v[i - 1];
+    return down == 0;
+}
+
+int32_t create_molecules(jam_context *ctx, const jam_molecule_desc *mols, int32_t n, jam_molecules **out)
+{
+    std::vector<int> atom_off(1, 0);
+    atom_off.reserve((size_t)n + 1);
+    for (int m = 0; m < n; m++) {
+        if (mols[m].n_atoms < 0) return fail(JAM_EINVAL, "negative atom count");
+        if ((int64_t)atom_off.back() + mols[m].n_atoms > INT32_MAX)
+            return fail(JAM_ETOOBIG, "too many atoms in one batch");
+        atom_off.push_back(atom_off.back() + mols[m].n_atoms);
+    }
+    const size_t na = (size_t)atom_off.back();
+    // molecules whose serial numbers descend somewhere: all atoms of the batch
+    // in order of serial number, ties in input order
+    std::vector<int> order;
+    for (int m = 0; m < n; m++) {
+        const int N = mols[m].n_atoms;
+        if (ascending(mols[m].serial, N)) continue;
+        if (order.empty()) {
+            order.resize(na);
+            for (int q = 0; q < n; q++) std::iota(order.begin() + atom_off[q], order.begin() + atom_off[q + 1], 0);
+        }
+        const int32_t *sr = mols[m].serial;
+        std::stable_sort(order.begin() + atom_off[m], order.begin() + atom_off[m + 1],
+                         [sr](int a, int b) { return sr[a] < sr[b]; });
+    }
+    HIP_TRY(hipSetDevice(ctx->device));
+    std::lock_guard<std::mutex> guard(ctx->up_mutex);
+    std::unique_ptr<jam_molecules> M(new jam_molecules());
+    M->ctx = ctx;
+    M->n_mols = n;
+    M->n_atoms = (int64_t)na;
+    hipStream_t s = ctx->stream;
+    // one block: the uploaded arrays first, as one image, then those made on
+    // the device
+    size_t bytes = 0;
+    auto place = [&](size_t b) {
+        const size_t at = bytes;
+        bytes += (std::max<size_t>(b, 1) + 255) & ~(size_t)255;
+        return at;
+    };
+    const size_t o_off = place(sizeof(int) * ((size_t)n + 1)), o_xyz = place(sizeof(double) * 3 * na);
+    const size_t o_name = place(4 * na), o_resname = place(4 * na), o_resseq = place(sizeof(int) * na);
+    const size_t o_chain8 = place(na), o_order = order.empty() ? bytes : place(sizeof(int) * na);
+    const size_t image = bytes;
+    const size_t o_chain = place(sizeof(int) * na), o_perm = place(sizeof(int) * na);
+    const size_t o_resoff = place(sizeof(int) * ((size_t)n + 1));
+    HIP_TRY(M->block.reserve(bytes));
+    char *base = M->block.as<char>();
+    M->atom_off.view(base + o_off, sizeof(int) * ((size_t)n + 1));
+    M->xyz.view(base + o_xyz, sizeof(double) * 3 * na);
+    M->name.view(base + o_name, 4 * na);
+    M->resname.view(base + o_resname, 4 * na);
+    M->resseq.view(base + o_resseq, sizeof(int) * na);
+    M->chain.view(base + o_chain, sizeof(int) * na);
+    std::vector<UploadPart> parts;
+    parts.reserve(5 * (size_t)n + 2);
+    parts.push_back({o_off, atom_off.data(), sizeof(int) * ((size_t)n + 1)});
+    auto add = [&](size_t at, size_t width, auto src) {
+        for (int m = 0; m < n; m++)
+            if (mols[m].n_atoms > 0)
+                parts.push_back({at + width * (size_t)atom_off[m], src(mols[m]), width * (size_t)mols[m].n_atoms});
+    };
+    add(o_xyz, sizeof(double) * 3, [](const jam_molecule_desc &d) { return (const void *)d.xyz; });
+    add(o_name, 4, [](const jam_molecule_desc &d) { return (const void *)d.names; });
+    add(o_resname, 4, [](const jam_molecule_desc &d) { return (const void *)d.resnames; });
+    add(o_resseq, sizeof(int), [](const jam_molecule_desc &d) { return (const void *)d.resseq; });
+    add(o_chain8, 1, [](const jam_molecule_desc &d) { return (const void *)d.chain2; });
+    if (!order.empty()) parts.push_back({o_order, order.data(), sizeof(int) * na});
+    int32_t rc = upload_parts(ctx, parts, image, base, s);
+    bool on_device = false;
+    if (rc == JAM_OK && n > 0) {
+        if (na > 0)
+            hipLaunchKernelGGL(jam::k_chain_words, dim3((unsigned)((na + ING_THREADS - 1) / ING_THREADS)),
+                               dim3(ING_THREADS), 0, s, (const signed char *)(base + o_chain8), (long long)na,
+                               M->chain.as<int>());
+        rc = residue_index(ctx, M.get(), order.empty() ? nullptr : (const int *)(base + o_order), base + o_perm,
+                           base + o_resoff, s, on_device);
+    }
+    if (rc == JAM_OK && !on_device) rc = host_residue_index(mols, n, M.get(), s);
+    // the pinned halves are free again, and so is the memory of a batch that
+    // is given up, only once its transfers are over
+    const hipError_t e = hipStreamSynchronize(s);
+    if (rc != JAM_OK) return rc;
+    HIP_TRY(e);
     *out = M.release();
     return JAM_OK;
+}
+
+}  // namespace
+
+extern "C" int32_t jam_molecules_create(jam_context *ctx, const jam_molecule_desc *mols, int32_t n,
+                                        jam_molecules **out)
+{
+    if (!ctx || !out || (n > 0 && !mols)) return fail(JAM_EINVAL, "NULL argument");
+    if (n < 0) return fail(JAM_EINVAL, "negative molecule count");
+    *out = nullptr;
+    try {
+        return create_molecules(ctx, mols, n, out);
+    } catch (const std::bad_alloc &) {
+        return fail(JAM_ENOMEM, "out of host memory");
+    }
 }
 
 extern "C" void jam_molecules_free(jam_molecules *m)
@@ -743,6 +926,49 @@ int32_t read_one(const T *dev, T &host, hipStream_t s)
 {
     HIP_TRY(hipMemcpyAsync(&host, dev, sizeof(T), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
+    return JAM_OK;
+}
+
+// The residue-name index of M (atom_off and resname on the device) by
+// k_residue_index, into perm and res_off where they are given (space in M's
+// block) and arrays of the exact size. `done` stays false where a molecule has
+// more names than the kernel holds. Synchronises once, for the number of
+// groups.
+int32_t residue_index(jam_context *c, jam_molecules *M, const int *order, void *perm, void *res_off, hipStream_t s,
+                      bool &done)
+{
+    const int n = M->n_mols;
+    const size_t na = (size_t)std::max<int64_t>(M->n_atoms, 1);
+    M->perm.view(perm, sizeof(int) * na);
+    M->res_off.view(res_off, sizeof(int) * ((size_t)n + 1));
+    HIP_TRY(c->u_keys.reserve(sizeof(uint32_t) * na));
+    HIP_TRY(c->u_starts.reserve(sizeof(int) * na));
+    HIP_TRY(c->u_nnames.reserve(sizeof(int) * (size_t)n));
+    const int *aoff = M->atom_off.as<const int>();
+    hipLaunchKernelGGL(jam::k_residue_index<IDX_MAX_NAMES>, dim3((unsigned)n), dim3(IDX_THREADS), 0, s, aoff,
+                       M->resname.as<const uint32_t>(), order, M->perm.as<int>(), c->u_keys.as<uint32_t>(),
+                       c->u_starts.as<int>(), c->u_nnames.as<int>());
+    HIP_TRY(hipGetLastError());
+    std::vector<int> names((size_t)n);
+    HIP_TRY(hipMemcpyAsync(names.data(), c->u_nnames.ptr, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost, s));
+    int32_t rc = device_scan<int, int>(c->u_nnames.as<const int>(), n, M->res_off.as<int>(), c->u_scan, 0, s);
+    HIP_TRY(hipStreamSynchronize(s));
+    if (rc != JAM_OK) return rc;
+    int64_t total = 0;
+    for (int x : names) {
+        if (x < 0) return JAM_OK;
+        total += x;
+    }
+    M->n_buckets = total;
+    const size_t nb = (size_t)std::max<int64_t>(total, 1);
+    HIP_TRY(M->res_key.reserve(3 * sizeof(uint32_t) * nb));
+    M->res_begin.view(M->res_key.as<int>() + nb, sizeof(int) * nb);
+    M->res_end.view(M->res_key.as<int>() + 2 * nb, sizeof(int) * nb);
+    hipLaunchKernelGGL(jam::k_index_ranges, dim3((unsigned)n), dim3(ING_THREADS), 0, s, aoff,
+                       c->u_keys.as<const uint32_t>(), c->u_starts.as<const int>(), M->res_off.as<const int>(),
+                       M->res_key.as<uint32_t>(), M->res_begin.as<int>(), M->res_end.as<int>());
+    HIP_TRY(hipGetLastError());
+    done = true;
     return JAM_OK;
 }
 

@@ -569,4 +569,198 @@ __global__ void __launch_bounds__(ING_THREADS) k_ing_ranges(const int *atom_off,
     res_end[b] = (int)(bucket_start[b + 1] - atom_off[lo]);
 }
 
+// The residue-name index of a batch in one launch (ResIndex_create,
+// patches/ResIndex.c.patch:34-119): a workgroup per molecule. The molecule's
+// distinct upper-cased names go through an LDS hash set and a bitonic sort
+// (groups ordered by key value, which the candidate kernels' binary search
+// expects); then each of the 16 waves takes a contiguous 16th of the atoms,
+// counts its atoms per name, and after a scan over (name, wave) walks them
+// again, 64 at a time, to their places: a lane's rank among the lanes of its
+// name comes from one ballot per bit of the name's number, so the counting
+// sort is stable and its second walk needs no workgroup barrier.
+// `order`, where given, is the order in which a molecule's atoms are visited
+// (its molecule-local indices by serial number, ties in input order); without
+// it they are visited as they come, which is the same thing for serial numbers
+// that never descend. Either way atoms end up by (name, serial, input order).
+//
+// keys / starts: the k-th name of molecule m and the first position of its
+// group at [atom_off[m] + k] (a molecule has no more names than atoms).
+// n_names[m] = -1 where a molecule has more than MAXN names, or one whose four
+// bytes are all 0xFF (the empty slot's mark).
+//
+// Bound by latency (two walks with one dependent load each and ~10 LDS steps
+// per 64 atoms of a wave) and by the waves in flight: 2 workgroups of 16 waves
+// per CU at MAXN = 256 (19 KB of LDS). One launch for all molecules instead of
+// a host sort: jam_molecules_create of 256 molecules (1.2 M atoms) 39.6 -> 3.2
+// ms, of 100,000 atoms 2.2 -> 0.57 ms, of 2,000 atoms 0.22 -> 0.07 ms, with
+// the upload through pinned memory that came with it.
+#define IDX_THREADS 1024
+#define IDX_WAVES (IDX_THREADS / JAM_WAVE)
+#define IDX_MAX_NAMES 256
+
+template <int MAXN>
+__global__ void __launch_bounds__(IDX_THREADS) k_residue_index(const int *atom_off, const uint32_t *resname,
+                                                               const int *order, int *perm, uint32_t *keys,
+                                                               int *starts, int *n_names)
+{
+    constexpr int SLOTS = 2 * MAXN;   // open addressing at half load at most
+    constexpr uint32_t EMPTY = 0xFFFFFFFFu;
+    __shared__ uint32_t slot[SLOTS];
+    __shared__ uint32_t list[MAXN];
+    __shared__ int run[IDX_WAVES][MAXN];   // per wave and name: atoms, then the next position
+    __shared__ int count, refused;
+    const int m = blockIdx.x, t = threadIdx.x, lane = lane_id(), w = t / JAM_WAVE;
+    for (int k = t; k < SLOTS; k += IDX_THREADS) slot[k] = EMPTY;
+    if (t == 0) {
+        count = 0;
+        refused = 0;
+    }
+    __syncthreads();
+    const int a0 = atom_off[m], n_atoms = atom_off[m + 1] - a0;
+    // distinct names: the first atom of a run of equal names (as stored)
+    // enters it for the run
+    for (int i = t; i < n_atoms; i += IDX_THREADS) {
+        const uint32_t key = jam_upper4(resname[a0 + i]);
+        if (i > 0 && jam_upper4(resname[a0 + i - 1]) == key) continue;
+        if (key == EMPTY) {
+            refused = 1;
+            continue;
+        }
+        uint32_t h = (key * 2654435761u) >> 7;
+        for (int probe = 0; probe < SLOTS; probe++) {
+            h &= SLOTS - 1;
+            const uint32_t old = atomicCAS(&slot[h], EMPTY, key);
+            if (old == EMPTY) {
+                const int c = atomicAdd(&count, 1);
+                if (c < MAXN) list[c] = key;
+                break;
+            }
+            if (old == key) break;
+            h++;
+        }
+        if (count > MAXN) break;
+    }
+    __syncthreads();
+    const int n = count;
+    if (n > MAXN || refused) {
+        if (t == 0) n_names[m] = -1;
+        return;
+    }
+    int n2 = 1, bits = 0;
+    while (n2 < n) {
+        n2 <<= 1;
+        bits++;
+    }
+    for (int k = n + t; k < n2; k += IDX_THREADS) list[k] = EMPTY;
+    for (int k = t; k < IDX_WAVES * n; k += IDX_THREADS) run[k / n][k % n] = 0;
+    __syncthreads();
+    for (int k = 2; k <= n2; k <<= 1) {
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            for (int i = t; i < n2; i += IDX_THREADS) {
+                const int ixj = i ^ j;
+                if (ixj > i) {
+                    const uint32_t u = list[i], v = list[ixj];
+                    if ((u > v) == ((i & k) == 0)) {
+                        list[i] = v;
+                        list[ixj] = u;
+                    }
+                }
+            }
+            __syncthreads();
+        }
+    }
+    // this wave's part of the atoms, a multiple of 64
+    const int per = ((n_atoms + IDX_THREADS - 1) / IDX_THREADS) * JAM_WAVE;
+    const int begin = min(w * per, n_atoms), end = min(begin + per, n_atoms);
+    // the i-th visited atom (molecule-local) and the number of its name
+    auto visit = [&](int i, int &atom, int &b) {
+        atom = order ? order[a0 + i] : i;
+        const uint32_t key = jam_upper4(resname[a0 + atom]);
+        int lo = 0, hi = n - 1;   // the last name <= key is key itself
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (list[mid] <= key) lo = mid;
+            else hi = mid - 1;
+        }
+        b = lo;
+    };
+    for (int i = begin + lane; i < end; i += JAM_WAVE) {
+        int atom, b;
+        visit(i, atom, b);
+        atomicAdd(&run[w][b], 1);
+    }
+    __syncthreads();
+    // where each name's group starts, and in it each wave's part
+    if (t < JAM_WAVE) {
+        int carry = 0;
+        for (int b0 = 0; b0 < n; b0 += JAM_WAVE) {
+            const int b = b0 + lane;
+            int v = 0;
+            if (b < n)
+                for (int q = 0; q < IDX_WAVES; q++) v += run[q][b];
+            int x = v;
+            for (int sh = 1; sh < JAM_WAVE; sh <<= 1) {
+                const int y = __shfl_up(x, sh, JAM_WAVE);
+                if (lane >= sh) x += y;
+            }
+            if (b < n) {
+                int at = carry + x - v;
+                keys[a0 + b] = list[b];
+                starts[a0 + b] = at;
+                for (int q = 0; q < IDX_WAVES; q++) {
+                    const int c = run[q][b];
+                    run[q][b] = at;
+                    at += c;
+                }
+            }
+            carry += __shfl(x, JAM_WAVE - 1, JAM_WAVE);
+        }
+        if (lane == 0) n_names[m] = n;
+    }
+    __syncthreads();
+    for (int i0 = begin; i0 < end; i0 += JAM_WAVE) {
+        const int i = i0 + lane;
+        const bool ok = i < end;
+        int atom = 0, b = 0;
+        if (ok) visit(i, atom, b);
+        unsigned long long peers = ballot(ok);
+        for (int q = 0; q < bits; q++) {
+            const bool bit = ((b >> q) & 1) != 0;
+            const unsigned long long x = ballot(bit);
+            peers &= bit ? x : ~x;
+        }
+        const int rank = rank_below(peers);
+        int at = 0;
+        if (ok) at = run[w][b];
+        wave_sync();
+        if (ok) {
+            perm[a0 + at + rank] = atom;
+            if (rank == 0) run[w][b] = at + __popcll(peers);
+        }
+        wave_sync();
+    }
+}
+
+// The names and ranges of every molecule's groups, packed (res_off: the
+// exclusive scan of n_names).
+__global__ void __launch_bounds__(ING_THREADS) k_index_ranges(const int *atom_off, const uint32_t *keys,
+                                                             const int *starts, const int *res_off, uint32_t *res_key,
+                                                             int *res_begin, int *res_end)
+{
+    const int m = blockIdx.x, a0 = atom_off[m], n_atoms = atom_off[m + 1] - a0;
+    const int r0 = res_off[m], n = res_off[m + 1] - r0;
+    for (int k = threadIdx.x; k < n; k += ING_THREADS) {
+        res_key[r0 + k] = keys[a0 + k];
+        res_begin[r0 + k] = starts[a0 + k];
+        res_end[r0 + k] = k + 1 < n ? starts[a0 + k + 1] : n_atoms;
+    }
+}
+
+// A chain byte per atom to the (sign-extended) word that the search compares.
+__global__ void __launch_bounds__(ING_THREADS) k_chain_words(const signed char *in, long long n, int *out)
+{
+    const long long i = (long long)blockIdx.x * ING_THREADS + threadIdx.x;
+    if (i < n) out[i] = in[i];
+}
+
 }  // namespace jam
