@@ -155,6 +155,9 @@ struct jam_context {
     unsigned kd_used = 0;       // bit k: the last kd launch uses side stream k
     // sort of the complete matches
     DBuf s_key[2], s_perm[2], s_pkey[2];
+    // groups of level-0 rows: matches, first position; each match's group, the
+    // sorted matches, the positions of large groups
+    DBuf sg_count, sg_start, sg_seg[2], sg_perm, sg_list;
     DBuf s_starts;   // per template size: complete matches of at most that many atoms
     // radix-sort histograms and their scan; scan temporaries of the query
     DBuf rs_hist, rs_off;
@@ -1436,6 +1439,23 @@ __global__ void k_zero_u64(unsigned long long *v, long long n)
         v[i] = 0ull;
 }
 
+// Sorting the complete matches by groups of level-0 rows. Up to
+// GROUP_RANK_MATCHES matches with up to GROUP_RANK_WORK comparisons (halved)
+// every group is ranked by comparison: the LDS sort's tiles would leave most
+// CUs idle (49,000 matches: 46 us in 4 passes). Above, groups of up to
+// GROUP_TILE / 2 matches are sorted in LDS (6.3 M matches: 0.72 ms) and larger
+// ones ranked, about 1.8 us per million comparisons (halved) and pass: past
+// group_work_max of them the radix passes are faster (470,000 matches of a
+// 100,000-atom assembly, 28 M in large groups: 0.56 ms against 1.7 ms by radix
+// passes; 6.3 M matches, 550 M in large groups: 3.2 against 2.4 ms).
+#ifndef GROUP_RANK_WORK
+#define GROUP_RANK_WORK 8000000ull
+#endif
+#ifndef GROUP_RANK_MATCHES
+#define GROUP_RANK_MATCHES 131072
+#endif
+unsigned long long group_work_max(int64_t n) { return 200000000ull + 16ull * (unsigned long long)n; }
+
 // workgroups of `kernel` (with `threads` threads) that stay resident on the device
 template <class K>
 int resident_grid(K kernel, int threads, int device)
@@ -1645,6 +1665,150 @@ hipError_t kd_join(jam_context *c, hipStream_t s)
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+// The complete matches in report order by LSD radix passes: first by template
+// size, then over the level positions (`bits` bits each, `per` levels per
+// 64-bit key), the last levels first, then the pair. The result is in
+// s_perm[cur].
+int32_t sort_radix(jam_context *c, const DevSets &st, const DevTpls &dt, const DevPairs &pr, const DevJoin &jn,
+                   int64_t n_done, int stride, int bits, int pbits, hipStream_t s, int &cur)
+{
+    const int T = dt.n_templates;
+    const unsigned gs = (unsigned)((n_done + 255) / 256);
+    int32_t rc;
+    cur = 0;
+    const int per = std::max(1, 64 / bits);
+    const int nt = stride;
+    // the matches by template size (stably): a match's levels at or
+    // past its template's size are 0, so a group of levels starting
+    // at l0 needs sorting only over the matches of more than l0
+    // atoms, a suffix; that suffix's order is the only one to change,
+    // so both permutation buffers keep the rest as it was
+    hipLaunchKernelGGL(jam::k_iota, dim3(gs), dim3(256), 0, s, c->s_perm[0].as<int>(), (long long)n_done);
+    hipLaunchKernelGGL(jam::k_sizekey, dim3(gs), dim3(256), 0, s, dt, jn, (long long)n_done,
+                       c->s_pkey[0].as<unsigned int>());
+    {
+        int which = 0;
+        if ((rc = radix_sort<unsigned int>(c->s_pkey[0].as<unsigned int>(), c->s_perm[0].as<int>(),
+                                           c->s_pkey[1].as<unsigned int>(), c->s_perm[1].as<int>(),
+                                           (long long)n_done, 6, c->rs_hist, c->rs_off, c->q_scan, s,
+                                           which)) != JAM_OK)
+            return rc;
+        cur = which;
+        HIP_TRY(c->s_starts.reserve(sizeof(long long) * (JAM_MAX_LEVELS + 1)));
+        hipLaunchKernelGGL(jam::k_size_starts, dim3(1), dim3(64), 0, s, c->s_pkey[which].as<const unsigned int>(),
+                           (long long)n_done, nt, c->s_starts.as<long long>());
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipMemcpyAsync(c->s_perm[cur ^ 1].as<int>(), c->s_perm[cur].as<const int>(),
+                               sizeof(int) * (size_t)n_done, hipMemcpyDeviceToDevice, s));
+        HIP_TRY(hipMemcpyAsync(c->hsmall, c->s_starts.as<const long long>(), sizeof(long long) * (size_t)(nt + 1),
+                               hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+    }
+    long long size_le[JAM_MAX_LEVELS + 1];
+    std::memcpy(size_le, c->hsmall, sizeof(long long) * (size_t)(nt + 1));
+    for (int l0 = ((nt - 1) / per) * per; l0 >= 0; l0 -= per) {
+        const int cnt_l = std::min(per, nt - l0);
+        const long long a = l0 == 0 ? 0 : size_le[l0];   // matches of at most l0 atoms stay put
+        const long long m = (long long)n_done - a;
+        if (m <= 1) continue;
+        // levels [l0, l0 + cnt_l) packed into cnt_l * bits bits
+        hipLaunchKernelGGL(jam::k_sortkey, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, st, dt, pr, jn,
+                           c->s_perm[cur].as<const int>() + a, m, l0, cnt_l, bits,
+                           c->s_key[0].as<unsigned long long>() + a);
+        int which = 0;
+        if ((rc = radix_sort<unsigned long long>(c->s_key[0].as<unsigned long long>() + a,
+                                                 c->s_perm[cur].as<int>() + a,
+                                                 c->s_key[1].as<unsigned long long>() + a,
+                                                 c->s_perm[cur ^ 1].as<int>() + a, m, cnt_l * bits,
+                                                 c->rs_hist, c->rs_off, c->q_scan, s, which)) != JAM_OK)
+            return rc;
+        cur ^= which;
+    }
+    hipLaunchKernelGGL(jam::k_pairkey, dim3(gs), dim3(256), 0, s, jn, T, c->s_perm[cur].as<const int>(),
+                       (long long)n_done, c->s_pkey[0].as<unsigned int>());
+    int which = 0;
+    if ((rc = radix_sort<unsigned int>(c->s_pkey[0].as<unsigned int>(), c->s_perm[cur].as<int>(),
+                                       c->s_pkey[1].as<unsigned int>(), c->s_perm[cur ^ 1].as<int>(),
+                                       (long long)n_done, pbits, c->rs_hist, c->rs_off, c->q_scan, s,
+                                       which)) != JAM_OK)
+        return rc;
+    cur ^= which;
+    HIP_TRY(hipGetLastError());
+    return JAM_OK;
+}
+
+// The same by groups of level-0 rows (k_group_count ... k_group_tile); the
+// result is `perm`. `perm` stays null, with nothing sorted, where the rows
+// cannot be numbered in 32 bits or the groups are too large.
+int32_t sort_groups(jam_context *c, const DevSets &st, const DevTpls &dt, const DevPairs &pr, const DevJoin &jn,
+                    int64_t n_done, int64_t n_rows, int stride, int bits, hipStream_t s, const int *&perm)
+{
+    perm = nullptr;
+    if (n_rows > (int64_t)UINT32_MAX) return JAM_OK;
+    // about as many groups as matches: fewer would mean more comparisons,
+    // more a longer scan
+    int shift = 0;
+    while ((n_rows >> shift) > std::max<int64_t>(2 * n_done, 1 << 16)) shift++;
+    const int64_t groups = (n_rows >> shift) + 1;
+    if (c->sg_count.reserve(sizeof(int) * (size_t)groups) != hipSuccess ||
+        c->sg_start.reserve(sizeof(int) * ((size_t)groups + 1)) != hipSuccess ||
+        c->sg_seg[0].reserve(sizeof(jam::GroupSeg) * (size_t)n_done) != hipSuccess ||
+        c->sg_seg[1].reserve(sizeof(jam::GroupSeg) * (size_t)n_done) != hipSuccess ||
+        c->sg_perm.reserve(sizeof(int) * (size_t)n_done) != hipSuccess ||
+        c->sg_list.reserve(sizeof(int) * (size_t)n_done) != hipSuccess) {
+        (void)hipGetLastError();   // no room for them: the radix passes need less
+        return JAM_OK;
+    }
+    HIP_TRY(c->s_starts.reserve(sizeof(long long) * (JAM_MAX_LEVELS + 1)));
+    const unsigned gs = (unsigned)((n_done + 255) / 256);
+    unsigned int *row = c->s_pkey[0].as<unsigned int>();
+    int *slot = c->s_pkey[1].as<int>();
+    unsigned long long *work = c->s_starts.as<unsigned long long>();
+    hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)std::min<int64_t>(2048, (groups + 255) / 256)), dim3(256), 0, s,
+                       c->sg_count.as<int>(), (long long)groups, 0);
+    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, work, 4ll);
+    hipLaunchKernelGGL(jam::k_group_count, dim3(std::min(gs, 2048u)), dim3(256), 0, s, st, dt, pr, jn, (long long)n_done,
+                       shift, row, slot, c->sg_count.as<int>(), work);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(c->hsmall, work, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    const int32_t rc = device_scan<int, int>(c->sg_count.as<const int>(), groups, c->sg_start.as<int>(), c->q_scan, 0, s);
+    HIP_TRY(hipStreamSynchronize(s));
+    if (rc != JAM_OK) return rc;
+    const unsigned long long all = c->hsmall[0], most = c->hsmall[1] + 1, big = c->hsmall[2];
+    if (big > group_work_max(n_done)) return JAM_OK;
+    // groups of at least `least` matches by ranking, the others in LDS
+    const bool rank_all = all <= GROUP_RANK_WORK && n_done <= GROUP_RANK_MATCHES;
+    const int half = GROUP_TILE / 2, least = rank_all ? 1 : half + 1;
+    int *list = rank_all ? nullptr : c->sg_list.as<int>();
+    unsigned long long *n_list = work + 3;
+    hipLaunchKernelGGL(jam::k_group_scatter, dim3(gs), dim3(256), 0, s, dt, pr, jn, (long long)n_done, shift, least,
+                       (const unsigned int *)row, (const int *)slot, c->sg_start.as<const int>(),
+                       c->s_perm[0].as<int>(), c->s_key[0].as<unsigned long long>(), c->sg_seg[0].as<jam::GroupSeg>());
+    if (!rank_all)
+        hipLaunchKernelGGL(jam::k_group_tile, dim3((unsigned)((n_done + half - 1) / half)), dim3(1024), 0, s, dt, pr, jn,
+                           (long long)n_done, shift, (const unsigned int *)row, c->s_perm[0].as<const int>(),
+                           c->sg_seg[0].as<const jam::GroupSeg>(), c->sg_perm.as<int>());
+    if (!rank_all && most >= (unsigned long long)least)
+        hipLaunchKernelGGL(jam::k_group_list, dim3(gs), dim3(256), 0, s, c->sg_seg[0].as<const jam::GroupSeg>(),
+                           (long long)n_done, least, list, n_list);
+    if (rank_all || most >= (unsigned long long)least) {
+        // passes: key words when every level takes `bits` bits (an upper bound)
+        const int per = 64 / bits, first = (64 - shift) / bits;
+        const int words = 1 + std::max(0, (stride - 1 - first + per - 1) / per);
+        const unsigned waves = (unsigned)std::min<int64_t>(8192, (n_done + 3) / 4);
+        int cur = 0;
+        for (int w = 0; w < words; w++, cur ^= 1)
+            hipLaunchKernelGGL(jam::k_group_rank, dim3(waves), dim3(256), 0, s, dt, pr, jn, (long long)n_done,
+                               (const int *)list, (const unsigned long long *)n_list, c->s_perm[cur].as<const int>(),
+                               c->s_key[cur].as<const unsigned long long>(), c->sg_seg[cur].as<const jam::GroupSeg>(),
+                               w + 1 < words ? c->s_perm[cur ^ 1].as<int>() : c->sg_perm.as<int>(),
+                               c->s_key[cur ^ 1].as<unsigned long long>(), c->sg_seg[cur ^ 1].as<jam::GroupSeg>());
+    }
+    HIP_TRY(hipGetLastError());
+    perm = c->sg_perm.as<const int>();
+    return JAM_OK;
 }
 
 }  // namespace
@@ -1862,6 +2026,7 @@ extern "C" int32_t jam_query(jam_context *c, const jam_templates *tp, const jam_
         if ((rc = grow_sort(c, n_done)) != JAM_OK) return rc;
         if ((rc = grow_events(c, n_done, stride)) != JAM_OK) return rc;
         int cur = 0;
+        const int *grouped = nullptr;
         const unsigned gs = (unsigned)((n_done + 255) / 256);
         int pbits = 1;
         while ((1ll << pbits) < (long long)n_pairs) pbits++;
@@ -1892,66 +2057,11 @@ extern "C" int32_t jam_query(jam_context *c, const jam_templates *tp, const jam_
                                c->s_perm[0].as<int>());
             HIP_TRY(hipGetLastError());
         } else if (n_done > 0) {
-            const int per = std::max(1, 64 / bits);
-            const int nt = stride;
-            // the matches by template size (stably): a match's levels at or
-            // past its template's size are 0, so a group of levels starting
-            // at l0 needs sorting only over the matches of more than l0
-            // atoms, a suffix; that suffix's order is the only one to change,
-            // so both permutation buffers keep the rest as it was
-            hipLaunchKernelGGL(jam::k_iota, dim3(gs), dim3(256), 0, s, c->s_perm[0].as<int>(), (long long)n_done);
-            hipLaunchKernelGGL(jam::k_sizekey, dim3(gs), dim3(256), 0, s, dt, jn, (long long)n_done,
-                               c->s_pkey[0].as<unsigned int>());
-            {
-                int which = 0;
-                if ((rc = radix_sort<unsigned int>(c->s_pkey[0].as<unsigned int>(), c->s_perm[0].as<int>(),
-                                                   c->s_pkey[1].as<unsigned int>(), c->s_perm[1].as<int>(),
-                                                   (long long)n_done, 6, c->rs_hist, c->rs_off, c->q_scan, s,
-                                                   which)) != JAM_OK)
-                    return rc;
-                cur = which;
-                HIP_TRY(c->s_starts.reserve(sizeof(long long) * (JAM_MAX_LEVELS + 1)));
-                hipLaunchKernelGGL(jam::k_size_starts, dim3(1), dim3(64), 0, s, c->s_pkey[which].as<const unsigned int>(),
-                                   (long long)n_done, nt, c->s_starts.as<long long>());
-                HIP_TRY(hipGetLastError());
-                HIP_TRY(hipMemcpyAsync(c->s_perm[cur ^ 1].as<int>(), c->s_perm[cur].as<const int>(),
-                                       sizeof(int) * (size_t)n_done, hipMemcpyDeviceToDevice, s));
-                HIP_TRY(hipMemcpyAsync(c->hsmall, c->s_starts.as<const long long>(), sizeof(long long) * (size_t)(nt + 1),
-                                       hipMemcpyDeviceToHost, s));
-                HIP_TRY(hipStreamSynchronize(s));
-            }
-            long long size_le[JAM_MAX_LEVELS + 1];
-            std::memcpy(size_le, c->hsmall, sizeof(long long) * (size_t)(nt + 1));
-            for (int l0 = ((nt - 1) / per) * per; l0 >= 0; l0 -= per) {
-                const int cnt_l = std::min(per, nt - l0);
-                const long long a = l0 == 0 ? 0 : size_le[l0];   // matches of at most l0 atoms stay put
-                const long long m = (long long)n_done - a;
-                if (m <= 1) continue;
-                // levels [l0, l0 + cnt_l) packed into cnt_l * bits bits
-                hipLaunchKernelGGL(jam::k_sortkey, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, st, dt, pr, jn,
-                                   c->s_perm[cur].as<const int>() + a, m, l0, cnt_l, bits,
-                                   c->s_key[0].as<unsigned long long>() + a);
-                int which = 0;
-                if ((rc = radix_sort<unsigned long long>(c->s_key[0].as<unsigned long long>() + a,
-                                                         c->s_perm[cur].as<int>() + a,
-                                                         c->s_key[1].as<unsigned long long>() + a,
-                                                         c->s_perm[cur ^ 1].as<int>() + a, m, cnt_l * bits,
-                                                         c->rs_hist, c->rs_off, c->q_scan, s, which)) != JAM_OK)
-                    return rc;
-                cur ^= which;
-            }
-            hipLaunchKernelGGL(jam::k_pairkey, dim3(gs), dim3(256), 0, s, jn, T, c->s_perm[cur].as<const int>(),
-                               (long long)n_done, c->s_pkey[0].as<unsigned int>());
-            int which = 0;
-            if ((rc = radix_sort<unsigned int>(c->s_pkey[0].as<unsigned int>(), c->s_perm[cur].as<int>(),
-                                               c->s_pkey[1].as<unsigned int>(), c->s_perm[cur ^ 1].as<int>(),
-                                               (long long)n_done, pbits, c->rs_hist, c->rs_off, c->q_scan, s,
-                                               which)) != JAM_OK)
+            if ((rc = sort_groups(c, st, dt, pr, jn, n_done, n0, stride, bits, s, grouped)) != JAM_OK) return rc;
+            if (!grouped && (rc = sort_radix(c, st, dt, pr, jn, n_done, stride, bits, pbits, s, cur)) != JAM_OK)
                 return rc;
-            cur ^= which;
-            HIP_TRY(hipGetLastError());
         }
-        const int *perm = c->s_perm[cur].as<const int>();
+        const int *perm = grouped ? grouped : c->s_perm[cur].as<const int>();
 
         // ---- superposition of every complete match; events in that order
         DevEvents ev;

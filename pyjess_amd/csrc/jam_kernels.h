@@ -15,10 +15,10 @@
 //                  64-entry blocks of the kd-ordered set whose box meets the
 //                  join box, each lane testing one candidate against every
 //                  annulus and check(); children appended in any order.
-//   k_sortkey      complete matches sorted by (molecule, template in scan
-//   k_rank         order, level positions): the reference's depth-first
-//                  order and each match's rank (radix passes, or rank
-//                  counting for a few thousand matches).
+//   k_rank         complete matches sorted by (molecule, template in scan
+//   k_group_*      order, level positions): the reference's depth-first
+//   k_sortkey      order and each match's rank (rank counting for a few
+//                  thousand matches, groups of level-0 rows, or radix passes).
 //   k_super        thread per complete match: FP64 superposition and RMSD
 //                  threshold, then (after a scan of the marks) the events in
 //                  that same order, each with the match's rank.
@@ -833,6 +833,316 @@ __global__ void __launch_bounds__(256) k_rank_scatter(const int *rank, long long
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) perm[rank[i]] = (int)i;
+}
+
+// Larger sorts: the level-0 rows of the query, numbered in report order
+// (molecule, template in scan order, list position), already group the
+// complete matches -- each match descends from one row -- so a counting sort
+// by that number (k_group_count, a scan, k_group_scatter) leaves only the
+// order inside a group of 2^shift neighbouring rows, by the kd positions of the
+// further levels, one 64-bit word of that key at a time. Two ways to it:
+// k_group_rank counts the smaller words of a match's group, k_group_tile sorts
+// the groups in LDS. Keys are unique, so the order in which the atomics hand
+// out a group's slots does not matter.
+
+#ifndef GROUP_TILE
+#define GROUP_TILE 4096
+#endif
+
+// Level-0 row of complete match i, in report order.
+__device__ static inline unsigned int level0_row(const DevSets &st, const DevPairs &pr, const DevJoin &jn,
+                                                 int n_templates, long long i)
+{
+    const int p = jn.done_pair[i];
+    const int m = p / n_templates;
+    const int ent = jn.done_ent[i * jn.stride];
+    // templates are scanned in reverse: the rows of the molecule's later
+    // templates come first
+    const long long before = pr.item_base[m * n_templates] + pr.item_base[(m + 1) * n_templates] -
+                             pr.item_base[p] - pr.nchunk[p];
+    // a one-atom template steps past list entry 0
+    return (unsigned int)(before + st.kidx[ent] - pr.n1[p]);
+}
+
+// Each match's row and its slot among the matches of its group. Per query:
+// work[0] += every slot (half the comparisons of k_group_rank's first pass),
+// work[1] = the largest, work[2] += the slots from GROUP_TILE / 2 on. Matches
+// lie in the order the join's waves wrote them, a few rows' matches to a wave:
+// one atomic per distinct group of the wave instead of one per match, and the
+// work counted by one atomic per workgroup of a bounded grid (one per wave on
+// the same words took 2.3 ms for 6.3 M matches).
+__global__ void __launch_bounds__(256) k_group_count(DevSets st, DevTpls tp, DevPairs pr, DevJoin jn, long long n,
+                                                     int shift, unsigned int *row, int *slot, int *count,
+                                                     unsigned long long *work)
+{
+    __shared__ unsigned long long part[3][256 / JAM_WAVE];
+    const int lane = lane_id();
+    unsigned long long sum = 0, most = 0, big = 0;
+    for (long long i0 = (long long)blockIdx.x * 256; i0 < n; i0 += (long long)gridDim.x * 256) {
+        const long long i = i0 + threadIdx.x;
+        unsigned int r = 0, g = 0;
+        bool pending = i < n;
+        if (pending) {
+            r = level0_row(st, pr, jn, tp.n_templates, i);
+            g = r >> shift;
+        }
+        // per lane: the first lane of its group, its rank in the group, the
+        // group's lanes (each round retires the lowest pending lane's group)
+        int leader = lane, rank = 0, peers = 0;
+        for (;;) {
+            const unsigned long long m = ballot(pending);
+            if (m == 0ull) break;
+            const int f = first_bit(m);
+            const unsigned int gf = (unsigned int)__shfl((int)g, f, JAM_WAVE);
+            const bool same = pending && g == gf;
+            const unsigned long long sm = ballot(same);
+            if (same) {
+                leader = f;
+                rank = rank_below(sm);
+                peers = __popcll(sm);
+                pending = false;
+            }
+        }
+        int base = 0;
+        if (i < n && lane == leader) base = atomicAdd(&count[g], peers);
+        const int k = __shfl(base, leader, JAM_WAVE) + rank;
+        if (i < n) {
+            row[i] = r;
+            slot[i] = k;
+            sum += (unsigned long long)k;
+            most = max(most, (unsigned long long)k);
+            if (k >= GROUP_TILE / 2) big += (unsigned long long)k;
+        }
+    }
+    for (int sh = JAM_WAVE / 2; sh >= 1; sh >>= 1) {
+        sum += __shfl_xor(sum, sh, JAM_WAVE);
+        most = max(most, __shfl_xor(most, sh, JAM_WAVE));
+        big += __shfl_xor(big, sh, JAM_WAVE);
+    }
+    if (lane == 0) {
+        part[0][threadIdx.x / JAM_WAVE] = sum;
+        part[1][threadIdx.x / JAM_WAVE] = most;
+        part[2][threadIdx.x / JAM_WAVE] = big;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < 256 / JAM_WAVE; q++) {
+            sum += part[0][q];
+            most = max(most, part[1][q]);
+            big += part[2][q];
+        }
+        if (sum) {
+            atomicAdd(&work[0], sum);
+            atomicMax(&work[1], most);
+        }
+        if (big) atomicAdd(&work[2], big);
+    }
+}
+
+// One word of the key of complete match i: `head` in its first `used` bits,
+// then the kd positions of as many levels from l on as fit, each in the bits
+// its pair's set needs (the same for every match of a pair); `l` moves past
+// them.
+__device__ static inline unsigned long long group_key(const DevTpls &tp, const DevPairs &pr, const DevJoin &jn, int i,
+                                                      unsigned long long head, int used, int &l)
+{
+    const int p = jn.done_pair[i];
+    const int t = p % tp.n_templates;
+    const int nt = tp.atom_off[t + 1] - tp.atom_off[t];
+    const int *ent = jn.done_ent + (long long)i * jn.stride;
+    const PairLevel *lv = pr.lvl + (size_t)p * JAM_MAX_LEVELS;
+    unsigned long long k = head;
+    while (l < nt) {
+        const PairLevel h = lv[l];
+        const int w = 32 - __clz(h.cnt - 1);   // 0 for one entry (cnt >= 1)
+        if (used + w > 64) break;
+        k = (k << w) | (unsigned int)(ent[l] - h.off);
+        used += w;
+        l++;
+    }
+    return used > 0 ? k << (64 - used) : 0ull;
+}
+
+// A match's group in the sorted order: first position, matches, and the next
+// level its key goes on with.
+struct GroupSeg {
+    int begin;
+    unsigned int size_level;   // matches * 64 + level
+};
+
+// Matches and groups, by group; the first key words of the groups of at least
+// `least` matches (the others are sorted by k_group_tile).
+__global__ void __launch_bounds__(256) k_group_scatter(DevTpls tp, DevPairs pr, DevJoin jn, long long n, int shift,
+                                                       int least, const unsigned int *row, const int *slot,
+                                                       const int *start, int *match, unsigned long long *key,
+                                                       GroupSeg *seg)
+{
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const unsigned int r = row[i], g = r >> shift;
+    const int a = start[g], c = start[g + 1] - a;
+    const long long d = a + slot[i];
+    int l = 1;
+    match[d] = (int)i;
+    if (c >= least) key[d] = group_key(tp, pr, jn, (int)i, r & ((1u << shift) - 1u), shift, l);
+    seg[d] = GroupSeg{a, (unsigned int)c * 64u + (unsigned int)l};
+}
+
+// The positions of the groups of at least `least` matches, neighbours
+// together: waves that rank one group at the same time read its words from L1.
+__global__ void __launch_bounds__(256) k_group_list(const GroupSeg *seg, long long n, int least, int *list,
+                                                    unsigned long long *n_list)
+{
+    const long long d = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const bool listed = d < n && (int)(seg[d].size_level >> 6) >= least;
+    const unsigned long long m = ballot(listed);
+    if (m == 0ull) return;
+    unsigned long long base = 0;
+    if (lane_id() == 0) base = atomicAdd(n_list, (unsigned long long)__popcll(m));
+    base = __shfl(base, 0, JAM_WAVE);
+    if (listed) list[base + rank_below(m)] = (int)d;
+}
+
+// One pass over the key words of the matches at the listed positions (all of
+// them without a list; the positions of a group stay its own from pass to
+// pass): a match's position is its group's start, plus the smaller words, plus
+// the equal ones before it; the equal ones are its group in the next pass,
+// with the next word (none after the last pass, which writes to `match_out`
+// what the caller reads). A wave per match, a lane per word of the group: with
+// a thread per match, one group of 23,747 matches took 1.3 ms a pass, a chain
+// of as many loads.
+__global__ void __launch_bounds__(256) k_group_rank(DevTpls tp, DevPairs pr, DevJoin jn, long long n,
+                                                    const int *list, const unsigned long long *n_list,
+                                                    const int *match_in, const unsigned long long *key_in,
+                                                    const GroupSeg *seg_in, int *match_out,
+                                                    unsigned long long *key_out, GroupSeg *seg_out)
+{
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / JAM_WAVE), lane = lane_id();
+    if (list) n = (long long)*n_list;
+    for (long long q = (long long)blockIdx.x * (256 / JAM_WAVE) + w; q < n; q += (long long)gridDim.x * (256 / JAM_WAVE)) {
+        const long long d = list ? list[q] : q;
+        const GroupSeg s = seg_in[d];
+        const int i = match_in[d], c = (int)(s.size_level >> 6);
+        long long o = d;
+        int begin = s.begin, equal = 1, l = (int)(s.size_level & 63u);
+        if (c > 1) {
+            const unsigned long long mine = key_in[d];
+            const unsigned long long *k = key_in + s.begin;
+            const int self = (int)(d - s.begin);
+            int less = 0, before = 0;
+            equal = 0;
+#pragma unroll 4
+            for (int e0 = 0; e0 < c; e0 += JAM_WAVE) {
+                const int e = e0 + lane;
+                const unsigned long long x = e < c ? k[e] : ~0ull;
+                const unsigned long long eq = ballot(e < c && x == mine);
+                less += __popcll(ballot(x < mine));
+                equal += __popcll(eq);
+                const int lim = self - e0;   // lanes of earlier positions
+                before += lim >= JAM_WAVE ? __popcll(eq) : lim > 0 ? __popcll(eq & ((1ull << lim) - 1ull)) : 0;
+            }
+            begin = s.begin + less;
+            o = (long long)begin + before;
+        }
+        if (lane == 0) {
+            match_out[o] = i;
+            if (equal > 1) key_out[o] = group_key(tp, pr, jn, i, 0ull, 0, l);
+            seg_out[o] = GroupSeg{begin, (unsigned int)equal * 64u + (unsigned int)l};
+        }
+    }
+}
+
+// The groups of at most GROUP_TILE / 2 matches that start in the workgroup's
+// GROUP_TILE / 2 positions (together fewer than GROUP_TILE matches), sorted in
+// LDS by one bitonic sort per key word: a word starts with the position where
+// the match's group starts, so all groups are sorted at once, and matches
+// equal in it are the smaller groups of the next word; it ends when none are.
+__global__ void __launch_bounds__(1024) k_group_tile(DevTpls tp, DevPairs pr, DevJoin jn, long long n, int shift,
+                                                     const unsigned int *row, const int *match, const GroupSeg *seg,
+                                                     int *perm)
+{
+    constexpr int HALF = GROUP_TILE / 2, PER = GROUP_TILE / 1024;
+    constexpr int PBITS = __builtin_ctz(GROUP_TILE);
+    __shared__ unsigned long long key[GROUP_TILE];
+    __shared__ unsigned short idx[GROUP_TILE];
+    __shared__ unsigned char level[GROUP_TILE];   // next level of match `idx`'s key
+    const int t = threadIdx.x;
+    // the group that position x lies in belongs to this side of x when it
+    // starts there, or is too large and left out on both sides
+    auto bound = [&](long long x, bool begin) {
+        if (x >= n) return n;
+        const GroupSeg s = seg[x];
+        const long long e = (long long)s.begin + (s.size_level >> 6);
+        if ((int)(s.size_level >> 6) > HALF) return begin ? e : (long long)s.begin;
+        return s.begin == x ? x : e;
+    };
+    const long long a = bound((long long)blockIdx.x * HALF, true), b = bound((long long)(blockIdx.x + 1) * HALF, false);
+    if (a >= b) return;
+    const int c = (int)(b - a);
+    int n2 = 2;
+    while (n2 < c) n2 <<= 1;
+    for (int q = t; q < n2; q += 1024) {
+        unsigned long long k = ~0ull;
+        int l = 1;
+        if (q < c) {
+            const int i = match[a + q];
+            const unsigned int low = row[i] & ((1u << shift) - 1u);
+            const unsigned long long at = (unsigned long long)(seg[a + q].begin - a);
+            k = group_key(tp, pr, jn, i, (at << shift) | low, PBITS + shift, l);
+        }
+        key[q] = k;
+        idx[q] = (unsigned short)q;
+        level[q] = (unsigned char)l;
+    }
+    __syncthreads();
+    for (int word = 0; word < JAM_MAX_LEVELS; word++) {
+        for (int k = 2; k <= n2; k <<= 1) {
+            for (int j = k >> 1; j > 0; j >>= 1) {
+                for (int p = t; p < n2 / 2; p += 1024) {
+                    const int i = ((p & ~(j - 1)) << 1) | (p & (j - 1)), o = i | j;
+                    const unsigned long long u = key[i], v = key[o];
+                    if ((u > v) == ((i & k) == 0)) {
+                        key[i] = v;
+                        key[o] = u;
+                        const unsigned short x = idx[i];
+                        idx[i] = idx[o];
+                        idx[o] = x;
+                    }
+                }
+                __syncthreads();
+            }
+        }
+        // the next word: equal neighbours go on from where their run starts
+        unsigned long long next[PER];
+        bool tie = false;
+#pragma unroll
+        for (int z = 0; z < PER; z++) {
+            const int q = t + z * 1024;
+            if (q >= c) break;
+            const unsigned long long x = key[q];
+            next[z] = (unsigned long long)q << (64 - PBITS);
+            if ((q > 0 && key[q - 1] == x) || (q + 1 < c && key[q + 1] == x)) {
+                tie = true;
+                int lo = 0, hi = q;   // the first position with this key
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (key[mid] < x) lo = mid + 1;
+                    else hi = mid;
+                }
+                int l = level[idx[q]];
+                next[z] = group_key(tp, pr, jn, match[a + idx[q]], (unsigned long long)lo, PBITS, l);
+                level[idx[q]] = (unsigned char)l;
+            }
+        }
+        if (!__syncthreads_or(tie)) break;
+#pragma unroll
+        for (int z = 0; z < PER; z++) {
+            const int q = t + z * 1024;
+            if (q < c) key[q] = next[z];
+        }
+        __syncthreads();
+    }
+    for (int q = t; q < c; q += 1024) perm[a + q] = match[a + idx[q]];
 }
 
 // first sorted position of every pair with complete matches
