@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -172,10 +173,11 @@ struct jam_context {
     // incremented by every query: a result's events live in e_* until the
     // next query on the context
     uint64_t query_gen = 0;
-    // pinned host staging for event copies: two halves of JAM_STAGE_BYTES,
-    // device-to-host copies into one half while the other is unpacked
+    // pinned host staging for event copies: stage_slots slots of
+    // JAM_STAGE_BYTES
     void *hstage = nullptr;
-    hipEvent_t stage_ev[2] = {};
+    int stage_slots = 0;
+    hipEvent_t stage_ev[16] = {};
     // pinned host words the device's counters are read back into
     unsigned long long *hsmall = nullptr;
     int64_t hsmall_cap = 0;
@@ -186,7 +188,7 @@ struct jam_context {
     // per-pair hit counts and digests of jam_result_pair_digests
     DBuf dig;
     // temporary buffers of jam_molecules_parse_pdb, kept for the next parse
-    DBuf g_buf, g_toff, g_nl, g_blk, g_blkoff, g_starts, g_kind, g_textof, g_first, g_lineatom, g_atomline, g_textrng;
+    DBuf g_buf, g_toff, g_blk, g_blkoff, g_starts, g_kind, g_textof, g_first, g_lineatom, g_atomline, g_textrng;
     DBuf g_err, g_firsterr, g_keys, g_nnames, g_resoff64, g_bucket, g_bcount, g_bstart, g_skey, g_sval;
     std::vector<std::unique_ptr<DBuf>> g_scan;
     // jam_molecules_create: two pinned halves of up_half bytes, one packed
@@ -746,6 +748,123 @@ extern "C" void jam_molecules_free(jam_molecules *m)
 }
 
 // ---------------------------------------------------------------------------
+// copies to the host
+// ---------------------------------------------------------------------------
+
+namespace {
+
+// Copies to the caller's memory go through pinned slots of JAM_STAGE_BYTES, two per host thread:
+// a thread unpacks one while the other is on its way from the device. 4 MB:
+// about 80 us of transfer, well above what issuing one takes, and small enough
+// that 64 MB keep eight threads unpacking while they arrive (two
+// halves of 64 MB had the unpacking of most copies wait for the whole
+// transfer).
+constexpr size_t JAM_STAGE_BYTES = size_t(4) << 20;
+constexpr int JAM_STAGE_THREADS = 8;
+
+struct CopyPiece {
+    void *dst;
+    const char *src;
+    size_t bytes;
+};
+
+// a field of `bytes` bytes at `src` for `dst` (may be NULL), cut into pieces of
+// at most one slot
+void add_pieces(std::vector<CopyPiece> &pieces, void *dst, const char *src, size_t bytes)
+{
+    if (!dst) return;
+    for (size_t o = 0; o < bytes; o += JAM_STAGE_BYTES)
+        pieces.push_back({(char *)dst + o, src + o, std::min(JAM_STAGE_BYTES, bytes - o)});
+}
+
+// pinned slots and their events, grown to `n` slots
+int32_t grow_stage(jam_context *c, int n)
+{
+    if (n <= c->stage_slots) return JAM_OK;
+    if (c->hstage) HIP_TRY(hipHostFree(c->hstage));
+    c->hstage = nullptr;
+    c->stage_slots = 0;
+    for (int k = 0; k < n; k++)
+        if (!c->stage_ev[k]) HIP_TRY(hipEventCreateWithFlags(&c->stage_ev[k], hipEventDisableTiming));
+    HIP_TRY(hipHostMalloc(&c->hstage, JAM_STAGE_BYTES * (size_t)n, hipHostMallocDefault));
+    c->stage_slots = n;
+    return JAM_OK;
+}
+
+// Copies the pieces (device to host) through the context's pinned slots, on
+// the context's stream, and waits for them.
+int32_t copy_out(jam_context *c, const std::vector<CopyPiece> &pieces)
+{
+    hipStream_t s = c->stream;
+    // batches of consecutive pieces, one slot each
+    struct Batch {
+        size_t first, last;
+    };
+    std::vector<Batch> batches;
+    for (size_t i = 0; i < pieces.size();) {
+        size_t used = 0, j = i;
+        while (j < pieces.size() && used + pieces[j].bytes <= JAM_STAGE_BYTES) used += pieces[j++].bytes;
+        batches.push_back({i, j});
+        i = j;
+    }
+    if (batches.empty()) return JAM_OK;
+    const int nt = (int)std::min<size_t>(JAM_STAGE_THREADS, (batches.size() + 1) / 2);
+    int32_t rc = grow_stage(c, (int)std::min<size_t>(batches.size(), 2 * (size_t)nt));
+    if (rc != JAM_OK) return rc;
+    auto issue = [&](const Batch &b, int slot) -> hipError_t {
+        char *h = (char *)c->hstage + (size_t)slot * JAM_STAGE_BYTES;
+        size_t o = 0;
+        for (size_t i = b.first; i < b.last;) {
+            // one transfer for every run of pieces contiguous on the device
+            size_t j = i + 1, bytes = pieces[i].bytes;
+            while (j < b.last && pieces[j].src == pieces[j - 1].src + pieces[j - 1].bytes) bytes += pieces[j++].bytes;
+            hipError_t e = hipMemcpyAsync(h + o, pieces[i].src, bytes, hipMemcpyDeviceToHost, s);
+            if (e != hipSuccess) return e;
+            o += bytes;
+            i = j;
+        }
+        return hipEventRecord(c->stage_ev[slot], s);
+    };
+    // thread w takes the batches w, w + nt, ...: its k-th in slot
+    // w + nt * (k & 1), issued two of its turns ahead (the first ones here, in
+    // order)
+    for (size_t k = 0; k < std::min<size_t>(batches.size(), 2 * (size_t)nt); k++) HIP_TRY(issue(batches[k], (int)k));
+    std::atomic<int> failed{(int)hipSuccess};
+    auto work = [&](size_t w) {
+        hipError_t e = hipSetDevice(c->device);
+        int turn = 0;
+        for (size_t k = w; k < batches.size() && e == hipSuccess; k += (size_t)nt, turn ^= 1) {
+            const int slot = (int)w + nt * turn;
+            e = hipEventSynchronize(c->stage_ev[slot]);
+            if (e != hipSuccess) break;
+            const char *h = (const char *)c->hstage + (size_t)slot * JAM_STAGE_BYTES;
+            size_t o = 0;
+            for (size_t i = batches[k].first; i < batches[k].last; i++) {
+                std::memcpy(pieces[i].dst, h + o, pieces[i].bytes);
+                o += pieces[i].bytes;
+            }
+            if (k + 2 * (size_t)nt < batches.size()) e = issue(batches[k + 2 * (size_t)nt], slot);
+        }
+        if (e != hipSuccess) failed.store((int)e);
+    };
+    std::vector<std::thread> th;
+    int started = 1;
+    try {
+        th.reserve((size_t)nt);
+        for (; started < nt; started++) th.emplace_back(work, (size_t)started);
+    } catch (...) {
+        // no more threads: their batches are done here
+    }
+    work(0);
+    for (int w = started; w < nt; w++) work((size_t)w);
+    for (auto &x : th) x.join();
+    HIP_TRY((hipError_t)failed.load());
+    return JAM_OK;
+}
+
+}  // namespace
+
+// ---------------------------------------------------------------------------
 // PDB ingestion on the device
 // ---------------------------------------------------------------------------
 
@@ -829,13 +948,6 @@ __global__ void k_fill_u64(unsigned long long *v, long long n, unsigned long lon
 {
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
         v[i] = x;
-}
-
-// a line feed at each of the n positions of buf
-__global__ void k_put_newlines(const long long *pos, long long n, unsigned char *buf)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) buf[pos[i]] = '\n';
 }
 
 __global__ void k_fill_i32(int *v, long long n, int x)
@@ -985,12 +1097,12 @@ extern "C" int32_t jam_molecules_parse_pdb(jam_context *c, const char *const *te
     if (flags & ~(JAM_PDB_SKIP_HETATM | JAM_PDB_IGNORE_ENDMDL)) return fail(JAM_EINVAL, "unknown flags");
     // where the texts go on the device: each one's bytes, then a line feed
     // when it does not end with one (its last line ends there)
-    std::vector<long long> toff(n + 1, 0), nl;
+    std::vector<long long> toff(n + 1, 0);
     for (int32_t k = 0; k < n; k++) {
         if (lengths[k] < 0 || (lengths[k] > 0 && !texts[k]))
             return fail(JAM_EINVAL, "text " + std::to_string(k) + ": negative length or NULL text");
         toff[k + 1] = toff[k] + lengths[k];
-        if (lengths[k] > 0 && texts[k][lengths[k] - 1] != '\n') nl.push_back(toff[k + 1]++);
+        if (lengths[k] > 0 && texts[k][lengths[k] - 1] != '\n') toff[k + 1]++;
     }
     HIP_TRY(hipSetDevice(c->device));
     hipStream_t s = c->stream;
@@ -1000,16 +1112,21 @@ extern "C" int32_t jam_molecules_parse_pdb(jam_context *c, const char *const *te
     M->parsed = true;
     std::vector<std::unique_ptr<DBuf>> &tmp = c->g_scan;
     HIP_TRY(c->g_buf.reserve((size_t)std::max<long long>(toff[n], 1)));
-    for (int32_t k = 0; k < n; k++)
-        if (lengths[k] > 0)
-            HIP_TRY(hipMemcpyAsync(c->g_buf.as<unsigned char>() + toff[k], texts[k], (size_t)lengths[k],
-                                   hipMemcpyHostToDevice, s));
-    if (!nl.empty()) {
-        HIP_TRY(upload(c->g_nl, nl, s));
-        hipLaunchKernelGGL(k_put_newlines, dim3((unsigned)((nl.size() + 255) / 256)), dim3(256), 0, s,
-                           c->g_nl.as<const long long>(), (long long)nl.size(), c->g_buf.as<unsigned char>());
+    {
+        // through the pinned halves, which the copy of the offsets waits for;
+        // the line feeds that are missing as parts of their own
+        std::lock_guard<std::mutex> guard(c->up_mutex);
+        static const char newline = '\n';
+        std::vector<UploadPart> parts;
+        for (int32_t k = 0; k < n; k++) {
+            if (lengths[k] > 0) parts.push_back({(size_t)toff[k], texts[k], (size_t)lengths[k]});
+            if (toff[k + 1] - toff[k] > lengths[k]) parts.push_back({(size_t)(toff[k + 1] - 1), &newline, 1});
+        }
+        int32_t up = upload_parts(c, parts, (size_t)toff[n], c->g_buf.as<char>(), s);
+        if (up == JAM_OK) HIP_TRY(upload(c->g_toff, toff, s));
+        else (void)hipStreamSynchronize(s);
+        if (up != JAM_OK) return up;
     }
-    HIP_TRY(upload(c->g_toff, toff, s));
     jam::IngText tx;
     tx.buf = c->g_buf.as<const unsigned char>();
     tx.n_bytes = toff[n];
@@ -1237,26 +1354,22 @@ extern "C" int32_t jam_molecules_copy_atoms(const jam_molecules *m, const jam_at
                        f->element || f->charge;
     if (extra && !m->parsed) return fail(JAM_EINVAL, "only molecules parsed on the device keep every atom field");
     HIP_TRY(hipSetDevice(m->ctx->device));
-    hipStream_t s = m->ctx->stream;
-    auto get = [&](void *dst, const DBuf &src, size_t bytes) -> hipError_t {
-        if (!dst) return hipSuccess;
-        return hipMemcpyAsync(dst, src.ptr, bytes, hipMemcpyDeviceToHost, s);
-    };
-    HIP_TRY(get(f->xyz, m->xyz, sizeof(double) * 3 * na));
-    HIP_TRY(get(f->names, m->name, 4 * na));
-    HIP_TRY(get(f->resnames, m->resname, 4 * na));
-    HIP_TRY(get(f->resseq, m->resseq, sizeof(int) * na));
-    HIP_TRY(get(f->chains, m->chains, 2 * na));
-    HIP_TRY(get(f->serial, m->serial, sizeof(int) * na));
-    HIP_TRY(get(f->altloc, m->altloc, na));
-    HIP_TRY(get(f->icode, m->icode, na));
-    HIP_TRY(get(f->occupancy, m->occupancy, sizeof(float) * na));
-    HIP_TRY(get(f->tempfactor, m->tempfactor, sizeof(float) * na));
-    HIP_TRY(get(f->segid, m->segid, 4 * na));
-    HIP_TRY(get(f->element, m->element, 2 * na));
-    HIP_TRY(get(f->charge, m->charge, sizeof(int) * na));
-    HIP_TRY(hipStreamSynchronize(s));
-    return JAM_OK;
+    std::vector<CopyPiece> pieces;
+    auto get = [&](void *dst, const DBuf &src, size_t bytes) { add_pieces(pieces, dst, src.as<const char>(), bytes); };
+    get(f->xyz, m->xyz, sizeof(double) * 3 * na);
+    get(f->names, m->name, 4 * na);
+    get(f->resnames, m->resname, 4 * na);
+    get(f->resseq, m->resseq, sizeof(int) * na);
+    get(f->chains, m->chains, 2 * na);
+    get(f->serial, m->serial, sizeof(int) * na);
+    get(f->altloc, m->altloc, na);
+    get(f->icode, m->icode, na);
+    get(f->occupancy, m->occupancy, sizeof(float) * na);
+    get(f->tempfactor, m->tempfactor, sizeof(float) * na);
+    get(f->segid, m->segid, 4 * na);
+    get(f->element, m->element, 2 * na);
+    get(f->charge, m->charge, sizeof(int) * na);
+    return copy_out(m->ctx, pieces);
 }
 
 extern "C" int32_t jam_molecules_residue_index(const jam_molecules *m, int32_t *perm, int32_t *res_off,
@@ -2153,60 +2266,19 @@ extern "C" int32_t jam_result_stride(const jam_result *r) { return r ? r->stride
 
 extern "C" int32_t jam_result_n_pairs(const jam_result *r) { return r ? r->n_pairs : 0; }
 
-namespace {
-
-constexpr size_t JAM_STAGE_BYTES = size_t(64) << 20;
-
-// memcpy spread over a few host threads when it is large
-void host_copy(void *dst, const void *src, size_t bytes)
-{
-    const size_t per = size_t(16) << 20;
-    const unsigned nt = (unsigned)std::min<size_t>(8, bytes / per);
-    if (nt < 2) {
-        std::memcpy(dst, src, bytes);
-        return;
-    }
-    std::vector<std::thread> th;
-    const size_t part = (bytes + nt - 1) / nt;
-    for (unsigned k = 0; k < nt; k++) {
-        const size_t b0 = k * part, b1 = std::min(bytes, b0 + part);
-        if (b0 < b1)
-            th.emplace_back([=] { std::memcpy((char *)dst + b0, (const char *)src + b0, b1 - b0); });
-    }
-    for (auto &x : th) x.join();
-}
-
-struct CopyPiece {
-    void *dst;
-    const char *src;
-    size_t bytes;
-};
-
-}  // namespace
-
 // Copies the fields of n events packed at `base` (device memory, the layout
 // of event_layout(n, stride)) to host buffers (any may be NULL) through the
-// context's pinned staging halves, on the context's stream.
+// context's pinned slots, on the context's stream.
 static int32_t copy_event_fields(jam_context *c, const char *base, size_t n, int stride, int32_t *pair,
                                  int64_t *rank, int32_t *flag, double *rmsd, double *rot, double *c0, double *c1,
                                  int32_t *atoms)
 {
     HIP_TRY(hipSetDevice(c->device));
-    hipStream_t s = c->stream;
-    if (!c->hstage) {
-        HIP_TRY(hipHostMalloc(&c->hstage, 2 * JAM_STAGE_BYTES, hipHostMallocDefault));
-        for (auto &ev : c->stage_ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    }
-    // the fields, cut into pieces of at most one staging half
-    // (in the order of the packed layout, so that neighbouring pieces are
-    // contiguous on the device)
+    // in the order of the packed layout, so that neighbouring pieces are
+    // contiguous on the device
     std::vector<CopyPiece> pieces;
     const EventLayout L = event_layout((int64_t)n, stride);
-    auto add = [&](void *dst, size_t at, size_t bytes) {
-        if (!dst) return;
-        for (size_t o = 0; o < bytes; o += JAM_STAGE_BYTES)
-            pieces.push_back({(char *)dst + o, base + at + o, std::min(JAM_STAGE_BYTES, bytes - o)});
-    };
+    auto add = [&](void *dst, size_t at, size_t bytes) { add_pieces(pieces, dst, base + at, bytes); };
     add(rank, L.rank, sizeof(int64_t) * n);
     add(rmsd, L.rmsd, sizeof(double) * n);
     add(rot, L.rot, sizeof(double) * 9 * n);
@@ -2215,45 +2287,7 @@ static int32_t copy_event_fields(jam_context *c, const char *base, size_t n, int
     add(pair, L.pair, sizeof(int32_t) * n);
     add(flag, L.flag, sizeof(int32_t) * n);
     add(atoms, L.atoms, sizeof(int32_t) * (size_t)stride * n);
-    // batches of consecutive pieces filling one half each; the copy of batch
-    // k + 1 runs while batch k is unpacked from the other half
-    struct Batch {
-        size_t first, last, half;
-    };
-    std::vector<Batch> batches;
-    for (size_t i = 0; i < pieces.size();) {
-        size_t used = 0, j = i;
-        while (j < pieces.size() && used + pieces[j].bytes <= JAM_STAGE_BYTES) used += pieces[j++].bytes;
-        batches.push_back({i, j, batches.size() & 1});
-        i = j;
-    }
-    auto issue = [&](const Batch &b) -> hipError_t {
-        char *h = (char *)c->hstage + b.half * JAM_STAGE_BYTES;
-        size_t o = 0;
-        for (size_t i = b.first; i < b.last;) {
-            // one transfer for every run of pieces contiguous on the device
-            size_t j = i + 1, bytes = pieces[i].bytes;
-            while (j < b.last && pieces[j].src == pieces[j - 1].src + pieces[j - 1].bytes) bytes += pieces[j++].bytes;
-            hipError_t e = hipMemcpyAsync(h + o, pieces[i].src, bytes, hipMemcpyDeviceToHost, s);
-            if (e != hipSuccess) return e;
-            o += bytes;
-            i = j;
-        }
-        return hipEventRecord(c->stage_ev[b.half], s);
-    };
-    if (!batches.empty()) HIP_TRY(issue(batches[0]));
-    for (size_t k = 0; k < batches.size(); k++) {
-        if (k + 1 < batches.size()) HIP_TRY(issue(batches[k + 1]));
-        const Batch &b = batches[k];
-        HIP_TRY(hipEventSynchronize(c->stage_ev[b.half]));
-        const char *h = (const char *)c->hstage + b.half * JAM_STAGE_BYTES;
-        size_t o = 0;
-        for (size_t i = b.first; i < b.last; i++) {
-            host_copy(pieces[i].dst, h + o, pieces[i].bytes);
-            o += pieces[i].bytes;
-        }
-    }
-    return JAM_OK;
+    return copy_out(c, pieces);
 }
 
 extern "C" int32_t jam_result_copy(const jam_result *r, int32_t *pair, int64_t *rank, int32_t *flag,
