@@ -126,7 +126,8 @@ void jam_molecules_free(jam_molecules *m);
  * JAM_EINVAL, naming the text and line, for an mmCIF data tag, a numeric
  * field that does not parse (or that uses a form other than decimal digits
  * with an optional point and exponent), or a byte above 0x7F in the first 80
- * columns of a record. HEADER records are not read. The context keeps the
+ * columns of a record. HEADER records are not read (jam_molecules_pdb_headers
+ * says where they are). The context keeps the
  * parse's temporary device buffers for its next parse. */
 int32_t jam_molecules_parse_pdb(jam_context *ctx, const char *const *texts, const int64_t *lengths, int32_t n,
                                 int32_t flags, jam_molecules **out);
@@ -149,6 +150,15 @@ typedef struct {
     char *element;
     int32_t *charge;
 } jam_atom_fields;
+
+/* What the host needs of the texts beside their atoms: whether no byte of them
+ * is above 0x7F (`ascii`), and where the HEADER records lie that
+ * PDBMoleculeParser.load would read (src/pyjess/_io.py:81-92; text and offset
+ * in it, ascending): their number `n`, the first `cap` of them in `text` and
+ * `offset`. `known` is 0 where the texts hold too many HEADER records to keep.
+ * Any of the three words may be NULL. */
+int32_t jam_molecules_pdb_headers(const jam_molecules *m, int32_t *ascii, int32_t *known, int32_t *text,
+                                  int64_t *offset, int32_t cap, int32_t *n);
 
 /* Atom offsets of the molecules of a batch (n + 1 entries) and the number
  * of residue-name buckets (either may be NULL). No reference counterpart. */

@@ -119,11 +119,16 @@ def _pdb_header(data: bytes, id_, date, name, ignore_endmdl: bool):
     end = len(data)
     if not ignore_endmdl:
         end = next(_record_starts(data, b"ENDMDL", end), end)
-    for i in _record_starts(data, b"HEADER", end):
+    return _header_fields(data, _record_starts(data, b"HEADER", end), id_, date, name)
+
+
+def _header_fields(data: bytes, starts, id_, date, name):
+    """id, date and name from the HEADER records at the offsets ``starts``."""
+    for i in starts:
         j = len(data)
         for sep in (b"\n", b"\r"):
-            k = data.find(sep, i)
-            if 0 <= k < j:
+            k = data.find(sep, i, j)
+            if k >= 0:
                 j = k
         line = data[i:j].decode("utf-8")
         if id_ is None:
@@ -676,10 +681,22 @@ class Molecule:
         from . import _native
 
         ctx = _native.context()
-        # the header fields come from the text (decoding also rejects what a
-        # text-mode read would)
-        heads = [_pdb_header(d, *h, ignore_endmdl) for d, h in zip(datas, headers)]
-        batch = _native.ParsedMolecules(ctx, datas, skip_hetatm=skip_hetatm, ignore_endmdl=ignore_endmdl)
+        # the header fields come from the text, from where the device found
+        # the records; a text with bytes above 0x7F is decoded, to reject what
+        # a text-mode read would, and where the parse fails the header's own
+        # errors come first
+        scan = [lambda d=d, h=h: _pdb_header(d, *h, ignore_endmdl) for d, h in zip(datas, headers)]
+        try:
+            batch = _native.ParsedMolecules(ctx, datas, skip_hetatm=skip_hetatm, ignore_endmdl=ignore_endmdl)
+        except Exception:
+            for f in scan:
+                f()
+            raise
+        is_ascii, starts = batch.headers()
+        if is_ascii and starts is not None:
+            heads = [_header_fields(d, at, *h) for d, at, h in zip(datas, starts, headers)]
+        else:
+            heads = [f() for f in scan]
         off = batch.atom_offsets()
         a = batch.arrays()
         mols = []

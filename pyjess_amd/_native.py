@@ -29,7 +29,7 @@ MAX_TEMPLATE_ATOMS = 32
 _SYMBOLS = (
     "jam_context_create", "jam_context_free", "jam_templates_create", "jam_templates_free",
     "jam_molecules_create", "jam_molecules_free", "jam_molecules_parse_pdb",
-    "jam_molecules_sizes", "jam_molecules_copy_atoms", "jam_molecules_residue_index", "jam_query", "jam_result_n_events",
+    "jam_molecules_sizes", "jam_molecules_pdb_headers", "jam_molecules_copy_atoms", "jam_molecules_residue_index", "jam_query", "jam_result_n_events",
     "jam_result_stride", "jam_result_n_pairs", "jam_result_copy", "jam_result_pair_matches",
     "jam_result_timings", "jam_result_pair_digests", "jam_result_join_kernels", "jam_context_set_profiling", "jam_result_level_partials", "jam_rmsd_forward",
     "jam_rmsd_backward", "jam_result_free", "jam_superpose_batch",
@@ -172,6 +172,8 @@ def lib():
         L.jam_molecules_sizes.restype = i32
         L.jam_molecules_copy_atoms.argtypes = [vp, P(AtomFields)]
         L.jam_molecules_copy_atoms.restype = i32
+        L.jam_molecules_pdb_headers.argtypes = [vp, P(i32), P(i32), vp, vp, i32, P(i32)]
+        L.jam_molecules_pdb_headers.restype = i32
         L.jam_molecules_residue_index.argtypes = [vp, vp, vp, vp, vp, vp]
         L.jam_molecules_residue_index.restype = i32
         L.jam_result_keep.argtypes = [vp, P(vp)]
@@ -378,6 +380,20 @@ class ParsedMolecules(MoleculeSet):
         self.ctx = ctx
         self.handle = h
         self.n_molecules = len(texts)
+
+    def headers(self):
+        """Whether the texts are ASCII, and the offsets of each one's HEADER
+        records that a parse reads (None where there are too many to keep)."""
+        ascii_, known, n = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
+        text, offset = np.zeros(256, dtype=np.int32), np.zeros(256, dtype=np.int64)
+        _check(lib().jam_molecules_pdb_headers(self.handle, ctypes.byref(ascii_), ctypes.byref(known), _ptr(text),
+                                               _ptr(offset), len(text), ctypes.byref(n)))
+        if not known.value or n.value > len(text):
+            return bool(ascii_.value), None
+        starts = [[] for _ in range(self.n_molecules)]
+        for t, o in zip(text[:n.value].tolist(), offset[:n.value].tolist()):
+            starts[t].append(o)
+        return bool(ascii_.value), starts
 
     def arrays(self) -> dict:
         """Every atom field of the batch, as numpy arrays (all molecules)."""

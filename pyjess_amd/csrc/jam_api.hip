@@ -188,8 +188,8 @@ struct jam_context {
     // per-pair hit counts and digests of jam_result_pair_digests
     DBuf dig;
     // temporary buffers of jam_molecules_parse_pdb, kept for the next parse
-    DBuf g_buf, g_toff, g_blk, g_blkoff, g_starts, g_kind, g_textof, g_first, g_lineatom, g_atomline, g_textrng;
-    DBuf g_err, g_firsterr, g_keys, g_nnames, g_resoff64, g_bucket, g_bcount, g_bstart, g_skey, g_sval;
+    DBuf g_buf, g_blk, g_blkoff, g_starts, g_kind, g_textof, g_back, g_lineatom, g_atomline;
+    DBuf g_err, g_firsterr, g_skey, g_sval;
     std::vector<std::unique_ptr<DBuf>> g_scan;
     // jam_molecules_create: two pinned halves of up_half bytes, one packed
     // while the other is on its way to the device, and the index's temporary
@@ -239,6 +239,10 @@ struct jam_molecules {
     DBuf atom_off, xyz, name, resname, chain, resseq, perm, res_off, res_key, res_begin, res_end;
     // the other atom fields, kept by jam_molecules_parse_pdb for the host's copy
     bool parsed = false;
+    // of the parsed texts: no byte above 0x7F; HEADER records read (text,
+    // offset in it), if there were few enough to keep
+    bool ascii = true, headers_known = true;
+    std::vector<std::pair<int, long long>> headers;
     DBuf serial, chains, altloc, icode, occupancy, tempfactor, segid, element, charge;
     DevMols dev() const
     {
@@ -513,7 +517,7 @@ extern "C" void jam_templates_free(jam_templates *t)
 
 namespace {
 int32_t residue_index(jam_context *c, jam_molecules *M, const int *order, void *perm, void *res_off, hipStream_t s,
-                      bool &done);
+                      int &refused);
 }
 
 // ---------------------------------------------------------------------------
@@ -706,16 +710,16 @@ int32_t create_molecules(jam_context *ctx, const jam_molecule_desc *mols, int32_
     add(o_chain8, 1, [](const jam_molecule_desc &d) { return (const void *)d.chain2; });
     if (!order.empty()) parts.push_back({o_order, order.data(), sizeof(int) * na});
     int32_t rc = upload_parts(ctx, parts, image, base, s);
-    bool on_device = false;
+    int refused = 0;   // a batch without molecules has nothing to launch
     if (rc == JAM_OK && n > 0) {
         if (na > 0)
             hipLaunchKernelGGL(jam::k_chain_words, dim3((unsigned)((na + ING_THREADS - 1) / ING_THREADS)),
                                dim3(ING_THREADS), 0, s, (const signed char *)(base + o_chain8), (long long)na,
                                M->chain.as<int>());
         rc = residue_index(ctx, M.get(), order.empty() ? nullptr : (const int *)(base + o_order), base + o_perm,
-                           base + o_resoff, s, on_device);
+                           base + o_resoff, s, refused);
     }
-    if (rc == JAM_OK && !on_device) rc = host_residue_index(mols, n, M.get(), s);
+    if (rc == JAM_OK && refused >= 0) rc = host_residue_index(mols, n, M.get(), s);
     // the pinned halves are free again, and so is the memory of a batch that
     // is given up, only once its transfers are over
     const hipError_t e = hipStreamSynchronize(s);
@@ -1044,13 +1048,13 @@ int32_t read_one(const T *dev, T &host, hipStream_t s)
     return JAM_OK;
 }
 
-// The residue-name index of M (atom_off and resname on the device) by
-// k_residue_index, into perm and res_off where they are given (space in M's
-// block) and arrays of the exact size. `done` stays false where a molecule has
-// more names than the kernel holds. Synchronises once, for the number of
-// groups.
+// The residue-name index of M (atom_off and resname on the device, n_mols > 0)
+// by k_residue_index, into `perm` and `res_off` (space in M's block) and arrays
+// of the exact size. `refused`: a molecule with more than ING_MAX_NAMES names
+// (or with a name the kernel cannot hold), -1 if there is none and the index
+// is made. Synchronises, for the number of groups. The caller holds up_mutex.
 int32_t residue_index(jam_context *c, jam_molecules *M, const int *order, void *perm, void *res_off, hipStream_t s,
-                      bool &done)
+                      int &refused)
 {
     const int n = M->n_mols;
     const size_t na = (size_t)std::max<int64_t>(M->n_atoms, 1);
@@ -1060,20 +1064,27 @@ int32_t residue_index(jam_context *c, jam_molecules *M, const int *order, void *
     HIP_TRY(c->u_starts.reserve(sizeof(int) * na));
     HIP_TRY(c->u_nnames.reserve(sizeof(int) * (size_t)n));
     const int *aoff = M->atom_off.as<const int>();
-    hipLaunchKernelGGL(jam::k_residue_index<IDX_MAX_NAMES>, dim3((unsigned)n), dim3(IDX_THREADS), 0, s, aoff,
-                       M->resname.as<const uint32_t>(), order, M->perm.as<int>(), c->u_keys.as<uint32_t>(),
-                       c->u_starts.as<int>(), c->u_nnames.as<int>());
-    HIP_TRY(hipGetLastError());
     std::vector<int> names((size_t)n);
-    HIP_TRY(hipMemcpyAsync(names.data(), c->u_nnames.ptr, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost, s));
-    int32_t rc = device_scan<int, int>(c->u_nnames.as<const int>(), n, M->res_off.as<int>(), c->u_scan, 0, s);
-    HIP_TRY(hipStreamSynchronize(s));
-    if (rc != JAM_OK) return rc;
     int64_t total = 0;
-    for (int x : names) {
-        if (x < 0) return JAM_OK;
-        total += x;
+    refused = -1;
+    for (int big = 0; big < 2; big++) {
+        auto *index = big ? jam::k_residue_index<ING_MAX_NAMES> : jam::k_residue_index<IDX_MAX_NAMES>;
+        hipLaunchKernelGGL(index, dim3((unsigned)n), dim3(IDX_THREADS), 0, s, aoff, M->resname.as<const uint32_t>(), order,
+                           M->perm.as<int>(), c->u_keys.as<uint32_t>(), c->u_starts.as<int>(), c->u_nnames.as<int>());
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipMemcpyAsync(names.data(), c->u_nnames.ptr, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost, s));
+        const int32_t rc = device_scan<int, int>(c->u_nnames.as<const int>(), n, M->res_off.as<int>(), c->u_scan, 0, s);
+        HIP_TRY(hipStreamSynchronize(s));
+        if (rc != JAM_OK) return rc;
+        refused = -1;
+        total = 0;
+        for (int m = 0; m < n && refused < 0; m++) {
+            if (names[m] < 0) refused = m;
+            total += names[m];
+        }
+        if (refused < 0) break;
     }
+    if (refused >= 0) return JAM_OK;
     M->n_buckets = total;
     const size_t nb = (size_t)std::max<int64_t>(total, 1);
     HIP_TRY(M->res_key.reserve(3 * sizeof(uint32_t) * nb));
@@ -1083,7 +1094,6 @@ int32_t residue_index(jam_context *c, jam_molecules *M, const int *order, void *
                        c->u_keys.as<const uint32_t>(), c->u_starts.as<const int>(), M->res_off.as<const int>(),
                        M->res_key.as<uint32_t>(), M->res_begin.as<int>(), M->res_end.as<int>());
     HIP_TRY(hipGetLastError());
-    done = true;
     return JAM_OK;
 }
 
@@ -1111,40 +1121,56 @@ extern "C" int32_t jam_molecules_parse_pdb(jam_context *c, const char *const *te
     M->n_mols = n;
     M->parsed = true;
     std::vector<std::unique_ptr<DBuf>> &tmp = c->g_scan;
-    HIP_TRY(c->g_buf.reserve((size_t)std::max<long long>(toff[n], 1)));
+    // the texts, then (aligned) their offsets, through the pinned halves, which
+    // are free again after the first read-back below; line feeds that are
+    // missing as parts of their own
+    const size_t toff_at = ((size_t)toff[n] + 255) & ~(size_t)255;
+    const size_t image = toff_at + sizeof(long long) * toff.size();
+    HIP_TRY(c->g_buf.reserve(image));
+    std::unique_lock<std::mutex> guard(c->up_mutex);
     {
-        // through the pinned halves, which the copy of the offsets waits for;
-        // the line feeds that are missing as parts of their own
-        std::lock_guard<std::mutex> guard(c->up_mutex);
         static const char newline = '\n';
         std::vector<UploadPart> parts;
         for (int32_t k = 0; k < n; k++) {
             if (lengths[k] > 0) parts.push_back({(size_t)toff[k], texts[k], (size_t)lengths[k]});
             if (toff[k + 1] - toff[k] > lengths[k]) parts.push_back({(size_t)(toff[k + 1] - 1), &newline, 1});
         }
-        int32_t up = upload_parts(c, parts, (size_t)toff[n], c->g_buf.as<char>(), s);
-        if (up == JAM_OK) HIP_TRY(upload(c->g_toff, toff, s));
-        else (void)hipStreamSynchronize(s);
-        if (up != JAM_OK) return up;
+        parts.push_back({toff_at, toff.data(), sizeof(long long) * toff.size()});
+        const int32_t up = upload_parts(c, parts, image, c->g_buf.as<char>(), s);
+        if (up != JAM_OK) {
+            (void)hipStreamSynchronize(s);
+            return up;
+        }
     }
     jam::IngText tx;
     tx.buf = c->g_buf.as<const unsigned char>();
     tx.n_bytes = toff[n];
-    tx.text_off = c->g_toff.as<const long long>();
+    tx.text_off = (const long long *)(c->g_buf.as<const char>() + toff_at);
     tx.n_texts = n;
     tx.flags = flags;
     const long long per_block = (long long)ING_THREADS * ING_BPT;
     const long long byte_blocks = std::max<long long>(1, (tx.n_bytes + per_block - 1) / per_block);
+    // what the host reads back, one array: the info words, the texts' ranges,
+    // their first ENDMDL and mmCIF lines
+    const size_t nt = (size_t)std::max(n, 1);
+    const size_t w_line = ING_INFO_WORDS, w_atom = w_line + (size_t)n + 1, w_first = w_atom + (size_t)n + 1;
+    const size_t words = w_first + 2 * nt;
+    HIP_TRY(c->g_back.reserve(sizeof(unsigned long long) * words));
+    unsigned long long *info = c->g_back.as<unsigned long long>();
+    long long *text_line = (long long *)info + w_line, *text_atom = (long long *)info + w_atom;
+    unsigned long long *first_endmdl = info + w_first, *first_mmcif = first_endmdl + nt;
+    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(256), 0, s, info, 2ll, 0ull);
     // ---- lines
     HIP_TRY(c->g_blk.reserve(sizeof(long long) * (size_t)byte_blocks));
     HIP_TRY(c->g_blkoff.reserve(sizeof(long long) * (size_t)(byte_blocks + 1)));
     hipLaunchKernelGGL(jam::k_ing_count, dim3((unsigned)byte_blocks), dim3(ING_THREADS), 0, s, tx,
-                       c->g_blk.as<long long>());
+                       c->g_blk.as<long long>(), info);
     int32_t rc;
     if ((rc = device_scan<long long>(c->g_blk.as<long long>(), byte_blocks, c->g_blkoff.as<long long>(), tmp, 0, s)) != JAM_OK)
         return rc;
     long long n_lines = 0;
     if ((rc = read_one(c->g_blkoff.as<long long>() + byte_blocks, n_lines, s)) != JAM_OK) return rc;
+    guard.unlock();   // the upload is over
     if (tx.n_bytes == 0) n_lines = 0;
     const long long lines_cap = std::max<long long>(n_lines, 1);
     HIP_TRY(c->g_starts.reserve(sizeof(long long) * (size_t)lines_cap));
@@ -1154,21 +1180,18 @@ extern "C" int32_t jam_molecules_parse_pdb(jam_context *c, const char *const *te
     // ---- record kinds, first ENDMDL / mmCIF tag per text
     HIP_TRY(c->g_kind.reserve((size_t)lines_cap));
     HIP_TRY(c->g_textof.reserve(sizeof(int) * (size_t)lines_cap));
-    HIP_TRY(c->g_first.reserve(sizeof(unsigned long long) * 2 * (size_t)std::max(n, 1)));
-    unsigned long long *first_endmdl = c->g_first.as<unsigned long long>();
-    unsigned long long *first_mmcif = first_endmdl + std::max(n, 1);
-    hipLaunchKernelGGL(k_fill_u64, dim3(16), dim3(256), 0, s, first_endmdl, 2 * (long long)std::max(n, 1),
+    hipLaunchKernelGGL(k_fill_u64, dim3(16), dim3(256), 0, s, first_endmdl, 2 * (long long)nt,
                        (unsigned long long)n_lines);
     const long long line_blocks = std::max<long long>(1, (n_lines + ING_THREADS - 1) / ING_THREADS);
     if (n_lines > 0)
         hipLaunchKernelGGL(jam::k_ing_classify, dim3((unsigned)line_blocks), dim3(ING_THREADS), 0, s, tx,
                            c->g_starts.as<const long long>(), n_lines, c->g_kind.as<unsigned char>(), c->g_textof.as<int>(),
-                           first_endmdl, first_mmcif);
+                           first_endmdl, first_mmcif, info);
     // ---- atom records
     HIP_TRY(c->g_blk.reserve(sizeof(long long) * (size_t)line_blocks));
     HIP_TRY(c->g_blkoff.reserve(sizeof(long long) * (size_t)(line_blocks + 1)));
     HIP_TRY(c->g_lineatom.reserve(sizeof(long long) * (size_t)lines_cap));
-    long long n_atoms = 0;
+    HIP_TRY(c->g_atomline.reserve(sizeof(long long) * (size_t)lines_cap));
     if (n_lines > 0) {
         hipLaunchKernelGGL(jam::k_ing_select_count, dim3((unsigned)line_blocks), dim3(ING_THREADS), 0, s, tx,
                            c->g_kind.as<const unsigned char>(), c->g_textof.as<const int>(),
@@ -1176,56 +1199,72 @@ extern "C" int32_t jam_molecules_parse_pdb(jam_context *c, const char *const *te
         if ((rc = device_scan<long long>(c->g_blk.as<long long>(), line_blocks, c->g_blkoff.as<long long>(), tmp, 0, s)) !=
             JAM_OK)
             return rc;
-        if ((rc = read_one(c->g_blkoff.as<long long>() + line_blocks, n_atoms, s)) != JAM_OK) return rc;
-    }
-    if (n_atoms >= INT32_MAX) return fail(JAM_ETOOBIG, "too many atoms in one batch");
-    const long long atoms_cap = std::max<long long>(n_atoms, 1);
-    HIP_TRY(c->g_atomline.reserve(sizeof(long long) * (size_t)atoms_cap));
-    if (n_lines > 0)
         hipLaunchKernelGGL(jam::k_ing_select, dim3((unsigned)line_blocks), dim3(ING_THREADS), 0, s, tx,
                            c->g_kind.as<const unsigned char>(), c->g_textof.as<const int>(),
                            (const unsigned long long *)first_endmdl, n_lines, c->g_blkoff.as<const long long>(),
                            c->g_atomline.as<long long>(), c->g_lineatom.as<long long>());
-    HIP_TRY(c->g_textrng.reserve(sizeof(long long) * 2 * (size_t)(n + 1)));
-    long long *text_line = c->g_textrng.as<long long>(), *text_atom = text_line + (n + 1);
+    }
     hipLaunchKernelGGL(jam::k_ing_text_ranges, dim3((unsigned)((n + 1 + 63) / 64)), dim3(64), 0, s, tx,
-                       c->g_starts.as<const long long>(), n_lines, c->g_lineatom.as<const long long>(), n_atoms, text_line,
-                       text_atom);
+                       c->g_starts.as<const long long>(), n_lines, c->g_lineatom.as<const long long>(),
+                       c->g_blkoff.as<const long long>() + line_blocks, text_line, text_atom);
     HIP_TRY(hipGetLastError());
-    std::vector<long long> h_rng(2 * (size_t)(n + 1)), h_first(2 * (size_t)std::max(n, 1));
-    HIP_TRY(hipMemcpyAsync(h_rng.data(), text_line, sizeof(long long) * h_rng.size(), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(h_first.data(), first_endmdl, sizeof(long long) * h_first.size(), hipMemcpyDeviceToHost, s));
+    std::vector<long long> back(words);
+    HIP_TRY(hipMemcpyAsync(back.data(), info, sizeof(long long) * words, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
+    const long long *h_line = back.data() + w_line, *h_atom = back.data() + w_atom;
+    const long long *h_endmdl = back.data() + w_first, *h_mmcif = h_endmdl + nt;
     // an mmCIF tag before the parse stops (PDBMoleculeParser raises)
     for (int32_t k = 0; k < n; k++) {
-        const long long tag = h_first[std::max(n, 1) + k], end = h_first[k];
-        if (tag < n_lines && ((flags & JAM_PDB_IGNORE_ENDMDL) || tag < end))
+        if (h_mmcif[k] < n_lines && ((flags & JAM_PDB_IGNORE_ENDMDL) || h_mmcif[k] < h_endmdl[k]))
             return fail(JAM_EINVAL, "text " + std::to_string(k) + ": mmCIF data tags found, file is not in PDB format");
     }
-    std::vector<int> aoff(n + 1);
-    for (int32_t k = 0; k <= n; k++) aoff[k] = (int)h_rng[(size_t)(n + 1) + k];
+    const long long n_atoms = h_atom[n];
+    if (n_atoms >= INT32_MAX) return fail(JAM_ETOOBIG, "too many atoms in one batch");
+    // HEADER records read before the parse stops, in order
+    M->ascii = back[0] == 0;
+    M->headers_known = back[1] <= ING_HEADERS;
+    for (long long h = 0; M->headers_known && h < back[1]; h++) {
+        const long long li = back[2 + 2 * h];
+        const int t = (int)(std::upper_bound(toff.begin(), toff.end(), back[3 + 2 * h]) - toff.begin()) - 1;
+        if ((flags & JAM_PDB_IGNORE_ENDMDL) || li < h_endmdl[t])
+            M->headers.push_back({t, back[3 + 2 * h] - toff[t]});
+    }
+    std::sort(M->headers.begin(), M->headers.end());
     M->n_atoms = n_atoms;
-    // ---- fields
-    const size_t na = (size_t)atoms_cap;
-    HIP_TRY(upload(M->atom_off, aoff, s));
-    HIP_TRY(M->xyz.reserve(sizeof(double) * 3 * na));
-    HIP_TRY(M->name.reserve(4 * na));
-    HIP_TRY(M->resname.reserve(4 * na));
-    HIP_TRY(M->chain.reserve(sizeof(int) * na));
-    HIP_TRY(M->chains.reserve(2 * na));
-    HIP_TRY(M->resseq.reserve(sizeof(int) * na));
-    HIP_TRY(M->serial.reserve(sizeof(int) * na));
-    HIP_TRY(M->altloc.reserve(na));
-    HIP_TRY(M->icode.reserve(na));
-    HIP_TRY(M->occupancy.reserve(sizeof(float) * na));
-    HIP_TRY(M->tempfactor.reserve(sizeof(float) * na));
-    HIP_TRY(M->segid.reserve(4 * na));
-    HIP_TRY(M->element.reserve(2 * na));
-    HIP_TRY(M->charge.reserve(sizeof(int) * na));
+    // ---- fields: one block, those that the host copies side by side
+    const size_t na = (size_t)std::max<long long>(n_atoms, 1);
+    size_t bytes = 0;
+    auto place = [&](size_t b, size_t align) {
+        bytes = (bytes + align - 1) / align * align;
+        const size_t at = bytes;
+        bytes += b;
+        return at;
+    };
+    DBuf *const f8[] = {&M->xyz};
+    DBuf *const f4[] = {&M->name, &M->resname, &M->resseq, &M->serial, &M->occupancy, &M->tempfactor, &M->segid, &M->charge};
+    DBuf *const f2[] = {&M->chains, &M->element};
+    DBuf *const f1[] = {&M->altloc, &M->icode};
+    std::vector<std::tuple<DBuf *, size_t, size_t>> at_of;
+    auto field = [&](DBuf *f, size_t width, size_t align) { at_of.emplace_back(f, place(width * na, align), width * na); };
+    for (DBuf *f : f8) field(f, 24, 8);
+    for (DBuf *f : f4) field(f, 4, 4);
+    for (DBuf *f : f2) field(f, 2, 2);
+    for (DBuf *f : f1) field(f, 1, 1);
+    field(&M->chain, 4, 256);
+    const size_t o_perm = place(4 * na, 256), o_resoff = place(sizeof(int) * ((size_t)n + 1), 256);
+    const size_t o_off = place(sizeof(int) * ((size_t)n + 1), 256);
+    HIP_TRY(M->block.reserve(bytes));
+    char *blk = M->block.as<char>();
+    for (auto &x : at_of) std::get<0>(x)->view(blk + std::get<1>(x), std::get<2>(x));
+    M->atom_off.view(blk + o_off, sizeof(int) * ((size_t)n + 1));
+    hipLaunchKernelGGL(jam::k_ing_narrow, dim3((unsigned)((n + 1 + 255) / 256)), dim3(256), 0, s,
+                       (const long long *)text_atom, n + 1, M->atom_off.as<int>());
     HIP_TRY(c->g_err.reserve(sizeof(unsigned int) * na));
-    HIP_TRY(c->g_firsterr.reserve(sizeof(unsigned long long)));
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, c->g_firsterr.as<unsigned long long>(), 1ll,
-                       (unsigned long long)n_atoms);
+    HIP_TRY(c->g_firsterr.reserve(2 * sizeof(unsigned long long)));
+    // first atom in error; whether serial numbers descend
+    unsigned long long *state = c->g_firsterr.as<unsigned long long>();
+    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, state, 1ll, (unsigned long long)n_atoms);
+    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, state + 1, 1ll, 0ull);
     jam::IngAtoms at;
     at.xyz = M->xyz.as<double>();
     at.name = M->name.as<uint32_t>();
@@ -1242,91 +1281,88 @@ extern "C" int32_t jam_molecules_parse_pdb(jam_context *c, const char *const *te
     at.element = M->element.as<unsigned short>();
     at.charge = M->charge.as<int>();
     at.err = c->g_err.as<unsigned int>();
-    at.first_err = c->g_firsterr.as<unsigned long long>();
-    if (n_atoms > 0)
-        hipLaunchKernelGGL(jam::k_ing_parse, dim3((unsigned)((n_atoms + ING_THREADS - 1) / ING_THREADS)),
-                           dim3(ING_THREADS), 0, s, tx, c->g_starts.as<const long long>(), n_lines,
-                           c->g_atomline.as<const long long>(), n_atoms, at);
+    at.first_err = state;
+    const unsigned ablocks = (unsigned)((n_atoms + ING_THREADS - 1) / ING_THREADS);
+    if (n_atoms > 0) {
+        hipLaunchKernelGGL(jam::k_ing_parse, dim3(ablocks), dim3(ING_THREADS), 0, s, tx, c->g_starts.as<const long long>(),
+                           n_lines, c->g_atomline.as<const long long>(), n_atoms, at);
+        hipLaunchKernelGGL(jam::k_ing_descends, dim3(ablocks), dim3(ING_THREADS), 0, s, n_atoms, M->serial.as<const int>(),
+                           c->g_atomline.as<const long long>(), c->g_textof.as<const int>(), state + 1);
+    }
     HIP_TRY(hipGetLastError());
-    unsigned long long first_err = 0;
-    if ((rc = read_one(c->g_firsterr.as<unsigned long long>(), first_err, s)) != JAM_OK) return rc;
-    if ((long long)first_err < n_atoms) {
+    unsigned long long h_state[2] = {0, 0};
+    HIP_TRY(hipMemcpyAsync(h_state, state, sizeof(h_state), hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    if ((long long)h_state[0] < n_atoms) {
         long long li = 0;
         unsigned int kind = 0;
-        HIP_TRY(hipMemcpyAsync(&li, c->g_atomline.as<long long>() + first_err, sizeof(li), hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipMemcpyAsync(&kind, c->g_err.as<unsigned int>() + first_err, sizeof(kind), hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipMemcpyAsync(&li, c->g_atomline.as<long long>() + h_state[0], sizeof(li), hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipMemcpyAsync(&kind, c->g_err.as<unsigned int>() + h_state[0], sizeof(kind), hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
         int t = 0;
-        while (t + 1 < n && h_rng[t + 1] <= li) t++;
-        return fail(JAM_EINVAL, "text " + std::to_string(t) + ", line " + std::to_string(li - h_rng[t] + 1) +
+        while (t + 1 < n && h_line[t + 1] <= li) t++;
+        return fail(JAM_EINVAL, "text " + std::to_string(t) + ", line " + std::to_string(li - h_line[t] + 1) +
                                     ": failed to parse atom (" +
                                     ((kind & ING_ENONASCII) ? "a non-ASCII character in the first 80 columns"
                                                             : "a numeric field does not parse") +
                                     ")");
     }
     // ---- residue-name index
-    HIP_TRY(c->g_keys.reserve(sizeof(uint32_t) * ING_MAX_NAMES * (size_t)std::max(n, 1)));
-    HIP_TRY(c->g_nnames.reserve(sizeof(int) * (size_t)std::max(n, 1)));
-    if (n > 0)
-        hipLaunchKernelGGL(jam::k_ing_names, dim3((unsigned)n), dim3(1024), 0, s, M->atom_off.as<const int>(),
-                           M->resname.as<const uint32_t>(), c->g_keys.as<uint32_t>(), c->g_nnames.as<int>());
-    HIP_TRY(hipGetLastError());
-    std::vector<int> nnames(std::max(n, 1), 0);
-    HIP_TRY(hipMemcpyAsync(nnames.data(), c->g_nnames.ptr, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    std::vector<long long> resoff64(n + 1, 0);
-    std::vector<int> resoff(n + 1, 0);
-    for (int32_t k = 0; k < n; k++) {
-        if (nnames[k] < 0)
-            return fail(JAM_ETOOBIG, "text " + std::to_string(k) + " has more than " + std::to_string(ING_MAX_NAMES) +
-                                         " distinct residue names");
-        resoff64[k + 1] = resoff64[k] + nnames[k];
-        resoff[k + 1] = (int)resoff64[k + 1];
-    }
-    const long long nb = resoff64[n];
-    M->n_buckets = nb;
-    const size_t nbc = (size_t)std::max<long long>(nb, 1);
-    HIP_TRY(upload(M->res_off, resoff, s));
-    HIP_TRY(upload(c->g_resoff64, resoff64, s));
-    HIP_TRY(M->res_key.reserve(sizeof(uint32_t) * nbc));
-    HIP_TRY(M->res_begin.reserve(sizeof(int) * nbc));
-    HIP_TRY(M->res_end.reserve(sizeof(int) * nbc));
-    HIP_TRY(M->perm.reserve(sizeof(int) * na));
-    if (n > 0)
-        hipLaunchKernelGGL(jam::k_ing_keys, dim3((unsigned)n), dim3(256), 0, s, c->g_keys.as<const uint32_t>(),
-                           c->g_nnames.as<const int>(), c->g_resoff64.as<const long long>(), n, M->res_key.as<uint32_t>());
-    HIP_TRY(c->g_bucket.reserve(sizeof(int) * na));
-    HIP_TRY(c->g_bcount.reserve(sizeof(int) * nbc));
-    HIP_TRY(c->g_bstart.reserve(sizeof(long long) * (nbc + 1)));
-    hipLaunchKernelGGL(k_fill_i32, dim3(64), dim3(256), 0, s, c->g_bcount.as<int>(), (long long)nbc, 0);
-    if (n_atoms > 0) {
-        const unsigned ablocks = (unsigned)((n_atoms + ING_THREADS - 1) / ING_THREADS);
-        hipLaunchKernelGGL(jam::k_ing_bucket, dim3(ablocks), dim3(ING_THREADS), 0, s, M->atom_off.as<const int>(), n,
-                           n_atoms, M->resname.as<const uint32_t>(), M->res_key.as<const uint32_t>(),
-                           c->g_resoff64.as<const long long>(), c->g_bucket.as<int>(), c->g_bcount.as<int>());
-        if ((rc = device_scan<int>(c->g_bcount.as<int>(), nb, c->g_bstart.as<long long>(), tmp, 0, s)) != JAM_OK) return rc;
-        // atoms sorted by (bucket, serial), stable
+    guard.lock();
+    const int *order = nullptr;
+    if (h_state[1] != 0) {
+        // serial numbers that descend: the atoms of each text in their order
         HIP_TRY(c->g_skey.reserve(sizeof(unsigned long long) * 2 * na));
         HIP_TRY(c->g_sval.reserve(sizeof(int) * 2 * na));
         unsigned long long *k0 = c->g_skey.as<unsigned long long>(), *k1 = k0 + na;
         int *v0 = c->g_sval.as<int>(), *v1 = v0 + na;
         hipLaunchKernelGGL(jam::k_ing_sortkeys, dim3(ablocks), dim3(ING_THREADS), 0, s, n_atoms,
-                           c->g_bucket.as<const int>(), M->serial.as<const int>(), k0, v0);
-        int bucket_bits = 0;
-        while ((1ll << bucket_bits) < nb) bucket_bits++;
+                           c->g_atomline.as<const long long>(), c->g_textof.as<const int>(), M->serial.as<const int>(),
+                           k0, v0);
+        int text_bits = 0;
+        while ((1ll << text_bits) < n) text_bits++;
         int which = 0;
-        if ((rc = radix_sort<unsigned long long>(k0, v0, k1, v1, n_atoms, 32 + bucket_bits, c->rs_hist, c->rs_off, tmp,
+        if ((rc = radix_sort<unsigned long long>(k0, v0, k1, v1, n_atoms, 32 + text_bits, c->rs_hist, c->rs_off, tmp,
                                                  s, which)) != JAM_OK)
             return rc;
-        hipLaunchKernelGGL(jam::k_ing_perm, dim3(ablocks), dim3(ING_THREADS), 0, s, M->atom_off.as<const int>(), n,
-                           n_atoms, (const int *)(which ? v1 : v0), M->perm.as<int>());
-        hipLaunchKernelGGL(jam::k_ing_ranges, dim3((unsigned)((nb + ING_THREADS - 1) / ING_THREADS)), dim3(ING_THREADS),
-                           0, s, M->atom_off.as<const int>(), c->g_resoff64.as<const long long>(), n, nb,
-                           c->g_bstart.as<const long long>(), M->res_begin.as<int>(), M->res_end.as<int>());
+        int *out_order = which ? v0 : v1;
+        hipLaunchKernelGGL(jam::k_ing_order, dim3(ablocks), dim3(ING_THREADS), 0, s, n_atoms,
+                           (const int *)(which ? v1 : v0), M->atom_off.as<const int>(),
+                           c->g_atomline.as<const long long>(), c->g_textof.as<const int>(), out_order);
+        HIP_TRY(hipGetLastError());
+        order = out_order;
     }
-    HIP_TRY(hipGetLastError());
+    if (n > 0) {
+        int refused = -1;
+        if ((rc = residue_index(c, M.get(), order, blk + o_perm, blk + o_resoff, s, refused)) != JAM_OK) return rc;
+        if (refused >= 0)
+            return fail(JAM_ETOOBIG, "text " + std::to_string(refused) + " has more than " +
+                                         std::to_string(ING_MAX_NAMES) + " distinct residue names");
+    } else {
+        M->perm.view(blk + o_perm, 4);
+        M->res_off.view(blk + o_resoff, sizeof(int));
+        HIP_TRY(M->res_key.reserve(4));
+        HIP_TRY(M->res_begin.reserve(4));
+        HIP_TRY(M->res_end.reserve(4));
+        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, M->res_off.as<int>(), 1ll, 0);
+    }
     HIP_TRY(hipStreamSynchronize(s));
     *out = M.release();
+    return JAM_OK;
+}
+
+extern "C" int32_t jam_molecules_pdb_headers(const jam_molecules *m, int32_t *ascii, int32_t *known, int32_t *text,
+                                             int64_t *offset, int32_t cap, int32_t *n)
+{
+    if (!m || !m->parsed || cap < 0 || (cap > 0 && (!text || !offset)))
+        return fail(JAM_EINVAL, "not a batch of parsed molecules, or NULL argument");
+    if (ascii) *ascii = m->ascii ? 1 : 0;
+    if (known) *known = m->headers_known ? 1 : 0;
+    if (n) *n = (int32_t)m->headers.size();
+    for (size_t k = 0; k < m->headers.size() && k < (size_t)cap; k++) {
+        text[k] = m->headers[k].first;
+        offset[k] = m->headers[k].second;
+    }
     return JAM_OK;
 }
 
@@ -1356,19 +1392,20 @@ extern "C" int32_t jam_molecules_copy_atoms(const jam_molecules *m, const jam_at
     HIP_TRY(hipSetDevice(m->ctx->device));
     std::vector<CopyPiece> pieces;
     auto get = [&](void *dst, const DBuf &src, size_t bytes) { add_pieces(pieces, dst, src.as<const char>(), bytes); };
+    // in the order in which a parsed batch holds them
     get(f->xyz, m->xyz, sizeof(double) * 3 * na);
     get(f->names, m->name, 4 * na);
     get(f->resnames, m->resname, 4 * na);
     get(f->resseq, m->resseq, sizeof(int) * na);
-    get(f->chains, m->chains, 2 * na);
     get(f->serial, m->serial, sizeof(int) * na);
-    get(f->altloc, m->altloc, na);
-    get(f->icode, m->icode, na);
     get(f->occupancy, m->occupancy, sizeof(float) * na);
     get(f->tempfactor, m->tempfactor, sizeof(float) * na);
     get(f->segid, m->segid, 4 * na);
-    get(f->element, m->element, 2 * na);
     get(f->charge, m->charge, sizeof(int) * na);
+    get(f->chains, m->chains, 2 * na);
+    get(f->element, m->element, 2 * na);
+    get(f->altloc, m->altloc, na);
+    get(f->icode, m->icode, na);
     return copy_out(m->ctx, pieces);
 }
 

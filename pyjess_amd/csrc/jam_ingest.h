@@ -17,11 +17,10 @@
 //                               first ENDMDL and first mmCIF tag of every text
 //   k_ing_select                atom records in order (a scan of 0/1 flags)
 //   k_ing_parse                 thread per atom record: the fixed columns
-//   k_ing_names ... k_ing_ranges the residue-name index: distinct names per
-//                               molecule (LDS hash set, sorted), per-atom
-//                               bucket, then one stable radix sort of the
-//                               atoms by (bucket, serial) and the buckets'
-//                               ranges
+//   k_residue_index             the residue-name index: workgroup per molecule,
+//                               a stable counting sort by name (of atoms
+//                               sorted by serial number before, where those
+//                               descend)
 // Numbers are parsed exactly: a decimal field of at most 19 significant
 // digits and a power of ten up to 22 is one correctly rounded division or
 // multiplication of two exact doubles (Clinger's fast path), which is what
@@ -46,6 +45,13 @@ namespace jam {
 #define ING_HETATM 2
 #define ING_ENDMDL 3
 #define ING_MMCIF 4
+#define ING_HEADER 5
+
+// what the line split and the record kinds report beside them: whether any
+// byte is above 0x7F, how many HEADER records there are, and of the first
+// ING_HEADERS of them (in any order) line and offset
+#define ING_HEADERS 256
+#define ING_INFO_WORDS (2 + 2 * ING_HEADERS)
 
 // parse errors (bit flags of the per-atom error word)
 #define ING_EBADFIELD 1     // a numeric field does not parse
@@ -88,15 +94,20 @@ __device__ static inline long long ing_block_scan(long long v, long long *lds, l
 }
 
 // Line starts of each block's ING_THREADS * ING_BPT bytes.
-__global__ void __launch_bounds__(ING_THREADS) k_ing_count(IngText tx, long long *block_lines)
+__global__ void __launch_bounds__(ING_THREADS) k_ing_count(IngText tx, long long *block_lines,
+                                                          unsigned long long *info)
 {
     __shared__ long long lds[ING_THREADS / JAM_WAVE];
     const long long b0 = ((long long)blockIdx.x * ING_THREADS + threadIdx.x) * ING_BPT;
     long long c = 0;
+    bool high = false;
     for (int k = 0; k < ING_BPT; k++) {
         const long long i = b0 + k;
-        if (i < tx.n_bytes && ing_line_start(tx.buf, i)) c++;
+        if (i >= tx.n_bytes) break;
+        if (ing_line_start(tx.buf, i)) c++;
+        high |= tx.buf[i] > 0x7F;
     }
+    if (ballot(high) != 0ull && lane_id() == 0) atomicOr(&info[0], 1ull);
     long long total;
     ing_block_scan(c, lds, total);
     if (threadIdx.x == 0) block_lines[blockIdx.x] = total;
@@ -148,7 +159,8 @@ __device__ static inline unsigned char ing_lower(unsigned char c) { return (c >=
 __global__ void __launch_bounds__(ING_THREADS) k_ing_classify(IngText tx, const long long *starts, long long n_lines,
                                                              unsigned char *kind, int *text_of,
                                                              unsigned long long *first_endmdl,
-                                                             unsigned long long *first_mmcif)
+                                                             unsigned long long *first_mmcif,
+                                                             unsigned long long *info)
 {
     const long long li = (long long)blockIdx.x * ING_THREADS + threadIdx.x;
     if (li >= n_lines) return;
@@ -160,6 +172,7 @@ __global__ void __launch_bounds__(ING_THREADS) k_ing_classify(IngText tx, const 
     if (at(0) == 'A' && at(1) == 'T' && at(2) == 'O' && at(3) == 'M') k = ING_ATOM;
     else if (at(0) == 'H' && at(1) == 'E' && at(2) == 'T' && at(3) == 'A' && at(4) == 'T' && at(5) == 'M') k = ING_HETATM;
     else if (at(0) == 'E' && at(1) == 'N' && at(2) == 'D' && at(3) == 'M' && at(4) == 'D' && at(5) == 'L') k = ING_ENDMDL;
+    else if (at(0) == 'H' && at(1) == 'E' && at(2) == 'A' && at(3) == 'D' && at(4) == 'E' && at(5) == 'R') k = ING_HEADER;
     else if (len >= 5) {
         const unsigned char a = ing_lower(p[0]), b = ing_lower(p[1]), c = ing_lower(p[2]), d = ing_lower(p[3]);
         if (p[4] == '_' && ((a == 'd' && b == 'a' && c == 't' && d == 'a') || (a == 'l' && b == 'o' && c == 'o' && d == 'p')))
@@ -170,6 +183,13 @@ __global__ void __launch_bounds__(ING_THREADS) k_ing_classify(IngText tx, const 
     text_of[li] = t;
     if (k == ING_ENDMDL) atomicMin(&first_endmdl[t], (unsigned long long)li);
     if (k == ING_MMCIF) atomicMin(&first_mmcif[t], (unsigned long long)li);
+    if (k == ING_HEADER) {
+        const unsigned long long h = atomicAdd(&info[1], 1ull);
+        if (h < ING_HEADERS) {
+            info[2 + 2 * h] = (unsigned long long)li;
+            info[3 + 2 * h] = (unsigned long long)s;
+        }
+    }
 }
 
 // whether line li is an atom record the reference would read
@@ -215,7 +235,7 @@ __global__ void __launch_bounds__(ING_THREADS) k_ing_select(IngText tx, const un
 
 // per text: its first line and its first atom (n_texts + 1 entries each)
 __global__ void k_ing_text_ranges(IngText tx, const long long *starts, long long n_lines, const long long *line_atom,
-                                  long long n_atoms, long long *text_line, long long *text_atom)
+                                  const long long *n_atoms, long long *text_line, long long *text_atom)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t > tx.n_texts) return;
@@ -227,7 +247,7 @@ __global__ void k_ing_text_ranges(IngText tx, const long long *starts, long long
         else hi = mid;
     }
     text_line[t] = lo;
-    text_atom[t] = lo < n_lines ? line_atom[lo] : n_atoms;
+    text_atom[t] = lo < n_lines ? line_atom[lo] : (n_lines > 0 ? *n_atoms : 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -406,167 +426,46 @@ __global__ void __launch_bounds__(ING_THREADS) k_ing_parse(IngText tx, const lon
 // residue-name index
 // ---------------------------------------------------------------------------
 
-// Block per molecule: its distinct upper-cased residue names, sorted, into
-// keys[m * ING_MAX_NAMES ...] and their number into n_names[m] (more than
-// ING_MAX_NAMES: n_names[m] = -1).
-__global__ void __launch_bounds__(1024) k_ing_names(const int *atom_off, const uint32_t *resname, uint32_t *keys,
-                                                    int *n_names)
-{
-    constexpr int SLOTS = 2 * ING_MAX_NAMES;   // open addressing at half load at most
-    __shared__ uint32_t slot[SLOTS];
-    __shared__ uint32_t list[ING_MAX_NAMES];
-    __shared__ int count, overflow;
-    const int m = blockIdx.x, t = threadIdx.x;
-    for (int k = t; k < SLOTS; k += blockDim.x) slot[k] = 0xFFFFFFFFu;   // never an upper-cased name
-    if (t == 0) {
-        count = 0;
-        overflow = 0;
-    }
-    __syncthreads();
-    const int a0 = atom_off[m], a1 = atom_off[m + 1];
-    for (int a = a0 + t; a < a1; a += blockDim.x) {
-        const uint32_t key = jam_upper4(resname[a]);
-        uint32_t h = (key * 2654435761u) & (SLOTS - 1);
-        for (int probe = 0; probe < SLOTS; probe++) {
-            const uint32_t old = atomicCAS(&slot[h], 0xFFFFFFFFu, key);
-            if (old == 0xFFFFFFFFu) {
-                const int c = atomicAdd(&count, 1);
-                if (c < ING_MAX_NAMES) list[c] = key;
-                else overflow = 1;
-                break;
-            }
-            if (old == key) break;
-            h = (h + 1) & (SLOTS - 1);
-        }
-    }
-    __syncthreads();
-    const int n = count;
-    if (overflow || n > ING_MAX_NAMES) {
-        if (t == 0) n_names[m] = -1;
-        return;
-    }
-    // bitonic sort of the n names (padded to a power of two with all-ones)
-    int n2 = 1;
-    while (n2 < n) n2 <<= 1;
-    for (int k = n + t; k < n2; k += blockDim.x) list[k] = 0xFFFFFFFFu;
-    __syncthreads();
-    for (int k = 2; k <= n2; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = t; i < n2; i += blockDim.x) {
-                const int ixj = i ^ j;
-                if (ixj > i) {
-                    const uint32_t u = list[i], v = list[ixj];
-                    const bool up = (i & k) == 0;
-                    if ((u > v) == up) {
-                        list[i] = v;
-                        list[ixj] = u;
-                    }
-                }
-            }
-            __syncthreads();
-        }
-    }
-    for (int k = t; k < n; k += blockDim.x) keys[(size_t)m * ING_MAX_NAMES + k] = list[k];
-    if (t == 0) n_names[m] = n;
-}
-
-// res_key[res_off[m] + k] = the k-th name of molecule m (res_off: scan of n_names)
-__global__ void k_ing_keys(const uint32_t *keys, const int *n_names, const long long *res_off, int n_mols,
-                           uint32_t *res_key)
-{
-    const int m = blockIdx.x;
-    if (m >= n_mols) return;
-    for (int k = threadIdx.x; k < n_names[m]; k += blockDim.x)
-        res_key[res_off[m] + k] = keys[(size_t)m * ING_MAX_NAMES + k];
-}
-
-// bucket (global index) of every atom, and the bucket sizes: one atomic add
-// per distinct bucket of a wave (atoms of a residue are adjacent, so a wave
-// holds few distinct names) instead of one per atom on a few hot words
-__global__ void __launch_bounds__(ING_THREADS) k_ing_bucket(const int *atom_off, int n_mols, long long n_atoms,
-                                                           const uint32_t *resname, const uint32_t *res_key,
-                                                           const long long *res_off, int *bucket, int *bucket_count)
+// *down != 0 where an atom's serial number is below that of the atom before it
+// in its text.
+__global__ void __launch_bounds__(ING_THREADS) k_ing_descends(long long n_atoms, const int *serial,
+                                                             const long long *atom_line, const int *text_of,
+                                                             unsigned long long *down)
 {
     const long long a = (long long)blockIdx.x * ING_THREADS + threadIdx.x;
-    const int lane = lane_id();
-    long long b0 = 0;
-    bool pending = a < n_atoms;
-    if (pending) {
-        int lo = 0, hi = n_mols;   // molecule of atom a: the last m with atom_off[m] <= a
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (atom_off[mid] <= a) lo = mid;
-            else hi = mid;
-        }
-        const uint32_t key = jam_upper4(resname[a]);
-        long long b1 = res_off[lo + 1];
-        b0 = res_off[lo];
-        while (b0 < b1) {
-            const long long mid = (b0 + b1) >> 1;
-            if (res_key[mid] < key) b0 = mid + 1;
-            else b1 = mid;
-        }
-        bucket[a] = (int)b0;
-    }
-    // every lane takes part in the ballots and shuffles; each round retires
-    // the lanes of the lowest pending lane's bucket (at most 64 rounds)
-    for (int round = 0; round < JAM_WAVE; round++) {
-        const unsigned long long m = ballot(pending);
-        if (m == 0ull) break;
-        const int leader = __ffsll((long long)m) - 1;
-        const long long lb = __shfl(b0, leader, JAM_WAVE);
-        const bool same = pending && b0 == lb;
-        const unsigned long long peers = ballot(same);
-        if (lane == leader) atomicAdd(&bucket_count[lb], __popcll(peers));
-        if (same) pending = false;
-    }
+    const bool d = a > 0 && a < n_atoms && serial[a] < serial[a - 1] && text_of[atom_line[a]] == text_of[atom_line[a - 1]];
+    if (ballot(d) != 0ull && lane_id() == 0) atomicOr(down, 1ull);
 }
 
-// Sort key of every atom: its bucket, then its serial number, which the
-// stable radix sort orders as ResIndex does (upper-cased residue name, then
-// serial, input order among equals); the value is the atom's index.
-__global__ void __launch_bounds__(ING_THREADS) k_ing_sortkeys(long long n_atoms, const int *bucket, const int *serial,
+// Sort key of every atom: its text, then its serial number, which a stable
+// sort orders as k_residue_index visits atoms whose serial numbers descend
+// somewhere; the value is the atom's index.
+__global__ void __launch_bounds__(ING_THREADS) k_ing_sortkeys(long long n_atoms, const long long *atom_line,
+                                                             const int *text_of, const int *serial,
                                                              unsigned long long *key, int *val)
 {
     const long long a = (long long)blockIdx.x * ING_THREADS + threadIdx.x;
     if (a >= n_atoms) return;
-    key[a] = ((unsigned long long)(unsigned int)bucket[a] << 32) | ((unsigned int)serial[a] ^ 0x80000000u);
+    key[a] = ((unsigned long long)(unsigned int)text_of[atom_line[a]] << 32) | ((unsigned int)serial[a] ^ 0x80000000u);
     val[a] = (int)a;
 }
 
-// perm[i]: the molecule-local index of the i-th atom in sorted order (the
-// buckets are molecule-major, so position i lies in its atom's molecule)
-__global__ void __launch_bounds__(ING_THREADS) k_ing_perm(const int *atom_off, int n_mols, long long n_atoms,
-                                                         const int *sorted, int *perm)
+// order[i]: the molecule-local index of the i-th sorted atom (a text's atoms
+// keep its positions)
+__global__ void __launch_bounds__(ING_THREADS) k_ing_order(long long n_atoms, const int *sorted, const int *atom_off,
+                                                          const long long *atom_line, const int *text_of, int *order)
 {
     const long long i = (long long)blockIdx.x * ING_THREADS + threadIdx.x;
     if (i >= n_atoms) return;
     const int a = sorted[i];
-    int lo = 0, hi = n_mols;   // the last m with atom_off[m] <= a
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (atom_off[mid] <= a) lo = mid;
-        else hi = mid;
-    }
-    perm[i] = a - atom_off[lo];
+    order[i] = a - atom_off[text_of[atom_line[a]]];
 }
 
-// res_begin / res_end of every bucket: its range in its molecule's part of
-// perm (bucket_start: the exclusive scan of the bucket sizes, nb + 1 values)
-__global__ void __launch_bounds__(ING_THREADS) k_ing_ranges(const int *atom_off, const long long *res_off, int n_mols,
-                                                           long long n_buckets, const long long *bucket_start,
-                                                           int *res_begin, int *res_end)
+// out[k] = (int)in[k]
+__global__ void k_ing_narrow(const long long *in, int n, int *out)
 {
-    const long long b = (long long)blockIdx.x * ING_THREADS + threadIdx.x;
-    if (b >= n_buckets) return;
-    int lo = 0, hi = n_mols;   // the last m with res_off[m] <= b: bucket b's molecule
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (res_off[mid] <= b) lo = mid;
-        else hi = mid;
-    }
-    res_begin[b] = (int)(bucket_start[b] - atom_off[lo]);
-    res_end[b] = (int)(bucket_start[b + 1] - atom_off[lo]);
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) out[k] = (int)in[k];
 }
 
 // The residue-name index of a batch in one launch (ResIndex_create,
@@ -590,7 +489,8 @@ __global__ void __launch_bounds__(ING_THREADS) k_ing_ranges(const int *atom_off,
 //
 // Bound by latency (two walks with one dependent load each and ~10 LDS steps
 // per 64 atoms of a wave) and by the waves in flight: 2 workgroups of 16 waves
-// per CU at MAXN = 256 (19 KB of LDS). One launch for all molecules instead of
+// per CU at MAXN = 256 (19 KB of LDS; 152 KB at ING_MAX_NAMES, for molecules
+// of more names). One launch for all molecules instead of
 // a host sort: jam_molecules_create of 256 molecules (1.2 M atoms) 39.6 -> 3.2
 // ms, of 100,000 atoms 2.2 -> 0.57 ms, of 2,000 atoms 0.22 -> 0.07 ms, with
 // the upload through pinned memory that came with it.
