@@ -29,7 +29,7 @@ def _ptr(t: Optional[torch.Tensor]):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
-def _check_inputs(a: torch.Tensor, b: torch.Tensor, offsets: torch.Tensor) -> None:
+def _check_inputs(a: torch.Tensor, b: torch.Tensor, offsets: torch.Tensor, even: bool) -> None:
     for name, t in (("a", a), ("b", b)):
         if not isinstance(t, torch.Tensor) or not t.is_cuda:
             raise TypeError(f"`{name}` must be a tensor on a GPU (the computation runs on the device only)")
@@ -41,7 +41,8 @@ def _check_inputs(a: torch.Tensor, b: torch.Tensor, offsets: torch.Tensor) -> No
         raise ValueError(f"`a` and `b` differ in shape: {tuple(a.shape)} and {tuple(b.shape)}")
     if a.device != b.device or offsets.device != a.device:
         raise ValueError("`a`, `b` and `offsets` must be on the same device")
-    _check_offsets(offsets, a.shape[0])
+    if not even:
+        _check_offsets(offsets, a.shape[0])
 
 
 # the offsets tensor last found valid: (weak reference, its version counter,
@@ -72,14 +73,18 @@ def _check_offsets(offsets: torch.Tensor, n_points: int) -> None:
 
 
 class SuperpositionRMSD(torch.autograd.Function):
-    """RMSD per point set; set s owns rows ``offsets[s]:offsets[s+1]`` of ``a`` and ``b``."""
+    """RMSD per point set; set s owns rows ``offsets[s]:offsets[s+1]`` of ``a`` and ``b``.
+
+    ``even``: the offsets were made for sets of equal size by
+    `superposition_rmsd`, so that nothing about them has to be read back from
+    the device."""
 
     @staticmethod
-    def forward(ctx, a: torch.Tensor, b: torch.Tensor, offsets: torch.Tensor) -> torch.Tensor:
+    def forward(ctx, a: torch.Tensor, b: torch.Tensor, offsets: torch.Tensor, even: bool = False) -> torch.Tensor:
         a = a.contiguous()
         b = b.contiguous()
         offsets = offsets.contiguous()
-        _check_inputs(a, b, offsets)
+        _check_inputs(a, b, offsets, even)
         n_sets = offsets.numel() - 1
         rmsd = torch.empty(n_sets, dtype=torch.float64, device=a.device)
         # the optimal rotations are kept for the backward pass when it will run
@@ -98,7 +103,7 @@ class SuperpositionRMSD(torch.autograd.Function):
         a, b, offsets, rmsd, rot = ctx.saved_tensors
         need_a, need_b = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         if not (need_a or need_b):
-            return None, None, None
+            return None, None, None, None
         g = grad_rmsd.to(torch.float64).contiguous()
         # the offsets were checked in forward: every row belongs to a set of at
         # least one point, and the kernel writes every such row
@@ -109,7 +114,7 @@ class SuperpositionRMSD(torch.autograd.Function):
             stream = ctypes.c_void_p(torch.cuda.current_stream(a.device).cuda_stream)
             _native._check(L.jam_rmsd_backward(_ptr(a), _ptr(b), _ptr(offsets), offsets.numel() - 1, a.shape[0],
                                                _ptr(rmsd), _ptr(rot), _ptr(g), _ptr(ga), _ptr(gb), stream))
-        return ga, gb, None
+        return ga, gb, None, None
 
 
 def superposition_rmsd(a: torch.Tensor, b: torch.Tensor, offsets: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -123,7 +128,10 @@ def superposition_rmsd(a: torch.Tensor, b: torch.Tensor, offsets: Optional[torch
         if a.dim() != 3:
             raise ValueError("without `offsets`, `a` and `b` must have shape (n_sets, k, 3)")
         n_sets, k = a.shape[0], a.shape[1]
-        offsets = torch.arange(0, n_sets + 1, dtype=torch.int64, device=a.device) * k
+        i64 = dict(dtype=torch.int64, device=a.device)
+        offsets = torch.arange(0, n_sets * k + 1, k, **i64) if k > 0 else torch.zeros(n_sets + 1, **i64)
+        even = a.shape[2] == 3   # else the rows below are not the sets'
         a = a.reshape(-1, 3)
         b = b.reshape(-1, 3)
+        return SuperpositionRMSD.apply(a, b, offsets, even)
     return SuperpositionRMSD.apply(a, b, offsets)
