@@ -353,7 +353,7 @@ __device__ static inline long long row_of(long long it, int parts)
 #ifndef JOIN_BOX_DIRECT
 #define JOIN_BOX_DIRECT 12
 #endif
-template <int MAXN, int TW>
+template <int MAXN, int TW, int LC>
 __device__ static void join_team(const DevMols &ms, const DevTpls &tp, const DevSets &st, const DevPairs &pr,
                                  const DevJoin &jn, const QueryParams &qp, JoinWaveLds<MAXN, TW> &S,
                                  bool active, long long it, int parts, int p, const int (&ent)[(MAXN + TW - 1) / TW],
@@ -363,7 +363,7 @@ __device__ static void join_team(const DevMols &ms, const DevTpls &tp, const Dev
     const int lane = lane_id();
     const int team = lane / TW, tl = lane % TW;
     JoinTeamLds<MAXN> &M = S.tm[team];
-    const int L = jn.level;
+    const int L = LC ? LC : jn.level;
     const long long i = active ? row_of(it, parts) : 0;
     const int part = active ? (int)(it - i * parts) : 0;
     constexpr int NE = (MAXN + TW - 1) / TW;
@@ -496,7 +496,7 @@ __device__ static void join_team(const DevMols &ms, const DevTpls &tp, const Dev
         for (int j = 0; j < L; j++) {
             // most candidates fail an early annulus: stop as soon as no lane
             // of the wave is still in
-            if (ballot(ok) == 0ull) break;
+            if (j > 0 && ballot(ok) == 0ull) break;
             // _Annulus_po: squared distance summed x, y, z from 0.0; inside
             // unless below the inner or above the outer squared radius
             const double tx = M.px[j] - c.x, ty = M.py[j] - c.y, tz = M.pz[j] - c.z;
@@ -606,7 +606,7 @@ __device__ static void join_team(const DevMols &ms, const DevTpls &tp, const Dev
 #ifndef JOIN_RUN
 #define JOIN_RUN 32
 #endif
-template <int MAXN, int TW>
+template <int MAXN, int TW, int LC>
 __global__ void __launch_bounds__(JOIN_WAVES * JAM_WAVE, JOIN_MIN_WAVES) k_join(DevMols ms, DevTpls tp, DevSets st,
                                                                               DevPairs pr, DevJoin jn,
                                                                               QueryParams qp)
@@ -641,7 +641,7 @@ __global__ void __launch_bounds__(JOIN_WAVES * JAM_WAVE, JOIN_MIN_WAVES) k_join(
     // while the current one is processed
     constexpr int NE = (MAXN + TW - 1) / TW;
     const int tl = lane_id() % TW;
-    const int L = jn.level;
+    const int L = LC ? LC : jn.level;
     int p_next = 0, e_next[NE];
     auto fetch = [&](long long it) {
 #pragma unroll
@@ -666,7 +666,7 @@ __global__ void __launch_bounds__(JOIN_WAVES * JAM_WAVE, JOIN_MIN_WAVES) k_join(
         for (int jj = 0; jj < NE; jj++) e[jj] = e_next[jj];
         const long long next = round_base(i + 1);
         if (next < items) fetch(next + team);
-        join_team<MAXN, TW>(ms, tp, st, pr, jn, qp, SW[w], it < items, it, parts, p, e, pc, staged, dstaged);
+        join_team<MAXN, TW, LC>(ms, tp, st, pr, jn, qp, SW[w], it < items, it, parts, p, e, pc, staged, dstaged);
         base = next;
     }
     join_write(jn, SW[w].sp, SW[w].se, staged, jn.n_out, jn.out_cap, jn.out_pair, jn.out_ent, jn.out_stride);
