@@ -135,7 +135,7 @@ struct jam_context {
     bool profile = false;       // join launches carry start/stop events (xev)
     // per-query workspace
     DBuf cnt, off, list, kidx, l2k, kent, katom, bbox, sbox, kscr, kd_bucket, kd_tied, kd_count;
-    DBuf p_ord, p_lvl, p_nchunk, p_n1, p_base, p_cm, p_first, i_pair;
+    DBuf p_ord, p_lvl, p_nchunk, p_n1, p_base, p_cm, p_first;
     // join: two frontiers (pair + stride entries per row), complete matches,
     // counters (rows per level, complete matches, overflow flag)
     DBuf j_pair[2], j_ent[2], d_pair, d_ent, j_count;
@@ -168,7 +168,6 @@ struct jam_context {
     DBuf keep_d, keep_i;  // superpositions kept between the two k_super passes (few matches)
     int64_t set_cap = 0, blk_cap = 0, sblk_cap = 0, event_cap = 0;
     int nsets_cap = 0, npairs_cap = 0;
-    int64_t items_cap = 0;
     int event_stride = 0;
     // incremented by every query: a result's events live in e_* until the
     // next query on the context
@@ -906,11 +905,16 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_scan_blocks(const T *in, long lo
 
 // The whole exclusive scan in one workgroup, SCAN_BLOCK elements at a time
 // with a running carry, the total into out[n]: for small arrays, where the
-// launches of the multi-block scan would dominate.
+// launches of the multi-block scan would dominate. The largest element (at
+// least 0, of 32 bits) and the total in 64 bits too, where they are asked for.
 template <class T, class O>
-__global__ void __launch_bounds__(SCAN_BLOCK) k_scan_one(const T *in, long long n, O *out)
+__global__ void __launch_bounds__(SCAN_BLOCK) k_scan_one(const T *in, long long n, O *out, int *largest,
+                                                        unsigned long long *total64)
 {
     __shared__ long long w[SCAN_BLOCK / JAM_WAVE];
+    __shared__ int top;
+    int most = 0;
+    if (threadIdx.x == 0) top = 0;
     const int lane = jam::lane_id(), wv = threadIdx.x / JAM_WAVE;
     long long carry = 0;
     for (long long b0 = 0; b0 < n; b0 += SCAN_BLOCK) {
@@ -930,22 +934,32 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_scan_one(const T *in, long long 
         }
         if (i < n) out[i] = (O)(carry + base + x - v);
         carry += total;
+        most = max(most, (int)v);
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[n] = (O)carry;
+    if (threadIdx.x == 0) {
+        out[n] = (O)carry;
+        if (total64) *total64 = (unsigned long long)carry;
+    }
+    if (largest) {
+        __syncthreads();
+        atomicMax(&top, most);
+        __syncthreads();
+        if (threadIdx.x == 0) *largest = top;
+    }
 }
 
+// Adds the blocks' offsets; the total (offs[blocks]) goes after the scan.
 template <class O>
-__global__ void __launch_bounds__(SCAN_BLOCK) k_scan_add(O *out, long long n, const long long *offs)
+__global__ void __launch_bounds__(SCAN_BLOCK) k_scan_add(O *out, long long n, const long long *offs,
+                                                        unsigned long long *total64)
 {
     const long long i = (long long)blockIdx.x * SCAN_BLOCK + threadIdx.x;
     if (i < n) out[i] += (O)offs[blockIdx.x];
-}
-
-template <class O>
-__global__ void k_scan_total(O *dst, const long long *src)
-{
-    if (threadIdx.x == 0) *dst = (O)*src;
+    if (i == 0) {
+        out[n] = (O)offs[gridDim.x];
+        if (total64) *total64 = (unsigned long long)offs[gridDim.x];
+    }
 }
 
 __global__ void k_fill_u64(unsigned long long *v, long long n, unsigned long long x)
@@ -976,14 +990,15 @@ __global__ void __launch_bounds__(1024) k_max_i32(const int *in, long long n, in
 }
 
 // out[0, n] = exclusive scan of in[0, n) followed by the total (n + 1
-// values), on stream s; temporary space from `tmp`, grown as needed
+// values), on stream s; temporary space from `tmp`, grown as needed. `largest`,
+// `total64`: the largest element (of int arrays) and the total in 64 bits
 template <class T, class O>
 int32_t device_scan(const T *in, long long n, O *out, std::vector<std::unique_ptr<DBuf>> &tmp, size_t level,
-                    hipStream_t s)
+                    hipStream_t s, int *largest = nullptr, unsigned long long *total64 = nullptr)
 {
     const long long blocks = std::max<long long>(1, (n + SCAN_BLOCK - 1) / SCAN_BLOCK);
     if (blocks <= SCAN_ONE_BLOCKS) {
-        hipLaunchKernelGGL((k_scan_one<T, O>), dim3(1), dim3(SCAN_BLOCK), 0, s, in, n, out);
+        hipLaunchKernelGGL((k_scan_one<T, O>), dim3(1), dim3(SCAN_BLOCK), 0, s, in, n, out, largest, total64);
         HIP_TRY(hipGetLastError());
         return JAM_OK;
     }
@@ -992,20 +1007,14 @@ int32_t device_scan(const T *in, long long n, O *out, std::vector<std::unique_pt
     long long *sums = tmp[level]->as<long long>();
     hipLaunchKernelGGL((k_scan_blocks<T, O>), dim3((unsigned)blocks), dim3(SCAN_BLOCK), 0, s, in, n, out, sums);
     HIP_TRY(hipGetLastError());
-    if (blocks == 1) {
-        // the total goes after the scan
-        hipLaunchKernelGGL(k_scan_total<O>, dim3(1), dim3(64), 0, s, out + n, (const long long *)sums);
-        HIP_TRY(hipGetLastError());
-        return JAM_OK;
-    }
     // scan of the block totals (with their total at [blocks]), added back
     HIP_TRY(tmp[level + 1]->reserve(sizeof(long long) * (size_t)(blocks + 1)));
     long long *offs = tmp[level + 1]->as<long long>();
     int32_t rc = device_scan<long long, long long>(sums, blocks, offs, tmp, level + 2, s);
     if (rc != JAM_OK) return rc;
     hipLaunchKernelGGL(k_scan_add<O>, dim3((unsigned)blocks), dim3(SCAN_BLOCK), 0, s, out, n,
-                       (const long long *)offs);
-    hipLaunchKernelGGL(k_scan_total<O>, dim3(1), dim3(64), 0, s, out + n, (const long long *)(offs + blocks));
+                       (const long long *)offs, total64);
+    if (largest) hipLaunchKernelGGL(k_max_i32, dim3(1), dim3(1024), 0, s, (const int *)in, n, largest);
     HIP_TRY(hipGetLastError());
     return JAM_OK;
 }
@@ -1506,15 +1515,6 @@ int32_t grow_hsmall(jam_context *c, int64_t words)
     return JAM_OK;
 }
 
-int32_t grow_items(jam_context *c, int64_t n_items)
-{
-    if (n_items <= c->items_cap) return JAM_OK;
-    n_items = std::max<int64_t>(n_items, 4096);
-    HIP_TRY(c->i_pair.reserve(sizeof(int) * (size_t)n_items));
-    c->items_cap = n_items;
-    return JAM_OK;
-}
-
 // join frontiers (both buffers), rows of `stride` entries
 int32_t grow_front(jam_context *c, int64_t rows, int stride)
 {
@@ -1572,15 +1572,6 @@ int32_t grow_events(jam_context *c, int64_t cap, int stride)
 __global__ void k_kd_setup(unsigned int *counts, int n)
 {
     if ((int)threadIdx.x < n) counts[threadIdx.x] = 0u;
-}
-
-__global__ void k_items_any(DevPairs pr)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= pr.n_pairs || *pr.n_items > pr.items_cap) return;   // does not fit: grown and run again
-    const int c = pr.nchunk[p];
-    const long long b = pr.item_base[p];
-    for (int i = 0; i < c; i++) pr.item_pair[b + i] = p;
 }
 
 __global__ void k_zero_u64(unsigned long long *v, long long n)
@@ -1998,12 +1989,10 @@ extern "C" int32_t jam_query(jam_context *c, const jam_templates *tp, const jam_
     if ((rc = grow_sets(c, std::max<int64_t>(c->set_cap, 1 << 16), n_sets)) != JAM_OK) return rc;
     if ((rc = grow_events(c, std::max<int64_t>(c->event_cap, 1 << 12), stride)) != JAM_OK) return rc;
     if ((rc = grow_pairs(c, n_pairs)) != JAM_OK) return rc;
-    if ((rc = grow_items(c, std::max<int64_t>(c->items_cap, 4096))) != JAM_OK) return rc;
     if ((rc = grow_hsmall(c, std::max<int64_t>(CNT_WORDS, (int64_t)n_pairs + 2))) != JAM_OK) return rc;
     HIP_TRY(c->j_count.reserve(sizeof(unsigned long long) * CNT_WORDS));
     DevMols dm = ms->dev();
     DevTpls dt = tp->dev();
-    const int pair_blocks = (n_pairs + 255) / 256;
 
     for (int attempt = 0; attempt < 8; attempt++) {
         DevSets st;
@@ -2029,23 +2018,20 @@ extern "C" int32_t jam_query(jam_context *c, const jam_templates *tp, const jam_
         DevPairs pr;
         pr.n_pairs = n_pairs;
         pr.n_items = (const long long *)(cnts + CNT_ITEMS);
-        pr.items_cap = c->items_cap;
         pr.ord = c->p_ord.as<unsigned char>();
         pr.lvl = c->p_lvl.as<PairLevel>();
         pr.nchunk = c->p_nchunk.as<int>();
         pr.n1 = c->p_n1.as<int>();
         pr.item_base = c->p_base.as<long long>();
-        pr.item_pair = c->i_pair.as<int>();
 
         const int wpb = 4;  // waves per block of the per-set candidate kernels
         const int set_blocks = (n_sets + wpb - 1) / wpb;
         HIP_TRY(hipEventRecord(c->ev[0], s));
         hipLaunchKernelGGL(jam::k_candidates<false>, dim3(set_blocks), dim3(64 * wpb), 0, s, dm, dt, st, pr,
-                           (long long *)nullptr);
+                           (long long *)nullptr, (unsigned long long *)nullptr, 0);
         HIP_TRY(hipGetLastError());
-        if ((rc = device_scan<int, int64_t>(st.cnt, n_sets, st.off, c->q_scan, 0, s)) != JAM_OK) return rc;
-        hipLaunchKernelGGL(k_max_i32, dim3(1), dim3(1024), 0, s, (const int *)st.cnt, (long long)n_sets, st.maxcnt);
-        hipLaunchKernelGGL(jam::k_pairs, dim3((unsigned)((n_pairs + 7) / 8)), dim3(256), 0, s, dt, st, pr, qp);
+        if ((rc = device_scan<int, int64_t>(st.cnt, n_sets, st.off, c->q_scan, 0, s, st.maxcnt)) != JAM_OK) return rc;
+        hipLaunchKernelGGL(jam::k_pairs, dim3((unsigned)((n_pairs + 7) / 8)), dim3(256), 0, s, dt, st, pr, qp, pcm + 1);
         HIP_TRY(hipGetLastError());
         if ((rc = device_scan<int, long long>(pr.nchunk, n_pairs, pr.item_base, c->q_scan, 0, s)) != JAM_OK)
             return rc;
@@ -2054,17 +2040,13 @@ extern "C" int32_t jam_query(jam_context *c, const jam_templates *tp, const jam_
         // reads them with the join's counters, growing and running the query
         // again when something did not fit
         hipLaunchKernelGGL(jam::k_candidates<true>, dim3(set_blocks), dim3(64 * wpb), 0, s, dm, dt, st, pr,
-                           (long long *)(cnts + CNT_ITEMS));
+                           (long long *)(cnts + CNT_ITEMS), cnts, CNT_TOTAL);
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipEventRecord(c->ev[1], s));
         if ((rc = launch_kd(c, dm, dt, st, s, M == 1, ms->n_atoms)) != JAM_OK) {
             drain_kd(c);
             return rc;
         }
-        // the join's counters and level-0 flags do not depend on the kd
-        // order: set them up while the exact passes still run
-        hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, cnts, (long long)CNT_TOTAL);
-        hipLaunchKernelGGL(k_items_any, dim3(pair_blocks), dim3(256), 0, s, pr);
         HIP_TRY(kd_join(c, s));
         c->kd_pending = false;   // the rest of the query is ordered after every kd pass
         HIP_TRY(hipGetLastError());
@@ -2098,8 +2080,9 @@ extern "C" int32_t jam_query(jam_context *c, const jam_templates *tp, const jam_
             jn.out_cap = c->front_cap;
             jn.out_pair = c->j_pair[0].as<int>();
             jn.out_ent = c->j_ent[0].as<int>();
-            const unsigned l0_blocks = (unsigned)std::min<int64_t>(4096, (c->items_cap + 255) / 256);
-            hipLaunchKernelGGL(jam::k_level0, dim3(l0_blocks), dim3(256), 0, s, st, pr, jn);
+            const int team = n_pairs > 4096 ? JAM_WAVE : 256, teams = 256 / team;
+            hipLaunchKernelGGL(jam::k_level0, dim3((unsigned)((n_pairs + teams - 1) / teams)), dim3(256), 0, s, st, pr,
+                               jn, team);
             HIP_TRY(hipGetLastError());
             for (int L = 1; L <= levels; L++) {
                 const int bi = (L - 1) & 1, bo = L & 1;
@@ -2132,10 +2115,9 @@ extern "C" int32_t jam_query(jam_context *c, const jam_templates *tp, const jam_
         if (total >= INT32_MAX) return fail(JAM_ETOOBIG, "more than 2^31 candidate-set entries in one query");
         const unsigned int ovf = (unsigned int)(jc[CNT_OVF] & 0xFFFFFFFFull);
         const int64_t n_done = (int64_t)jc[CNT_DONE];
-        const bool regrow = total > c->set_cap || n0 > c->items_cap || n0 > c->front_cap;
+        const bool regrow = total > c->set_cap || n0 > c->front_cap;
         if (regrow) {
             if (total > c->set_cap && (rc = grow_sets(c, total, n_sets)) != JAM_OK) return rc;
-            if (n0 > c->items_cap && (rc = grow_items(c, n0)) != JAM_OK) return rc;
             if (n0 > c->front_cap && (rc = grow_front(c, std::max<int64_t>(2 * c->front_cap, n0), stride)) != JAM_OK)
                 return rc;
             continue;
@@ -2210,8 +2192,6 @@ extern "C" int32_t jam_query(jam_context *c, const jam_templates *tp, const jam_
         // marks and their scan reuse the (now free) 64-bit sort keys
         int *sel = c->s_key[0].as<int>();
         int *pos = c->s_key[1].as<int>();
-        hipLaunchKernelGGL(k_zero_u64, dim3((unsigned)std::min(1024, (n_pairs + 256) / 256)), dim3(256), 0, s, pcm,
-                           (long long)n_pairs + 1);
         if (n_done > 0) {
             const long long *first = c->p_first.as<long long>();
             // few matches: the mark pass keeps its superpositions for the emit
@@ -2228,21 +2208,15 @@ extern "C" int32_t jam_query(jam_context *c, const jam_templates *tp, const jam_
             hipLaunchKernelGGL(jam::k_first, dim3(gs), dim3(256), 0, s, jn, perm, (long long)n_done,
                                c->p_first.as<long long>());
             hipLaunchKernelGGL(jam::k_super<false>, dim3(gs), dim3(256), 0, s, dm, dt, st, pr, jn, ev, qp, perm,
-                               (long long)n_done, first, sel, (const int *)pos, keep_d, keep_i);
-            if ((rc = device_scan<int, int>((const int *)sel, (long long)n_done, pos, c->q_scan, 0, s)) != JAM_OK)
+                               (long long)n_done, first, sel, (const int *)pos, keep_d, keep_i, (long long *)(pcm + 1));
+            if ((rc = device_scan<int, int>((const int *)sel, (long long)n_done, pos, c->q_scan, 0, s, nullptr,
+                                            ev.count)) != JAM_OK)
                 return rc;
-            hipLaunchKernelGGL(jam::k_event_total, dim3(1), dim3(64), 0, s, (const int *)sel, (const int *)pos,
-                               (long long)n_done, ev.count);
             hipLaunchKernelGGL(jam::k_super<true>, dim3(gs), dim3(256), 0, s, dm, dt, st, pr, jn, ev, qp, perm,
-                               (long long)n_done, first, sel, (const int *)pos, keep_d, keep_i);
+                               (long long)n_done, first, sel, (const int *)pos, keep_d, keep_i, (long long *)(pcm + 1));
             HIP_TRY(hipGetLastError());
         }
         HIP_TRY(hipEventRecord(c->ev[4], s));
-        if (n_done > 0) {
-            hipLaunchKernelGGL(jam::k_pair_matches, dim3(gs), dim3(256), 0, s, jn, perm, (long long)n_done,
-                               (const long long *)c->p_first.as<long long>(), (long long *)(pcm + 1));
-            HIP_TRY(hipGetLastError());
-        }
         HIP_TRY(hipMemcpyAsync(c->hsmall, pcm, sizeof(unsigned long long) * ((size_t)n_pairs + 2),
                                hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));

@@ -96,13 +96,11 @@ struct PairLevel {
 struct DevPairs {
     int n_pairs;
     const long long *n_items; // level-0 partial matches in all (device scalar)
-    long long items_cap;      // capacity of item_pair
     unsigned char *ord;       // JAM_MAX_LEVELS per pair: level -> template atom
     PairLevel *lvl;           // JAM_MAX_LEVELS per pair
     int *nchunk;              // level-0 partial matches per pair
     int *n1;                  // first level-0 list index (1 for one-atom templates)
     long long *item_base;     // exclusive scan of nchunk
-    int *item_pair;           // pair of every level-0 partial
 };
 
 // One level of the join. Rows are partial matches: the pair and, per placed

@@ -80,13 +80,17 @@ __device__ static inline int find_bucket(const DevMols &ms, int b0, int b1, uint
 
 template <bool FILL>
 __global__ void __launch_bounds__(256) k_candidates(DevMols ms, DevTpls tp, DevSets st, DevPairs pr,
-                                                    long long *n_items)
+                                                    long long *n_items, unsigned long long *clear, int n_clear)
 {
-    if (FILL && blockIdx.x == 0 && threadIdx.x == 0) {
-        // level-0 items of all pairs: the end of the scan of the pair chunks
-        const int np = pr.n_pairs;
-        *st.kd_err = 0u;   // the kd passes come after this
-        *n_items = np > 0 ? pr.item_base[np - 1] + pr.nchunk[np - 1] : 0;
+    if (FILL && blockIdx.x == 0) {
+        // what the kernels after this one count in
+        if ((int)threadIdx.x < n_clear) clear[threadIdx.x] = 0ull;
+        if (threadIdx.x == 0) {
+            // level-0 items of all pairs: the end of the scan of the pair chunks
+            const int np = pr.n_pairs;
+            *st.kd_err = 0u;
+            *n_items = np > 0 ? pr.item_base[np - 1] + pr.nchunk[np - 1] : 0;
+        }
     }
     const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) / JAM_WAVE);
     const int lane = lane_id();
@@ -133,14 +137,17 @@ __global__ void __launch_bounds__(256) k_candidates(DevMols ms, DevTpls tp, DevS
 
 // Thread per pair: candidate-set sizes, the level order (stable by size when
 // reordering, _CandidateSet_size_compare_r, patches/Scanner.c.patch:98-108),
-// and the number of level-0 partial matches. A pair with an empty set has
+// and the number of level-0 partial matches; clears the pair's complete
+// matches, which the end of the query counts. A pair with an empty set has
 // none (Scanner_reuse returns NULL, patches/Scanner.c.patch:162-166).
 // Half a wave per pair, lane k for template atom k (templates have at most
 // 32 atoms): the level of atom k is its rank by (set size, k) when
 // reordering, k otherwise.
-__global__ void __launch_bounds__(256) k_pairs(DevTpls tp, DevSets st, DevPairs pr, QueryParams qp)
+__global__ void __launch_bounds__(256) k_pairs(DevTpls tp, DevSets st, DevPairs pr, QueryParams qp,
+                                               unsigned long long *pair_matches)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
+        pair_matches[-1] = 0ull;   // the event count
         // candidate-set entries of the query: the end of the scan of the set sizes
         const int ns = st.n_sets;
         *st.total = ns > 0 ? st.off[ns - 1] + st.cnt[ns - 1] : 0;
@@ -187,7 +194,10 @@ __global__ void __launch_bounds__(256) k_pairs(DevTpls tp, DevSets st, DevPairs 
         h.off = (int)off;
         pr.lvl[(size_t)p * JAM_MAX_LEVELS + rank] = h;
     }
-    if (valid && k == 0) pr.n1[p] = (n == 1) ? 1 : 0;
+    if (valid && k == 0) {
+        pr.n1[p] = (n == 1) ? 1 : 0;
+        pair_matches[p] = 0ull;
+    }
     // level-0 list size: the atom of rank 0; a one-atom template steps past
     // entry 0 before its first match
     if (valid && (n == 0 || any_empty) && k == 0) pr.nchunk[p] = 0;
@@ -221,21 +231,26 @@ __global__ void __launch_bounds__(256) k_pairs(DevTpls tp, DevSets st, DevPairs 
 // The buffers were sized before the sizes were known: when the candidate
 // sets, the items or the frontier do not fit, no row is written (the join then
 // has nothing to do) and the host grows the buffers and runs the query again.
-__global__ void __launch_bounds__(256) k_level0(DevSets st, DevPairs pr, DevJoin jn)
+// `team` threads per pair: a workgroup's 256 where the pairs are few, else a
+// wave's 64.
+__global__ void __launch_bounds__(256) k_level0(DevSets st, DevPairs pr, DevJoin jn, int team)
 {
     const long long n = *pr.n_items;
-    const bool fits = *st.total <= st.cap && n <= pr.items_cap && n <= jn.out_cap;
+    const bool fits = *st.total <= st.cap && n <= jn.out_cap;
     if (blockIdx.x == 0 && threadIdx.x == 0) *jn.n_out = fits ? (unsigned long long)n : 0ull;
     if (!fits) return;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (long long)gridDim.x * blockDim.x) {
-        const int p = pr.item_pair[i];
+    const int teams = 256 / team, mine = (int)threadIdx.x / team, lane = (int)threadIdx.x % team;
+    for (int p = blockIdx.x * teams + mine; p < pr.n_pairs; p += gridDim.x * teams) {
+        const int c = pr.nchunk[p];
+        if (c == 0) continue;
+        const long long base = pr.item_base[p];
         const int off0 = pr.lvl[(size_t)p * JAM_MAX_LEVELS].off;
-        int k = (int)(i - pr.item_base[p]);
         // a one-atom template steps past list entry 0: skip its kd position
-        if (pr.n1[p] && k >= st.l2k[off0]) k++;
-        jn.out_pair[i] = p;
-        jn.out_ent[i] = off0 + k;   // level 0's frontier: one entry per row
+        const int skip = pr.n1[p] ? st.l2k[off0] : INT32_MAX;
+        for (int i = lane; i < c; i += team) {
+            jn.out_pair[base + i] = p;
+            jn.out_ent[base + i] = off0 + i + (i >= skip ? 1 : 0);   // level 0's frontier: one entry per row
+        }
     }
 }
 
@@ -1154,16 +1169,6 @@ __global__ void __launch_bounds__(256) k_first(DevJoin jn, const int *perm, long
     if (s == 0 || jn.done_pair[perm[s - 1]] != p) first[p] = s;
 }
 
-// complete matches per pair
-__global__ void __launch_bounds__(256) k_pair_matches(DevJoin jn, const int *perm, long long n,
-                                                      const long long *first, long long *out)
-{
-    const long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const int p = jn.done_pair[perm[s]];
-    if (s == n - 1 || jn.done_pair[perm[s + 1]] != p) out[p] = s - first[p] + 1;
-}
-
 // ---------------------------------------------------------------------------
 // superposition + events
 // ---------------------------------------------------------------------------
@@ -1202,16 +1207,22 @@ __device__ __attribute__((always_inline)) static inline int super_of(DevMols ms,
 // Each event carries the match's rank within its pair.
 // With keep_d / keep_i (few matches), pass 1 also keeps each superposition
 // (16 doubles, then pair, size and atoms as stride + 2 ints per match) and
-// pass 2 reads it back instead of computing it again.
+// pass 2 reads it back instead of computing it again. Pass 2 also writes the
+// number of complete matches of every pair that has any.
 template <bool EMIT>
 __global__ void __launch_bounds__(256) k_super(DevMols ms, DevTpls tp, DevSets st, DevPairs pr, DevJoin jn,
                                                DevEvents ev, QueryParams qp, const int *perm, long long n_matches,
                                                const long long *first, int *sel, const int *pos, double *keep_d,
-                                               int *keep_i)
+                                               int *keep_i, long long *pair_matches)
 {
     const long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n_matches) return;
-    if (EMIT && !sel[s]) return;
+    if (EMIT) {
+        // the last match of a pair: its complete matches
+        const int p = jn.done_pair[perm[s]];
+        if (s == n_matches - 1 || jn.done_pair[perm[s + 1]] != p) pair_matches[p] = s - first[p] + 1;
+        if (!sel[s]) return;
+    }
     int atoms[JAM_MAX_LEVELS];
     int n, pair;
     double rmsd, rot[9], c0[3], c1[3];
@@ -1271,12 +1282,6 @@ __global__ void __launch_bounds__(256) k_super(DevMols ms, DevTpls tp, DevSets s
     }
     int *eat = (int *)(ev.base + L.atoms) + e * (size_t)ev.stride;
     for (int k = 0; k < ev.stride; k++) eat[k] = k < n ? atoms[k] : -1;
-}
-
-// number of events: the scan's last position plus the last mark
-__global__ void k_event_total(const int *sel, const int *pos, long long n, unsigned long long *count)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) *count = n > 0 ? (unsigned long long)(pos[n - 1] + sel[n - 1]) : 0ull;
 }
 
 // ---------------------------------------------------------------------------
