@@ -1174,12 +1174,13 @@ __global__ void __launch_bounds__(256) k_first(DevJoin jn, const int *perm, long
 // ---------------------------------------------------------------------------
 
 // Superposition of complete match s (sorted position): pair, molecule-local
-// atoms in template order, RMSD, rotation, centroids.
+// atoms in template order (atom k at atoms[k * JAM_WAVE]: a lane's column of
+// its wave's LDS), RMSD, rotation, centroids.
 __device__ __attribute__((always_inline)) static inline int super_of(DevMols ms, DevTpls tp, DevSets st,
                                                                      DevPairs pr, DevJoin jn, const int *perm,
-                                                                     long long s, int atoms[JAM_MAX_LEVELS],
-                                                                     int *n_out, double *rmsd, double rot[9],
-                                                                     double c0[3], double c1[3])
+                                                                     long long s, int *atoms, int *n_out,
+                                                                     double *rmsd, double rot[9], double c0[3],
+                                                                     double c1[3])
 {
     const int i = perm[s];
     const int pair = jn.done_pair[i];
@@ -1191,12 +1192,25 @@ __device__ __attribute__((always_inline)) static inline int super_of(DevMols ms,
     const unsigned char *ord = pr.ord + (size_t)pair * JAM_MAX_LEVELS;
     const int *row = jn.done_ent + (long long)i * jn.stride;
     // molecule-local atom of template atom k: placed at the level l with ord[l] == k
-    for (int l = 0; l < n; l++) atoms[ord[l]] = st.katom[row[l]];
-    auto pa = [&](int k, int d) { return ms.xyz[3 * (size_t)(abase + atoms[k]) + d]; };
+    for (int l = 0; l < n; l++) atoms[ord[l] * JAM_WAVE] = st.katom[row[l]];
+    auto pa = [&](int k, int d) { return ms.xyz[3 * (size_t)(abase + atoms[k * JAM_WAVE]) + d]; };
     auto pb = [&](int k, int d) { return tp.pos[3 * (size_t)(tbase + k) + d]; };
     superpose(n, pa, pb, rmsd, rot, c0, c1);
     *n_out = n;
     return pair;
+}
+
+// Writes the first `width` values of each of the wave's events (those of lanes
+// `on`, the r-th of them event e0 + r) to an array of `width` doubles per
+// event: through LDS, so that the stores are consecutive.
+__device__ static inline void emit_rows(double *lds, const double *v, int width, bool on, int r, int count,
+                                        double *out)
+{
+    if (on)
+        for (int k = 0; k < width; k++) lds[r * width + k] = v[k];
+    wave_sync();
+    for (int q = lane_id(); q < count * width; q += JAM_WAVE) out[q] = lds[q];
+    wave_sync();
 }
 
 // Thread per complete match, in reference order. Pass 1 (EMIT = false)
@@ -1209,41 +1223,57 @@ __device__ __attribute__((always_inline)) static inline int super_of(DevMols ms,
 // (16 doubles, then pair, size and atoms as stride + 2 ints per match) and
 // pass 2 reads it back instead of computing it again. Pass 2 also writes the
 // number of complete matches of every pair that has any.
+// Bound by the gathers of the match's atoms and coordinates, pass 2 by its
+// stores too: the events of a wave are consecutive, so its lanes write them
+// side by side, and a match's atoms lie in LDS instead of scratch memory
+// (6.3 M matches of 13 atoms on average, 5.9 M events: 0.56 and 1.22 ms ->
+// 0.48 and 0.80 ms).
 template <bool EMIT>
 __global__ void __launch_bounds__(256) k_super(DevMols ms, DevTpls tp, DevSets st, DevPairs pr, DevJoin jn,
                                                DevEvents ev, QueryParams qp, const int *perm, long long n_matches,
                                                const long long *first, int *sel, const int *pos, double *keep_d,
                                                int *keep_i, long long *pair_matches)
 {
+    // a wave's atoms, then (pass 2) its rotations and centroids
+    __shared__ double space[256 / JAM_WAVE][JAM_WAVE * JAM_MAX_LEVELS / 2];
+    __shared__ int event_lane[256 / JAM_WAVE][JAM_WAVE];   // of the r-th event: lane and atoms (* 64)
+    static_assert(JAM_MAX_LEVELS / 2 >= 9, "a wave's rotations fit");
     const long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n_matches) return;
-    if (EMIT) {
+    const int lane = lane_id(), w = (int)threadIdx.x / JAM_WAVE;
+    double *lds = space[w];
+    int *atoms = (int *)lds + lane;
+    bool on = s < n_matches;
+    long long e = 0;
+    if (EMIT && on) {
         // the last match of a pair: its complete matches
         const int p = jn.done_pair[perm[s]];
         if (s == n_matches - 1 || jn.done_pair[perm[s + 1]] != p) pair_matches[p] = s - first[p] + 1;
-        if (!sel[s]) return;
+        e = pos[s];
+        on = sel[s] && e < ev.cap;
     }
-    int atoms[JAM_MAX_LEVELS];
-    int n, pair;
-    double rmsd, rot[9], c0[3], c1[3];
+    int n = 0, pair = 0;
+    double rmsd = 0.0, rot[9], c0[3], c1[3];
     double *kd = keep_d ? keep_d + 16 * s : nullptr;
     int *ki = keep_i ? keep_i + (size_t)(ev.stride + 2) * s : nullptr;
-    if (EMIT && kd) {
-        rmsd = kd[0];
+    if (on) {
+        if (EMIT && kd) {
+            rmsd = kd[0];
 #pragma unroll
-        for (int k = 0; k < 9; k++) rot[k] = kd[1 + k];
+            for (int k = 0; k < 9; k++) rot[k] = kd[1 + k];
 #pragma unroll
-        for (int d = 0; d < 3; d++) {
-            c0[d] = kd[10 + d];
-            c1[d] = kd[13 + d];
+            for (int d = 0; d < 3; d++) {
+                c0[d] = kd[10 + d];
+                c1[d] = kd[13 + d];
+            }
+            pair = ki[0];
+            n = ki[1];
+            for (int k = 0; k < n; k++) atoms[k * JAM_WAVE] = ki[2 + k];
+        } else {
+            pair = super_of(ms, tp, st, pr, jn, perm, s, atoms, &n, &rmsd, rot, c0, c1);
         }
-        pair = ki[0];
-        n = ki[1];
-        for (int k = 0; k < n; k++) atoms[k] = ki[2 + k];
-    } else {
-        pair = super_of(ms, tp, st, pr, jn, perm, s, atoms, &n, &rmsd, rot, c0, c1);
     }
     if (!EMIT) {
+        if (!on) return;
         sel[s] = (rmsd <= qp.rmsd_threshold) ? 1 : 0;
         if (kd) {
             kd[0] = rmsd;
@@ -1256,32 +1286,36 @@ __global__ void __launch_bounds__(256) k_super(DevMols ms, DevTpls tp, DevSets s
             }
             ki[0] = pair;
             ki[1] = n;
-            for (int k = 0; k < n; k++) ki[2 + k] = atoms[k];
+            for (int k = 0; k < n; k++) ki[2 + k] = atoms[k * JAM_WAVE];
         }
         return;
     }
-    bool nan = false;
-#pragma unroll
-    for (int k = 0; k < 9; k++) nan |= isnan(rot[k]);
-    const long long e = pos[s];
-    if (e >= ev.cap) return;
+    const unsigned long long mask = ballot(on);
+    if (mask == 0ull) return;
+    const int count = __popcll(mask), r = rank_below(mask);
+    const long long e0 = __shfl(e, first_bit(mask), JAM_WAVE);
     const EventLayout L = event_layout((int64_t)*ev.count, ev.stride);
-    ((int *)(ev.base + L.pair))[e] = pair;
-    ((long long *)(ev.base + L.rank))[e] = s - first[pair];
-    ((int *)(ev.base + L.flag))[e] = nan ? 2 : 1;
-    ((double *)(ev.base + L.rmsd))[e] = rmsd;
-    double *erot = (double *)(ev.base + L.rot) + 9 * e;
-    double *ec0 = (double *)(ev.base + L.c0) + 3 * e;
-    double *ec1 = (double *)(ev.base + L.c1) + 3 * e;
+    if (on) {
+        bool nan = false;
 #pragma unroll
-    for (int k = 0; k < 9; k++) erot[k] = rot[k];
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-        ec0[d] = c0[d];
-        ec1[d] = c1[d];
+        for (int k = 0; k < 9; k++) nan |= isnan(rot[k]);
+        ((int *)(ev.base + L.pair))[e] = pair;
+        ((long long *)(ev.base + L.rank))[e] = s - first[pair];
+        ((int *)(ev.base + L.flag))[e] = nan ? 2 : 1;
+        ((double *)(ev.base + L.rmsd))[e] = rmsd;
+        event_lane[w][r] = n * JAM_WAVE + lane;
     }
-    int *eat = (int *)(ev.base + L.atoms) + e * (size_t)ev.stride;
-    for (int k = 0; k < ev.stride; k++) eat[k] = k < n ? atoms[k] : -1;
+    wave_sync();
+    int *eat = (int *)(ev.base + L.atoms) + e0 * (size_t)ev.stride;
+    for (int q = lane; q < count * ev.stride; q += JAM_WAVE) {
+        const int x = q / ev.stride, k = q - x * ev.stride;
+        const int nl = event_lane[w][x];
+        eat[q] = k < nl / JAM_WAVE ? ((const int *)lds)[k * JAM_WAVE + nl % JAM_WAVE] : -1;
+    }
+    wave_sync();
+    emit_rows(lds, rot, 9, on, r, count, (double *)(ev.base + L.rot) + 9 * e0);
+    emit_rows(lds, c0, 3, on, r, count, (double *)(ev.base + L.c0) + 3 * e0);
+    emit_rows(lds, c1, 3, on, r, count, (double *)(ev.base + L.c1) + 3 * e0);
 }
 
 // ---------------------------------------------------------------------------
