@@ -1584,17 +1584,22 @@ __global__ void k_zero_u64(unsigned long long *v, long long n)
 // GROUP_RANK_MATCHES matches with up to GROUP_RANK_WORK comparisons (halved)
 // every group is ranked by comparison: the LDS sort's tiles would leave most
 // CUs idle (49,000 matches: 46 us in 4 passes). Above, groups of up to
-// GROUP_TILE / 2 matches are sorted in LDS (6.3 M matches: 0.72 ms) and larger
+// GROUP_TILE / 2 matches are sorted in LDS (470,000 matches: 0.25 ms) and larger
 // ones ranked, about 1.8 us per million comparisons (halved) and pass: past
 // group_work_max of them the radix passes are faster (470,000 matches of a
 // 100,000-atom assembly, 28 M in large groups: 0.56 ms against 1.7 ms by radix
-// passes; 6.3 M matches, 550 M in large groups: 3.2 against 2.4 ms).
+// passes; 6.3 M matches, 550 M in large groups: 3.2 against 2.4 ms). More than
+// GROUP_MATCHES_MAX matches go by radix passes at once: so many come from
+// symmetric templates, whose groups are large, and finding that out costs 0.3
+// ms for 6.3 M matches and 2.5 ms for the 51 M of 16 assemblies x 7,000
+// templates.
 #ifndef GROUP_RANK_WORK
 #define GROUP_RANK_WORK 8000000ull
 #endif
 #ifndef GROUP_RANK_MATCHES
 #define GROUP_RANK_MATCHES 131072
 #endif
+constexpr int64_t GROUP_MATCHES_MAX = int64_t(1) << 22;
 unsigned long long group_work_max(int64_t n) { return 200000000ull + 16ull * (unsigned long long)n; }
 
 // workgroups of `kernel` (with `threads` threads) that stay resident on the device
@@ -1868,12 +1873,13 @@ int32_t sort_radix(jam_context *c, const DevSets &st, const DevTpls &dt, const D
 
 // The same by groups of level-0 rows (k_group_count ... k_group_tile); the
 // result is `perm`. `perm` stays null, with nothing sorted, where the rows
-// cannot be numbered in 32 bits or the groups are too large.
+// cannot be numbered in 32 bits, or the matches are too many or their groups
+// too large.
 int32_t sort_groups(jam_context *c, const DevSets &st, const DevTpls &dt, const DevPairs &pr, const DevJoin &jn,
                     int64_t n_done, int64_t n_rows, int stride, int bits, hipStream_t s, const int *&perm)
 {
     perm = nullptr;
-    if (n_rows > (int64_t)UINT32_MAX) return JAM_OK;
+    if (n_rows > (int64_t)UINT32_MAX || n_done > GROUP_MATCHES_MAX) return JAM_OK;
     // about as many groups as matches: fewer would mean more comparisons,
     // more a longer scan
     int shift = 0;
