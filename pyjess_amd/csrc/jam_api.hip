@@ -173,7 +173,8 @@ struct jam_context {
     // next query on the context
     uint64_t query_gen = 0;
     // pinned host staging for event copies: stage_slots slots of
-    // JAM_STAGE_BYTES
+    // JAM_STAGE_BYTES; one copy at a time uses them
+    std::mutex stage_mutex;
     void *hstage = nullptr;
     int stage_slots = 0;
     hipEvent_t stage_ev[16] = {};
@@ -811,6 +812,7 @@ int32_t copy_out(jam_context *c, const std::vector<CopyPiece> &pieces)
         i = j;
     }
     if (batches.empty()) return JAM_OK;
+    std::lock_guard<std::mutex> guard(c->stage_mutex);
     const int nt = (int)std::min<size_t>(JAM_STAGE_THREADS, (batches.size() + 1) / 2);
     int32_t rc = grow_stage(c, (int)std::min<size_t>(batches.size(), 2 * (size_t)nt));
     if (rc != JAM_OK) return rc;
