@@ -287,9 +287,10 @@ extern "C" int32_t jam_rmsd_forward(const double *a, const double *b, const int6
     if (n_sets < 0 || n_points < 0) return fail(JAM_EINVAL, "invalid sizes");
     if (n_sets == 0) return JAM_OK;
     if (!off || !rmsd || (n_points > 0 && (!a || !b))) return fail(JAM_EINVAL, "NULL argument");
-    const int tb = RG_SETS;
-    hipLaunchKernelGGL(jam::k_rmsd_fwd, dim3((unsigned)((n_sets + tb - 1) / tb)), dim3(tb), 0,
-                       (hipStream_t)stream, a, b, off, (long long)n_sets, (long long)n_points, rmsd, rot9);
+    const int64_t tiles = (n_sets + RG_SETS - 1) / RG_SETS;
+    auto *kernel = tiles <= RG_FEW_TILES ? jam::k_rmsd_fwd<false> : jam::k_rmsd_fwd<true>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(RG_SETS), 0, (hipStream_t)stream, a, b, off,
+                       (long long)n_sets, (long long)n_points, rmsd, rot9);
     HIP_TRY(hipGetLastError());
     return JAM_OK;
 }
@@ -302,10 +303,10 @@ extern "C" int32_t jam_rmsd_backward(const double *a, const double *b, const int
     if (n_sets == 0) return JAM_OK;
     if (!off || !rmsd || !grad_rmsd || (!grad_a && !grad_b) || (n_points > 0 && (!a || !b)))
         return fail(JAM_EINVAL, "NULL argument");
-    const int tb = RG_SETS;
-    hipLaunchKernelGGL(jam::k_rmsd_bwd, dim3((unsigned)((n_sets + tb - 1) / tb)), dim3(tb), 0,
-                       (hipStream_t)stream, a, b, off, (long long)n_sets, (long long)n_points, rmsd, rot9,
-                       grad_rmsd, grad_a, grad_b);
+    const int64_t tiles = (n_sets + RG_SETS - 1) / RG_SETS;
+    auto *kernel = tiles <= RG_FEW_TILES ? jam::k_rmsd_bwd<false> : jam::k_rmsd_bwd<true>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(RG_SETS), 0, (hipStream_t)stream, a, b, off,
+                       (long long)n_sets, (long long)n_points, rmsd, rot9, grad_rmsd, grad_a, grad_b);
     HIP_TRY(hipGetLastError());
     return JAM_OK;
 }

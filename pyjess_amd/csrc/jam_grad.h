@@ -131,151 +131,158 @@ __device__ static inline void optimal_rotation(const double X[3][3], double R[3]
         for (int k = 0; k < 3; k++) R[j][k] = u1[j] * v1[k] + u2[j] * v2[k] + sgn * u3[j] * v3[k];
 }
 
-// Centroids and the correlation X of points [0, n) of A and B.
-__device__ static inline void centre_and_correlate(int n, const double *A, const double *B, double ca[3],
-                                                   double cb[3], double X[3][3])
+// One point of a set (a's at A, b's at B, three doubles each) added to the
+// sums of the centroids.
+__device__ static inline void add_centroid(const double *A, const double *B, double ca[3], double cb[3])
+{
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        ca[d] += A[d];
+        cb[d] += B[d];
+    }
+}
+
+// ... to the correlation X.
+__device__ static inline void add_correlation(const double *A, const double *B, const double ca[3],
+                                              const double cb[3], double X[3][3])
+{
+    double u[3], v[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        u[d] = A[d] - ca[d];
+        v[d] = B[d] - cb[d];
+    }
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+#pragma unroll
+        for (int k = 0; k < 3; k++) X[j][k] += v[j] * u[k];
+}
+
+// ... to the squared residuals of rotation R.
+__device__ static inline void add_residual(const double *A, const double *B, const double ca[3], const double cb[3],
+                                           const double R[3][3], double &e)
+{
+    double u[3], v[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        u[d] = A[d] - ca[d];
+        v[d] = B[d] - cb[d];
+    }
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const double ra = R[d][0] * u[0] + R[d][1] * u[1] + R[d][2] * u[2];
+        const double r = v[d] - ra;
+        e += r * r;
+    }
+}
+
+// The point's gradients, in place of the point (scale: the RMSD's gradient over
+// n * rmsd).
+__device__ static inline void to_gradient(double *A, double *B, const double ca[3], const double cb[3],
+                                          const double R[3][3], double scale)
+{
+    double u[3], v[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        u[d] = A[d] - ca[d];
+        v[d] = B[d] - cb[d];
+    }
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        // (R^T B_i)_d and (R A_i)_d
+        const double rtb = R[0][d] * v[0] + R[1][d] * v[1] + R[2][d] * v[2];
+        const double ra = R[d][0] * u[0] + R[d][1] * u[1] + R[d][2] * u[2];
+        A[d] = scale * (u[d] - rtb);
+        B[d] = scale * (v[d] - ra);
+    }
+}
+
+// The sums above over a set of n points, which `each` hands to its argument in
+// order.
+template <class E>
+__device__ static inline void centroids(int n, E each, double ca[3], double cb[3])
 {
 #pragma unroll
     for (int d = 0; d < 3; d++) {
         ca[d] = 0.0;
         cb[d] = 0.0;
     }
-    for (int i = 0; i < n; i++)
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            ca[d] += A[3 * i + d];
-            cb[d] += B[3 * i + d];
-        }
+    each([&](double *A, double *B) { add_centroid(A, B, ca, cb); });
 #pragma unroll
     for (int d = 0; d < 3; d++) {
         ca[d] /= (double)n;
         cb[d] /= (double)n;
     }
+}
+
+template <class E>
+__device__ static inline void correlate(E each, const double ca[3], const double cb[3], double X[3][3])
+{
 #pragma unroll
     for (int j = 0; j < 3; j++)
 #pragma unroll
         for (int k = 0; k < 3; k++) X[j][k] = 0.0;
-    for (int i = 0; i < n; i++) {
-        double u[3], v[3];
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            u[d] = A[3 * i + d] - ca[d];
-            v[d] = B[3 * i + d] - cb[d];
-        }
-#pragma unroll
-        for (int j = 0; j < 3; j++)
-#pragma unroll
-            for (int k = 0; k < 3; k++) X[j][k] += v[j] * u[k];
-    }
+    each([&](double *A, double *B) { add_correlation(A, B, ca, cb, X); });
 }
 
-// One set: RMSD from the residuals of rotation R.
-__device__ static inline double residual_rmsd(int n, const double *A, const double *B, const double ca[3],
-                                              const double cb[3], const double R[3][3])
+template <class E>
+__device__ static inline double residual(int n, E each, const double ca[3], const double cb[3], const double R[3][3])
 {
     double e = 0.0;
-    for (int i = 0; i < n; i++) {
-        double u[3], v[3];
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            u[d] = A[3 * i + d] - ca[d];
-            v[d] = B[3 * i + d] - cb[d];
-        }
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            const double ra = R[d][0] * u[0] + R[d][1] * u[1] + R[d][2] * u[2];
-            const double r = v[d] - ra;
-            e += r * r;
-        }
-    }
+    each([&](double *A, double *B) { add_residual(A, B, ca, cb, R, e); });
     return sqrt(e / (double)n);
 }
 
-// One set: the gradient of g * rmsd, written to GA / GB (which may alias A /
-// B: every point is read before its gradient is written). rot: the set's
-// optimal rotation from the forward pass, or null to compute it again.
-__device__ __attribute__((always_inline)) static inline void rmsd_grad_one(int n, const double *A, const double *B,
-                                                                           double r, double g, const double *rot,
-                                                                           double *GA, double *GB)
-{
-    if (!(r > 0.0) || g == 0.0) {
-        for (int q = 0; q < 3 * n; q++) {
-            if (GA) GA[q] = 0.0;
-            if (GB) GB[q] = 0.0;
-        }
-        return;
-    }
-    double ca[3], cb[3], R[3][3];
-    if (rot) {
-        // centroids only: the rotation is the forward pass's
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            ca[d] = 0.0;
-            cb[d] = 0.0;
-        }
-        for (int i = 0; i < n; i++)
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                ca[d] += A[3 * i + d];
-                cb[d] += B[3 * i + d];
-            }
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            ca[d] /= (double)n;
-            cb[d] /= (double)n;
-        }
-#pragma unroll
-        for (int j = 0; j < 3; j++)
-#pragma unroll
-            for (int k = 0; k < 3; k++) R[j][k] = rot[3 * j + k];
-    } else {
-        double X[3][3];
-        centre_and_correlate(n, A, B, ca, cb, X);
-        optimal_rotation(X, R);
-    }
-    const double scale = g / ((double)n * r);
-    for (int i = 0; i < n; i++) {
-        double u[3], v[3];
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            u[d] = A[3 * i + d] - ca[d];
-            v[d] = B[3 * i + d] - cb[d];
-        }
-        double ga[3], gb[3];
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            // (R^T B_i)_d and (R A_i)_d
-            const double rtb = R[0][d] * v[0] + R[1][d] * v[1] + R[2][d] * v[2];
-            const double ra = R[d][0] * u[0] + R[d][1] * u[1] + R[d][2] * u[2];
-            ga[d] = scale * (u[d] - rtb);
-            gb[d] = scale * (v[d] - ra);
-        }
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            if (GA) GA[3 * i + d] = ga[d];
-            if (GB) GB[3 * i + d] = gb[d];
-        }
-    }
-}
-
-// One wave per tile of RG_SETS consecutive sets (one set per lane), its points
-// moved by coalesced loads and stores through one LDS buffer. A tile of sets of
-// up to RG_REG points that fits the buffer (RG_CAP points of one array) goes
-// through it an array at a time: a, which every lane takes into registers, then
-// b, which stays in LDS; the gradients leave the same way (in the forward pass
-// larger sets may be among them). Any other tile goes in rounds of as many sets as the buffer holds of both arrays (RG_CAP / 2
-// points); a set too large for that is read from global memory by its lane.
+// One wave per tile of RG_SETS consecutive sets (one set per lane), a lane
+// summing its set point by point: the same operations in the same order
+// whichever way the points reach it.
 //
-// Bound by latency: the rotation is a chain of some hundreds of dependent FP64
-// operations per lane, so what counts is the waves per SIMD: one array in LDS
-// (18 KB) instead of two (37 KB) makes them two instead of one, and the loads
-// of both arrays are all in flight before the first LDS store. 1 M sets of 3 to
-// 12 points, forward and backward: 0.49 -> 0.31 ms (0.25 ms at the rate of a
-// copy); 400,000 sets of 24 points: 1.27 -> 0.67 ms.
+// k_rmsd_*<false>, up to RG_FEW_TILES tiles: one wave for each of the 1,024
+// SIMDs, which do not compete for the caches. Both arrays of the tile in LDS (37
+// KB) where its points fit, else every lane reads its set from global memory,
+// RG_FAR points in flight. 64 sets of 8 points, forward and backward: 14 + 11 us;
+// of 200: 77 + 128 us (in chunks 374 + 351).
+//
+// k_rmsd_*<true>, more tiles: bound by the waves per SIMD (the rotation is a chain of some hundreds
+// of dependent FP64 operations) and by memory, so one array in LDS (18 KB) and
+// two waves per SIMD, whose lanes reading 64 sets at once would thrash the L1 (1.25 M
+// sets of 16 points: 1.05 + 2.0 ms):
+//   sets of at most RG_REG points, together at most RG_CAP: a through LDS into
+//     registers, then b, which stays there; the gradients leave the same way. In
+//     the forward pass larger sets may be among them, whose lanes read the
+//     array that is not in LDS from global memory. 1 M sets of 3 to 12 points, forward
+//     and backward: 0.31 ms, against 0.49 with both arrays in LDS (0.25 at the
+//     rate of a copy);
+//   else up to RG_ROUNDS rounds of as many sets as LDS holds of both arrays (a
+//     set too large for that alone, from global memory): 416,666 sets of 24 points
+//     (four rounds) 0.31 + 0.29 ms, in chunks 0.39 + 0.40;
+//   else RG_CHUNK points of every set at a time, once for each of the sums
+//     (centroids, correlation, residuals or gradients), the next chunk's loads
+//     in flight: all lanes work, and the rotation is done once. 312,500 sets of 32
+//     points 0.39 + 0.45 ms, in six rounds 0.46 + 0.45; 50,000 of 200 points
+//     and up in rounds of one to three lanes: 7 ms and more.
 #define RG_SETS 64
-#define RG_CAP 768   // points per tile held in LDS (12 per set on average)
 #define RG_REG 12    // points of a set held in registers
+#define RG_CAP (RG_SETS * RG_REG)   // points of one array held in LDS
 #define RG_LOADS (3 * RG_CAP / RG_SETS)
+#define RG_NEAR 2    // points in flight from LDS
+#define RG_FAR 4     // ... from global memory
+#define RG_FEW_TILES 1024
+#define RG_ROUNDS 4
+#define RG_CHUNK 5   // 15 doubles a set: an odd stride, so that the lanes' reads spread over the banks
+#define RG_TEAM 16   // lanes that load a set's chunk
+#define RG_ROWS (RG_SETS * RG_TEAM / JAM_WAVE)
+
+struct RmsdChunks {
+    double a[RG_SETS * 3 * RG_CHUNK], b[RG_SETS * 3 * RG_CHUNK];
+    long long at[RG_SETS], len[RG_SETS];   // each set's first double and number of doubles
+};
+
+template <bool MANY>
+union RmsdLds {
+    double l[3 * RG_CAP * (MANY ? 1 : 2)];
+    RmsdChunks c;
+};
 
 // m doubles of src (m <= N * RG_SETS), one in RG_SETS to each lane
 template <int N>
@@ -298,18 +305,23 @@ __device__ static inline void tile_store(const double (&r)[N], int m, int lane, 
     }
 }
 
-// m doubles of a and of b (m <= 3 * RG_CAP / 2) into LDS
-__device__ static inline void stage_pair(const double *a, const double *b, int m, int lane, double *la, double *lb)
+// m doubles of a and of b into LDS, the loads of N * RG_SETS of each in flight
+template <int N>
+__device__ static inline void stage_both(const double *a, const double *b, int m, int lane, double *la, double *lb)
 {
-    double ra[RG_LOADS / 2], rb[RG_LOADS / 2];
-    tile_load(a, m, lane, ra);
-    tile_load(b, m, lane, rb);
-    tile_store(ra, m, lane, la);
-    tile_store(rb, m, lane, lb);
+    for (int q = 0; q < m; q += N * RG_SETS) {
+        double ra[N], rb[N];
+        tile_load(a + q, m - q, lane, ra);
+        tile_load(b + q, m - q, lane, rb);
+        tile_store(ra, m - q, lane, la + q);
+        tile_store(rb, m - q, lane, lb + q);
+    }
+    wave_sync();
 }
 
 // Both arrays of the tile: a's points of this lane's set (n of them from p)
-// into A, b's into LDS; `between` runs while a's are there.
+// into A where they are at most RG_REG, b's into LDS; `between` runs while a's
+// are there.
 template <class F>
 __device__ static inline void stage_tile(const double *a, const double *b, int m, int lane, int p, int n, double *l,
                                          double (&A)[3 * RG_REG], F between)
@@ -322,129 +334,123 @@ __device__ static inline void stage_tile(const double *a, const double *b, int m
 #pragma unroll
     for (int i = 0; i < RG_REG; i++)
 #pragma unroll
-        for (int d = 0; d < 3; d++) A[3 * i + d] = (i < n && n <= RG_REG) ? l[3 * (p + i) + d] : 0.0;
+        for (int d = 0; d < 3; d++) A[3 * i + d] = i < n && n <= RG_REG ? l[3 * (p + i) + d] : 0.0;
     between();
     wave_sync();
     tile_store(rb, m, lane, l);
     wave_sync();
 }
 
-// The functions above (whose operations and order these keep) for A in
-// registers, n <= RG_REG.
-__device__ static inline void centroids_reg(int n, const double (&A)[3 * RG_REG], const double *B, double ca[3],
-                                            double cb[3])
+// The points of a set in registers (A) and LDS (B), n <= RG_REG.
+template <class F>
+__device__ static inline void each_staged(int n, double (&A)[3 * RG_REG], double *B, F point)
 {
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-        ca[d] = 0.0;
-        cb[d] = 0.0;
-    }
+    for (int i = 0; i < RG_REG; i++)
+        if (i < n) point(A + 3 * i, B + 3 * i);
+}
+
+// The points of a set at A and B, the loads of U points in flight.
+template <int U, class F>
+__device__ static inline void each_at(int n, const double *A, const double *B, F point)
+{
+#pragma unroll U
+    for (int i = 0; i < n; i++) {
+        double x[3], y[3];
 #pragma unroll
-    for (int i = 0; i < RG_REG; i++) {
-        if (i < n) {
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                ca[d] += A[3 * i + d];
-                cb[d] += B[3 * i + d];
-            }
+        for (int d = 0; d < 3; d++) {
+            x[d] = A[3 * i + d];
+            y[d] = B[3 * i + d];
         }
-    }
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-        ca[d] /= (double)n;
-        cb[d] /= (double)n;
+        point(x, y);
     }
 }
 
-__device__ static inline void correlate_reg(int n, const double (&A)[3 * RG_REG], const double *B, const double ca[3],
-                                            const double cb[3], double X[3][3])
+// The same, what point() makes of them going to GA and GB (each may be null;
+// they may be A and B).
+template <int U, class F>
+__device__ static inline void each_into(int n, const double *A, const double *B, double *GA, double *GB, F point)
 {
+    int i = 0;
+    each_at<U>(n, A, B, [&](double *x, double *y) {
+        point(x, y);
 #pragma unroll
-    for (int j = 0; j < 3; j++)
-#pragma unroll
-        for (int k = 0; k < 3; k++) X[j][k] = 0.0;
-#pragma unroll
-    for (int i = 0; i < RG_REG; i++) {
-        if (i < n) {
-            double u[3], v[3];
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                u[d] = A[3 * i + d] - ca[d];
-                v[d] = B[3 * i + d] - cb[d];
-            }
-#pragma unroll
-            for (int j = 0; j < 3; j++)
-#pragma unroll
-                for (int k = 0; k < 3; k++) X[j][k] += v[j] * u[k];
+        for (int d = 0; d < 3; d++) {
+            if (GA) GA[3 * i + d] = x[d];
+            if (GB) GB[3 * i + d] = y[d];
         }
+        i++;
+    });
+}
+
+// Doubles [3c, 3c + 15) of every set of the tile, RG_TEAM lanes a set.
+__device__ static inline void chunk_load(const RmsdChunks &S, const double *src, long long c, int lane,
+                                         double (&r)[RG_ROWS])
+{
+    const int i = lane % RG_TEAM;
+#pragma unroll
+    for (int u = 0; u < RG_ROWS; u++) {
+        const int j = u * (JAM_WAVE / RG_TEAM) + lane / RG_TEAM;
+        const bool in = i < 3 * RG_CHUNK && 3 * c + i < S.len[j];
+        r[u] = in ? src[S.at[j] + 3 * c + i] : 0.0;
     }
 }
 
-__device__ static inline double residual_reg(int n, const double (&A)[3 * RG_REG], const double *B, const double ca[3],
-                                             const double cb[3], const double R[3][3])
+__device__ static inline void chunk_put(double *l, int lane, const double (&r)[RG_ROWS])
 {
-    double e = 0.0;
+    const int i = lane % RG_TEAM;
 #pragma unroll
-    for (int i = 0; i < RG_REG; i++) {
-        if (i < n) {
-            double u[3], v[3];
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                u[d] = A[3 * i + d] - ca[d];
-                v[d] = B[3 * i + d] - cb[d];
-            }
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                const double ra = R[d][0] * u[0] + R[d][1] * u[1] + R[d][2] * u[2];
-                const double r = v[d] - ra;
-                e += r * r;
-            }
-        }
-    }
-    return sqrt(e / (double)n);
+    for (int u = 0; u < RG_ROWS; u++)
+        if (i < 3 * RG_CHUNK) l[(u * (JAM_WAVE / RG_TEAM) + lane / RG_TEAM) * 3 * RG_CHUNK + i] = r[u];
 }
 
-// gradients replace A and B
-__device__ static inline void rmsd_grad_reg(int n, double (&A)[3 * RG_REG], double *B, double r, double g,
-                                            const double *rot)
+__device__ static inline void chunk_store(const RmsdChunks &S, const double *l, long long c, int lane, double *dst)
 {
-    if (!(r > 0.0) || g == 0.0) {
+    const int i = lane % RG_TEAM;
 #pragma unroll
-        for (int q = 0; q < 3 * RG_REG; q++) A[q] = 0.0;
-        for (int q = 0; q < 3 * n; q++) B[q] = 0.0;
-        return;
+    for (int u = 0; u < RG_ROWS; u++) {
+        const int j = u * (JAM_WAVE / RG_TEAM) + lane / RG_TEAM;
+        if (i < 3 * RG_CHUNK && 3 * c + i < S.len[j]) dst[S.at[j] + 3 * c + i] = l[j * 3 * RG_CHUNK + i];
     }
-    double ca[3], cb[3], R[3][3];
-    centroids_reg(n, A, B, ca, cb);
-    if (rot) {
-#pragma unroll
-        for (int j = 0; j < 3; j++)
-#pragma unroll
-            for (int k = 0; k < 3; k++) R[j][k] = rot[3 * j + k];
-    } else {
-        double X[3][3];
-        correlate_reg(n, A, B, ca, cb, X);
-        optimal_rotation(X, R);
-    }
-    const double scale = g / ((double)n * r);
-#pragma unroll
-    for (int i = 0; i < RG_REG; i++) {
-        if (i < n) {
-            double u[3], v[3];
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                u[d] = A[3 * i + d] - ca[d];
-                v[d] = B[3 * i + d] - cb[d];
-            }
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                const double rtb = R[0][d] * v[0] + R[1][d] * v[1] + R[2][d] * v[2];
-                const double ra = R[d][0] * u[0] + R[d][1] * u[1] + R[d][2] * u[2];
-                A[3 * i + d] = scale * (u[d] - rtb);
-                B[3 * i + d] = scale * (v[d] - ra);
-            }
+}
+
+// point() for every point of the lanes' sets (n of the lane's, `most` of the
+// largest), a chunk at a time; after(c) when all lanes are done with chunk c.
+// The whole wave calls it.
+template <class F, class G>
+__device__ static inline void each_chunked(const double *a, const double *b, RmsdChunks &S, int n, int most, int lane,
+                                           F point, G after)
+{
+    double ra[RG_ROWS], rb[RG_ROWS];
+    chunk_load(S, a, 0, lane, ra);
+    chunk_load(S, b, 0, lane, rb);
+    for (long long c = 0; c < most; c += RG_CHUNK) {
+        wave_sync();
+        chunk_put(S.a, lane, ra);
+        chunk_put(S.b, lane, rb);
+        wave_sync();
+        if (c + RG_CHUNK < most) {
+            chunk_load(S, a, c + RG_CHUNK, lane, ra);
+            chunk_load(S, b, c + RG_CHUNK, lane, rb);
         }
+#pragma unroll
+        for (int i = 0; i < RG_CHUNK; i++)
+            if (c + i < n) point(S.a + 3 * (RG_CHUNK * lane + i), S.b + 3 * (RG_CHUNK * lane + i));
+        after(c);
     }
+    wave_sync();
+}
+
+// The table of the lanes' sets ([p0, p0 + n) of each), and the largest n.
+__device__ static inline int chunk_table(RmsdChunks &S, int64_t p0, int n, int lane)
+{
+    S.at[lane] = 3 * (long long)p0;
+    S.len[lane] = 3 * (long long)max(n, 0);
+    wave_sync();
+    int most = n;
+#pragma unroll
+    for (int sh = JAM_WAVE / 2; sh >= 1; sh >>= 1) most = max(most, __shfl_xor(most, sh, JAM_WAVE));
+    return most;
 }
 
 // Range of set s, clamped into [lo, hi]: with valid offsets (off[0] = 0,
@@ -474,146 +480,215 @@ __device__ static inline void tile_ranges(const int64_t *off, long long n_sets, 
     if (s < s1) set_range(off, s, P0, P1, p0, p1);
 }
 
-// The sets [g0, g1) of the tile that one round takes: its first point, and g1
-// (g0 where the first set alone is too large). The lanes' ranges never
-// descend, so that those that fit are the first ones.
-__device__ static inline int64_t tile_round(int64_t p0, int64_t p1, int g0, int lane, int &g1)
+// The sets [g0, g1) of the tile that one round takes, and their points [q0, q1):
+// those that fit half the buffer, or one set alone, where that is larger. The
+// lanes' ranges never descend, so that those that fit are the first ones.
+__device__ static inline bool tile_round(int64_t p0, int64_t p1, int g0, int lane, int &g1, int64_t &q0, int64_t &q1)
 {
-    const int64_t q0 = __shfl(p0, g0, JAM_WAVE);
-    g1 = g0 + __popcll(ballot(lane >= g0 && p1 - q0 <= RG_CAP / 2));
-    return q0;
+    q0 = __shfl(p0, g0, JAM_WAVE);
+    const int fit = __popcll(ballot(lane >= g0 && p1 - q0 <= RG_CAP / 2));
+    g1 = g0 + max(fit, 1);
+    q1 = __shfl(p1, g1 - 1, JAM_WAVE);
+    // within the buffer whatever the offsets
+    if (fit) q1 = q1 < q0 ? q0 : (q1 > q0 + RG_CAP / 2 ? q0 + RG_CAP / 2 : q1);
+    return fit > 0;
 }
 
-// The round's end: the last point of its last set, within the buffer whatever
-// the offsets.
-__device__ static inline int64_t round_end(int64_t p1, int64_t q0, int g1)
+// Whether the tile takes at most `most` rounds.
+__device__ static inline bool few_rounds(int64_t p0, int64_t p1, int lane, int most)
 {
-    const int64_t q1 = __shfl(p1, g1 - 1, JAM_WAVE);
-    return q1 < q0 ? q0 : (q1 > q0 + RG_CAP / 2 ? q0 + RG_CAP / 2 : q1);
+    int g1 = 0;
+    int64_t q0, q1;
+    for (int k = 0; k < most && g1 < RG_SETS; k++) (void)tile_round(p0, p1, g1, lane, g1, q0, q1);
+    return g1 >= RG_SETS;
+}
+
+// RMSD and rotation of a set of n points.
+template <class E>
+__device__ static inline double rmsd_of(int n, E each, double R[3][3])
+{
+    double ca[3], cb[3], X[3][3];
+    centroids(n, each, ca, cb);
+    correlate(each, ca, cb, X);
+    optimal_rotation(X, R);
+    return residual(n, each, ca, cb, R);
 }
 
 // Set s owns points [off[s], off[s+1]) of a and b, 3 doubles per point.
-__global__ void __launch_bounds__(RG_SETS, 2) k_rmsd_fwd(const double *a, const double *b, const int64_t *off,
-                                                         long long n_sets, long long n_points, double *rmsd,
-                                                         double *rot)
+template <bool MANY>
+__global__ void __launch_bounds__(RG_SETS, MANY ? 2 : 1) k_rmsd_fwd(const double *a, const double *b,
+                                                                   const int64_t *off, long long n_sets,
+                                                                   long long n_points, double *rmsd, double *rot)
 {
-    __shared__ double l[3 * RG_CAP];
+    __shared__ RmsdLds<MANY> S;
     const int lane = threadIdx.x;
     const long long s = (long long)blockIdx.x * RG_SETS + lane;
     int64_t P0, P1, p0, p1;
     tile_ranges(off, n_sets, n_points, s, P0, P1, p0, p1);
     const int n = (int)(p1 - p0);
-    double r = 0.0;
-    double *rt = rot ? rot + 9 * s : nullptr;
-    double ca[3], cb[3], X[3][3], R[3][3];
-    if (P1 - P0 <= RG_CAP) {
-        // larger sets than the registers hold read the array that is not in
-        // LDS from global memory, where the tile's loads have just been
-        const int at = (int)(p0 - P0);
-        const bool small = n <= RG_REG;
-        double A[3 * RG_REG];
-        stage_tile(a + 3 * P0, b + 3 * P0, (int)(3 * (P1 - P0)), lane, at, n, l, A, [&] {
-            if (!small) centre_and_correlate(n, l + 3 * at, b + 3 * p0, ca, cb, X);
+    const bool fits = P1 - P0 <= RG_CAP;
+    const int at = 3 * (int)(p0 - P0), m = (int)(3 * (P1 - P0));   // where it fits
+    double r = 0.0, R[3][3];
+    if (!MANY) {
+        if (fits) {
+            const double *A = S.l + at, *B = A + 3 * RG_CAP;
+            stage_both<12>(a + 3 * P0, b + 3 * P0, m, lane, S.l, S.l + 3 * RG_CAP);
+            if (n > 0) r = rmsd_of(n, [&](auto point) { each_at<RG_NEAR>(n, A, B, point); }, R);
+        } else if (n > 0) {
+            r = rmsd_of(n, [&](auto point) { each_at<RG_FAR>(n, a + 3 * p0, b + 3 * p0, point); }, R);
+        }
+    } else if (fits) {
+        double A[3 * RG_REG], ca[3], cb[3], X[3][3];
+        const bool large = n > RG_REG;
+        stage_tile(a + 3 * P0, b + 3 * P0, m, lane, at / 3, n, S.l, A, [&] {
+            if (!large) return;
+            auto each = [&](auto point) { each_at<RG_FAR>(n, S.l + at, b + 3 * p0, point); };
+            centroids(n, each, ca, cb);
+            correlate(each, ca, cb, X);
         });
-        if (small) {
-            centroids_reg(n, A, l + 3 * at, ca, cb);
-            correlate_reg(n, A, l + 3 * at, ca, cb, X);
+        auto each = [&](auto point) { each_staged(n, A, S.l + at, point); };
+        if (!large) {
+            centroids(n, each, ca, cb);
+            correlate(each, ca, cb, X);
         }
         if (n > 0) {
             optimal_rotation(X, R);
-            r = small ? residual_reg(n, A, l + 3 * at, ca, cb, R)
-                      : residual_rmsd(n, a + 3 * p0, l + 3 * at, ca, cb, R);
+            r = large ? residual(n, [&](auto point) { each_at<RG_FAR>(n, a + 3 * p0, S.l + at, point); }, ca, cb, R)
+                      : residual(n, each, ca, cb, R);
         }
-    } else {
+    } else if (few_rounds(p0, p1, lane, RG_ROUNDS)) {
         for (int g0 = 0, g1; g0 < RG_SETS; g0 = g1) {
-            const int64_t q0 = tile_round(p0, p1, g0, lane, g1);
+            int64_t q0, q1;
             const double *A = a + 3 * p0, *B = b + 3 * p0;
-            bool now = lane == g0 && n > 0;
-            if (g1 > g0) {
-                const int64_t q1 = round_end(p1, q0, g1);
-                stage_pair(a + 3 * q0, b + 3 * q0, (int)(3 * (q1 - q0)), lane, l, l + 3 * RG_CAP / 2);
-                wave_sync();
-                now = lane >= g0 && lane < g1 && n > 0 && p0 >= q0 && p1 <= q1;
-                A = l + 3 * (int)(p0 - q0);
+            const bool staged = tile_round(p0, p1, g0, lane, g1, q0, q1);
+            bool now = lane >= g0 && lane < g1 && n > 0;
+            if (staged) {
+                stage_both<RG_LOADS / 2>(a + 3 * q0, b + 3 * q0, (int)(3 * (q1 - q0)), lane, S.l,
+                                         S.l + 3 * RG_CAP / 2);
+                now = now && p0 >= q0 && p1 <= q1;
+                A = S.l + 3 * (int)(p0 - q0);
                 B = A + 3 * RG_CAP / 2;
-            } else {
-                g1++;   // larger than the buffer
             }
-            if (now) {
-                centre_and_correlate(n, A, B, ca, cb, X);
-                optimal_rotation(X, R);
-                r = residual_rmsd(n, A, B, ca, cb, R);
-            }
+            if (now) r = rmsd_of(n, [&](auto point) { each_at<RG_FAR>(n, A, B, point); }, R);
             wave_sync();
         }
+    } else {
+        const int most = chunk_table(S.c, p0, n, lane);
+        r = rmsd_of(n, [&](auto point) { each_chunked(a, b, S.c, n, most, lane, point, [](long long) {}); }, R);
+        if (n <= 0) r = 0.0;
     }
     if (s >= n_sets) return;
     rmsd[s] = r;
+    double *rt = rot ? rot + 9 * s : nullptr;
     if (rt)
 #pragma unroll
         for (int q = 0; q < 9; q++) rt[q] = n > 0 ? R[q / 3][q % 3] : (q % 4 == 0) ? 1.0 : 0.0;
 }
 
-__global__ void __launch_bounds__(RG_SETS, 2) k_rmsd_bwd(const double *a, const double *b, const int64_t *off,
-                                                         long long n_sets, long long n_points, const double *rmsd,
-                                                         const double *rot, const double *grad_rmsd, double *grad_a,
-                                                         double *grad_b)
+template <bool MANY>
+__global__ void __launch_bounds__(RG_SETS, MANY ? 2 : 1) k_rmsd_bwd(const double *a, const double *b,
+                                                                   const int64_t *off, long long n_sets,
+                                                                   long long n_points, const double *rmsd,
+                                                                   const double *rot, const double *grad_rmsd,
+                                                                   double *grad_a, double *grad_b)
 {
-    __shared__ double l[3 * RG_CAP];
+    __shared__ RmsdLds<MANY> S;
     const int lane = threadIdx.x;
     const long long s = (long long)blockIdx.x * RG_SETS + lane;
     int64_t P0, P1, p0, p1;
     tile_ranges(off, n_sets, n_points, s, P0, P1, p0, p1);
-    const int n = (int)(p1 - p0);
-    const bool mine = n > 0;   // never past the last set
-    const double *rt = rot ? rot + 9 * s : nullptr;
-    if (P1 - P0 <= RG_CAP && ballot(n > RG_REG) == 0ull) {
-        const int at = (int)(p0 - P0), m = (int)(3 * (P1 - P0));
-        double A[3 * RG_REG];
-        stage_tile(a + 3 * P0, b + 3 * P0, m, lane, at, n, l, A, [] {});
-        if (mine) rmsd_grad_reg(n, A, l + 3 * at, rmsd[s], grad_rmsd[s], rt);
+    const int n = (int)(p1 - p0);   // 0 past the last set
+    const bool fits = P1 - P0 <= RG_CAP;
+    const int at = 3 * (int)(p0 - P0), m = (int)(3 * (P1 - P0));   // where it fits
+    const double r = n > 0 ? rmsd[s] : 0.0, g = n > 0 ? grad_rmsd[s] : 0.0;
+    bool zero = true;
+    double ca[3], cb[3], R[3][3], scale = 0.0;
+    // what gradient() needs; rot: the optimal rotations of the forward pass, or
+    // null to compute them again
+    auto prepare = [&](auto each) {
+        zero = !(r > 0.0) || g == 0.0;
+        scale = g / ((double)n * r);
+        centroids(n, each, ca, cb);
+        if (rot) {
+            if (n > 0)
+#pragma unroll
+                for (int q = 0; q < 9; q++) R[q / 3][q % 3] = rot[9 * s + q];
+        } else {
+            double X[3][3];
+            correlate(each, ca, cb, X);
+            optimal_rotation(X, R);
+        }
+    };
+    auto gradient = [&](double *A, double *B) {
+        if (zero) {
+#pragma unroll
+            for (int d = 0; d < 3; d++) A[d] = B[d] = 0.0;
+        } else {
+            to_gradient(A, B, ca, cb, R, scale);
+        }
+    };
+    const double *Ag = a + 3 * p0, *Bg = b + 3 * p0;
+    if (MANY && fits && ballot(n > RG_REG) == 0ull) {
+        double A[3 * RG_REG], *B = S.l + at;
+        stage_tile(a + 3 * P0, b + 3 * P0, m, lane, at / 3, n, S.l, A, [] {});
+        if (n > 0) {
+            prepare([&](auto point) { each_staged(n, A, B, point); });
+            each_staged(n, A, B, gradient);
+        }
         // b's gradients from LDS, then a's through it
         wave_sync();
         if (grad_b)
-            for (int q = lane; q < m; q += RG_SETS) grad_b[3 * P0 + q] = l[q];
+            for (int q = lane; q < m; q += RG_SETS) grad_b[3 * P0 + q] = S.l[q];
         wave_sync();
         if (!grad_a) return;
-        if (mine)
+        each_staged(n, A, B, [](double *x, double *l) {
 #pragma unroll
-            for (int i = 0; i < RG_REG; i++)
-#pragma unroll
-                for (int d = 0; d < 3; d++)
-                    if (i < n) l[3 * (at + i) + d] = A[3 * i + d];
+            for (int d = 0; d < 3; d++) l[d] = x[d];
+        });
         wave_sync();
-        for (int q = lane; q < m; q += RG_SETS) grad_a[3 * P0 + q] = l[q];
-        return;
-    }
-    for (int g0 = 0, g1; g0 < RG_SETS; g0 = g1) {
-        const int64_t q0 = tile_round(p0, p1, g0, lane, g1);
-        if (g1 == g0) {
-            // larger than the buffer
-            if (lane == g0)
-                rmsd_grad_one(n, a + 3 * p0, b + 3 * p0, rmsd[s], grad_rmsd[s], rt,
-                              grad_a ? grad_a + 3 * p0 : nullptr, grad_b ? grad_b + 3 * p0 : nullptr);
-            g1++;
-            continue;
+        for (int q = lane; q < m; q += RG_SETS) grad_a[3 * P0 + q] = S.l[q];
+    } else if (!MANY && !fits) {
+        if (n > 0) {
+            prepare([&](auto point) { each_at<RG_FAR>(n, Ag, Bg, point); });
+            each_into<RG_FAR>(n, Ag, Bg, grad_a ? grad_a + 3 * p0 : nullptr, grad_b ? grad_b + 3 * p0 : nullptr,
+                              gradient);
         }
-        const int64_t q1 = round_end(p1, q0, g1);
-        const int m = (int)(3 * (q1 - q0));
-        double *la = l, *lb = l + 3 * RG_CAP / 2;
-        stage_pair(a + 3 * q0, b + 3 * q0, m, lane, la, lb);
-        wave_sync();
-        if (lane >= g0 && lane < g1 && mine && p0 >= q0 && p1 <= q1) {
-            // gradients replace the points in LDS
-            const int at = 3 * (int)(p0 - q0);
-            rmsd_grad_one(n, la + at, lb + at, rmsd[s], grad_rmsd[s], rt, la + at, lb + at);
+    } else if (!MANY || few_rounds(p0, p1, lane, RG_ROUNDS)) {
+        // rounds; without MANY one, of the whole tile
+        constexpr int HALF = 3 * RG_CAP / (MANY ? 2 : 1), NEAR = MANY ? RG_FAR : RG_NEAR;
+        for (int g0 = 0, g1 = RG_SETS; g0 < RG_SETS; g0 = g1) {
+            int64_t q0 = P0, q1 = P1;
+            if (MANY && !tile_round(p0, p1, g0, lane, g1, q0, q1)) {
+                if (lane == g0) {   // larger than the buffer
+                    prepare([&](auto point) { each_at<RG_FAR>(n, Ag, Bg, point); });
+                    each_into<RG_FAR>(n, Ag, Bg, grad_a ? grad_a + 3 * p0 : nullptr,
+                                      grad_b ? grad_b + 3 * p0 : nullptr, gradient);
+                }
+                continue;
+            }
+            const int k = (int)(3 * (q1 - q0));
+            stage_both<MANY ? RG_LOADS / 2 : 12>(a + 3 * q0, b + 3 * q0, k, lane, S.l, S.l + HALF);
+            if (lane >= g0 && lane < g1 && n > 0 && p0 >= q0 && p1 <= q1) {
+                // gradients replace the points in LDS
+                double *A = S.l + 3 * (int)(p0 - q0), *B = A + HALF;
+                prepare([&](auto point) { each_at<NEAR>(n, A, B, point); });
+                each_into<NEAR>(n, A, B, A, B, gradient);
+            }
+            wave_sync();
+            for (int q = lane; q < k; q += RG_SETS) {
+                if (grad_a) grad_a[3 * q0 + q] = S.l[q];
+                if (grad_b) grad_b[3 * q0 + q] = S.l[HALF + q];
+            }
+            wave_sync();
         }
-        wave_sync();
-        for (int q = lane; q < m; q += RG_SETS) {
-            if (grad_a) grad_a[3 * q0 + q] = la[q];
-            if (grad_b) grad_b[3 * q0 + q] = lb[q];
-        }
-        wave_sync();
+    } else {
+        const int most = chunk_table(S.c, p0, n, lane);
+        prepare([&](auto point) { each_chunked(a, b, S.c, n, most, lane, point, [](long long) {}); });
+        each_chunked(a, b, S.c, n, most, lane, gradient, [&](long long c) {
+            wave_sync();
+            if (grad_a) chunk_store(S.c, S.c.a, c, lane, grad_a);
+            if (grad_b) chunk_store(S.c, S.c.b, c, lane, grad_b);
+        });
     }
 }
 
