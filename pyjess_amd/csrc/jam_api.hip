@@ -1655,7 +1655,10 @@ void launch_join(jam_context *c, hipStream_t s, const DevMols &dm, const DevTpls
 // of 1,024-thread workgroups, one position per thread -- two of them per CU,
 // so all sets run at once -- and the larger ones beside it on side streams:
 // one of them where the molecule is too small for more than an odd set of
-// that size (KD_ONE_STREAM_ATOMS), three, by size, in larger ones.
+// that size (KD_ONE_STREAM_ATOMS), three, by size, in larger ones. Sets beyond
+// KD_LDS_MAX get a fast and an exact pass in global scratch, as below (without
+// equal coordinates, one set of 40,000 entries: 40 ms against 55 by the exact
+// pass alone).
 //
 // Several molecules: the sets are bucketed by size tier, and every tier gets
 // a stream of its own. Tiers 0 and 1 (<= 128 entries, mostly without ties)
@@ -1728,15 +1731,19 @@ int32_t launch_kd(jam_context *c, const DevMols &dm, const DevTpls &dt, const De
         if (n_atoms > KD_BIG) {
             const bool spread = n_atoms > KD_ONE_STREAM_ATOMS;
             HIP_TRY(fork(5));
-            lds8(c->kd_side[5], nullptr, nullptr);
-            big_exact(c->kd_side[5], nullptr, nullptr);
-            if (spread) HIP_TRY(hipStreamWaitEvent(c->kd_side[4], c->kd_fast[5], 0));
-            lds4(c->kd_side[spread ? 4 : 5], nullptr, nullptr);
-            if (spread) HIP_TRY(hipStreamWaitEvent(c->kd_side[3], c->kd_fast[5], 0));
-            lds2(c->kd_side[spread ? 3 : 5], nullptr, nullptr);
-            HIP_TRY(joined(5));
-            if (spread) HIP_TRY(joined(4));
-            if (spread) HIP_TRY(joined(3));
+            auto side = [&](int k) -> hipStream_t { return c->kd_side[spread ? k : 5]; };
+            for (int k = 3; k < 5 && spread; k++) HIP_TRY(hipStreamWaitEvent(c->kd_side[k], c->kd_fast[5], 0));
+            lds8(side(5), nullptr, nullptr);
+            lds4(side(4), nullptr, nullptr);
+            lds2(side(3), nullptr, nullptr);
+            if (n_atoms > KD_LDS_MAX) {
+                int *lst = tied + 5 * ns;
+                hipLaunchKernelGGL(k_kd_setup, dim3(1), dim3(64), 0, side(5), nt + 5, 1);
+                hipLaunchKernelGGL(jam::k_kdbig, grid(2), dim3(KD_THREADS), 0, side(5), dm, dt, st, scr,
+                                   (const int *)nullptr, (const unsigned int *)nullptr, lst, nt + 5, KD_LDS_MAX);
+                big_exact(side(5), lst, nt + 5);
+            }
+            for (int k = spread ? 3 : 5; k <= 5; k++) HIP_TRY(joined(k));
         }
         hipLaunchKernelGGL((jam::k_kdexact_lds<KD_BIG, 1>), grid(8), dim3(KD_BIG), 0, s, dm, dt, st,
                            (const int *)nullptr, (const unsigned int *)nullptr, 0);

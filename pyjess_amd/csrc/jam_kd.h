@@ -29,7 +29,7 @@
 //          are found by following each push back to the element it started
 //          as. Nearly as fast as the fast path's sorts, so only sets that
 //          seldom have a tie (up to 128 entries of many molecules, and those
-//          too large for LDS) try the fast path first.
+//          too large for LDS unless a sample of them has one) try the fast path first.
 //
 // Fast path: sets of up to 64 entries in one wave's registers, up to KD_BIG
 // with one position per thread, above KD_LDS_MAX in global scratch. Exact
@@ -1291,18 +1291,60 @@ __device__ static void kd_load_global(const DevMols &ms, const DevSets &st, int 
     __syncthreads();
 }
 
-// fast path of the sets of `list` larger than min_n; sets with a split tie
-// go to `tied`
+// Whether the fast path is not worth trying: equal coordinates among (up to)
+// KD_SAMPLE elements of an axis, or a coordinate that is not a number
+// anywhere. The fast path finds a split tie only after its sorts, and has then
+// cost as much as the exact path (9,000 entries on 0.001 A coordinates: 7 ms
+// each); on such coordinates 2,048 of them hold equal ones for sure (21
+// pairs an axis in 100 A, 2 in 1,000 A), on unrounded ones they do not.
+#define KD_SAMPLE 2048
+__device__ static bool kd_repeats(const double *c, size_t stride, int n, unsigned long long *slot, int *flag)
+{
+    constexpr int SLOTS = 2 * KD_SAMPLE;
+    constexpr unsigned long long EMPTY = ~0ull;   // the bits of a NaN
+    const int every = max(n / KD_SAMPLE, 1), sampled = min(n / every, KD_SAMPLE);
+    if (threadIdx.x == 0) flag[0] = 0;
+    for (int a = 0; a < 3; a++) {
+        const double *x = c + a * stride;
+        for (int i = threadIdx.x; i < SLOTS; i += blockDim.x) slot[i] = EMPTY;
+        __syncthreads();
+        bool stop = false;
+        for (int i = threadIdx.x; i < n; i += blockDim.x) stop |= x[i] != x[i];
+        for (int i = threadIdx.x; i < sampled && !stop; i += blockDim.x) {
+            const double v = x[i * every] + 0.0;   // one zero
+            unsigned long long bits;
+            __builtin_memcpy(&bits, &v, sizeof(bits));
+            unsigned int h = (unsigned int)((bits * 0x9E3779B97F4A7C15ull) >> 40);
+            for (int probe = 0; probe < SLOTS; probe++, h++) {
+                const unsigned long long old = atomicCAS(&slot[h % SLOTS], EMPTY, bits);
+                if (old == EMPTY) break;
+                stop |= old == bits;
+                if (stop) break;
+            }
+        }
+        if (stop) flag[0] = 1;
+        __syncthreads();
+        if (flag[0]) break;
+    }
+    const bool found = flag[0] != 0;
+    __syncthreads();
+    return found;
+}
+
+// fast path of the sets of `list` (every set of the query where there is none)
+// larger than min_n; sets with a split tie go to `tied`, and so do those that
+// are likely to have one
 __global__ void __launch_bounds__(KD_THREADS) k_kdbig(DevMols ms, DevTpls tp, DevSets st, unsigned char *scr,
                                                       const int *list, const unsigned int *count, int *tied,
                                                       unsigned int *n_tied, int min_n)
 {
     __shared__ int partial[KD_THREADS];
     __shared__ int flag[2];
+    __shared__ unsigned long long slot[2 * KD_SAMPLE];
     if (*st.total > st.cap) return;
-    const int cnt = (int)*count;
+    const int cnt = list ? (int)*count : st.n_sets;
     for (int q = blockIdx.x; q < cnt; q += gridDim.x) {
-        const int s = list[q];
+        const int s = list ? list[q] : q;
         const int n = st.cnt[s];
         if (n <= min_n) continue;
         const int64_t off = st.off[s];
@@ -1322,7 +1364,8 @@ __global__ void __launch_bounds__(KD_THREADS) k_kdbig(DevMols ms, DevTpls tp, De
         kd_load_global(ms, st, n, off, abase, w.c, (size_t)n2);
         // the arrangement after the work arrays: 61 * n2 + 4 * n <= 128 * n bytes
         int *order = (int *)((unsigned char *)(ib + 9 * n2) + n2);
-        if (!kd_fast<KD_THREADS>(w, n, order, partial, flag)) kd_emit_order<KD_THREADS>(ms, st, s, n, off, abase, order);
+        if (!kd_repeats(w.c, (size_t)n2, n, slot, flag) && !kd_fast<KD_THREADS>(w, n, order, partial, flag))
+            kd_emit_order<KD_THREADS>(ms, st, s, n, off, abase, order);
         else if (threadIdx.x == 0) tied[atomicAdd(n_tied, 1u)] = s;
         __syncthreads();
     }
