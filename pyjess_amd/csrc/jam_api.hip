@@ -198,7 +198,7 @@ struct jam_context {
     void *up_stage = nullptr;
     size_t up_half = 0;
     hipEvent_t up_ev[2] = {};
-    DBuf u_keys, u_starts, u_nnames;
+    DBuf u_keys, u_starts, u_nnames, u_names;
     std::vector<std::unique_ptr<DBuf>> u_scan;
 };
 
@@ -653,19 +653,28 @@ int32_t create_molecules(jam_context *ctx, const jam_molecule_desc *mols, int32_
         atom_off.push_back(atom_off.back() + mols[m].n_atoms);
     }
     const size_t na = (size_t)atom_off.back();
-    // molecules whose serial numbers descend somewhere: all atoms of the batch
-    // in order of serial number, ties in input order
-    std::vector<int> order;
-    for (int m = 0; m < n; m++) {
-        const int N = mols[m].n_atoms;
-        if (ascending(mols[m].serial, N)) continue;
-        if (order.empty()) {
-            order.resize(na);
-            for (int q = 0; q < n; q++) std::iota(order.begin() + atom_off[q], order.begin() + atom_off[q + 1], 0);
-        }
+    // molecules whose serial numbers descend somewhere (five columns of a PDB
+    // text wrap after 99,999 atoms): all atoms of the batch in order of serial
+    // number, ties in input order; on the device where they descend at few
+    // atoms
+    std::vector<int> order, down;
+    std::vector<int> mixed;
+    for (int m = 0; m < n; m++)
+        if (!ascending(mols[m].serial, mols[m].n_atoms)) mixed.push_back(m);
+    for (int m : mixed) {
         const int32_t *sr = mols[m].serial;
-        std::stable_sort(order.begin() + atom_off[m], order.begin() + atom_off[m + 1],
-                         [sr](int a, int b) { return sr[a] < sr[b]; });
+        for (int i = 1; i < mols[m].n_atoms && down.size() <= ING_RUNS; i++)
+            if (sr[i] < sr[i - 1]) down.push_back(atom_off[m] + i);
+    }
+    const bool runs = !down.empty() && down.size() <= ING_RUNS;
+    if (!down.empty() && !runs) {
+        order.resize(na);
+        for (int m = 0; m < n; m++) std::iota(order.begin() + atom_off[m], order.begin() + atom_off[m + 1], 0);
+        for (int m : mixed) {
+            const int32_t *sr = mols[m].serial;
+            std::stable_sort(order.begin() + atom_off[m], order.begin() + atom_off[m + 1],
+                             [sr](int a, int b) { return sr[a] < sr[b]; });
+        }
     }
     HIP_TRY(hipSetDevice(ctx->device));
     std::lock_guard<std::mutex> guard(ctx->up_mutex);
@@ -685,7 +694,9 @@ int32_t create_molecules(jam_context *ctx, const jam_molecule_desc *mols, int32_
     const size_t o_off = place(sizeof(int) * ((size_t)n + 1)), o_xyz = place(sizeof(double) * 3 * na);
     const size_t o_name = place(4 * na), o_resname = place(4 * na), o_resseq = place(sizeof(int) * na);
     const size_t o_chain8 = place(na), o_order = order.empty() ? bytes : place(sizeof(int) * na);
+    const size_t o_serial = runs ? place(sizeof(int) * na) : bytes, o_down = runs ? place(sizeof(int) * ING_RUNS) : bytes;
     const size_t image = bytes;
+    const size_t o_ranks = runs ? place(sizeof(int) * na) : o_order;
     const size_t o_chain = place(sizeof(int) * na), o_perm = place(sizeof(int) * na);
     const size_t o_resoff = place(sizeof(int) * ((size_t)n + 1));
     HIP_TRY(M->block.reserve(bytes));
@@ -697,7 +708,7 @@ int32_t create_molecules(jam_context *ctx, const jam_molecule_desc *mols, int32_
     M->resseq.view(base + o_resseq, sizeof(int) * na);
     M->chain.view(base + o_chain, sizeof(int) * na);
     std::vector<UploadPart> parts;
-    parts.reserve(5 * (size_t)n + 2);
+    parts.reserve(6 * (size_t)n + 3);
     parts.push_back({o_off, atom_off.data(), sizeof(int) * ((size_t)n + 1)});
     auto add = [&](size_t at, size_t width, auto src) {
         for (int m = 0; m < n; m++)
@@ -710,6 +721,10 @@ int32_t create_molecules(jam_context *ctx, const jam_molecule_desc *mols, int32_
     add(o_resseq, sizeof(int), [](const jam_molecule_desc &d) { return (const void *)d.resseq; });
     add(o_chain8, 1, [](const jam_molecule_desc &d) { return (const void *)d.chain2; });
     if (!order.empty()) parts.push_back({o_order, order.data(), sizeof(int) * na});
+    if (runs) {
+        add(o_serial, sizeof(int), [](const jam_molecule_desc &d) { return (const void *)d.serial; });
+        parts.push_back({o_down, down.data(), sizeof(int) * down.size()});
+    }
     int32_t rc = upload_parts(ctx, parts, image, base, s);
     int refused = 0;   // a batch without molecules has nothing to launch
     if (rc == JAM_OK && n > 0) {
@@ -717,8 +732,12 @@ int32_t create_molecules(jam_context *ctx, const jam_molecule_desc *mols, int32_
             hipLaunchKernelGGL(jam::k_chain_words, dim3((unsigned)((na + ING_THREADS - 1) / ING_THREADS)),
                                dim3(ING_THREADS), 0, s, (const signed char *)(base + o_chain8), (long long)na,
                                M->chain.as<int>());
-        rc = residue_index(ctx, M.get(), order.empty() ? nullptr : (const int *)(base + o_order), base + o_perm,
-                           base + o_resoff, s, refused);
+        if (runs)
+            hipLaunchKernelGGL(jam::k_run_order, dim3((unsigned)((na + ING_THREADS - 1) / ING_THREADS)),
+                               dim3(ING_THREADS), 0, s, M->atom_off.as<const int>(), n, (const int *)(base + o_serial),
+                               (const int *)(base + o_down), (int)down.size(), (int *)(base + o_ranks));
+        rc = residue_index(ctx, M.get(), order.empty() && !runs ? nullptr : (const int *)(base + o_ranks),
+                           base + o_perm, base + o_resoff, s, refused);
     }
     if (rc == JAM_OK && refused >= 0) rc = host_residue_index(mols, n, M.get(), s);
     // the pinned halves are free again, and so is the memory of a batch that
@@ -1076,13 +1095,20 @@ int32_t residue_index(jam_context *c, jam_molecules *M, const int *order, void *
     HIP_TRY(c->u_starts.reserve(sizeof(int) * na));
     HIP_TRY(c->u_nnames.reserve(sizeof(int) * (size_t)n));
     const int *aoff = M->atom_off.as<const int>();
+    const uint32_t *visited = M->resname.as<const uint32_t>();
+    if (order && M->n_atoms > 0) {
+        HIP_TRY(c->u_names.reserve(sizeof(uint32_t) * na));
+        hipLaunchKernelGGL(jam::k_visited_names, dim3((unsigned)((na + ING_THREADS - 1) / ING_THREADS)),
+                           dim3(ING_THREADS), 0, s, aoff, n, visited, order, c->u_names.as<uint32_t>());
+        visited = c->u_names.as<const uint32_t>();
+    }
     std::vector<int> names((size_t)n);
     int64_t total = 0;
     refused = -1;
     for (int big = 0; big < 2; big++) {
         auto *index = big ? jam::k_residue_index<ING_MAX_NAMES> : jam::k_residue_index<IDX_MAX_NAMES>;
-        hipLaunchKernelGGL(index, dim3((unsigned)n), dim3(IDX_THREADS), 0, s, aoff, M->resname.as<const uint32_t>(), order,
-                           M->perm.as<int>(), c->u_keys.as<uint32_t>(), c->u_starts.as<int>(), c->u_nnames.as<int>());
+        hipLaunchKernelGGL(index, dim3((unsigned)n), dim3(IDX_THREADS), 0, s, aoff, M->resname.as<const uint32_t>(),
+                           visited, order, M->perm.as<int>(), c->u_keys.as<uint32_t>(), c->u_starts.as<int>(), c->u_nnames.as<int>());
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipMemcpyAsync(names.data(), c->u_nnames.ptr, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost, s));
         const int32_t rc = device_scan<int, int>(c->u_nnames.as<const int>(), n, M->res_off.as<int>(), c->u_scan, 0, s);
@@ -1272,8 +1298,8 @@ extern "C" int32_t jam_molecules_parse_pdb(jam_context *c, const char *const *te
     hipLaunchKernelGGL(jam::k_ing_narrow, dim3((unsigned)((n + 1 + 255) / 256)), dim3(256), 0, s,
                        (const long long *)text_atom, n + 1, M->atom_off.as<int>());
     HIP_TRY(c->g_err.reserve(sizeof(unsigned int) * na));
-    HIP_TRY(c->g_firsterr.reserve(2 * sizeof(unsigned long long)));
-    // first atom in error; whether serial numbers descend
+    HIP_TRY(c->g_firsterr.reserve(2 * sizeof(unsigned long long) + sizeof(int) * ING_RUNS));
+    // first atom in error; atoms at which serial numbers descend, and the first of them
     unsigned long long *state = c->g_firsterr.as<unsigned long long>();
     hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, state, 1ll, (unsigned long long)n_atoms);
     hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, state + 1, 1ll, 0ull);
@@ -1299,7 +1325,8 @@ extern "C" int32_t jam_molecules_parse_pdb(jam_context *c, const char *const *te
         hipLaunchKernelGGL(jam::k_ing_parse, dim3(ablocks), dim3(ING_THREADS), 0, s, tx, c->g_starts.as<const long long>(),
                            n_lines, c->g_atomline.as<const long long>(), n_atoms, at);
         hipLaunchKernelGGL(jam::k_ing_descends, dim3(ablocks), dim3(ING_THREADS), 0, s, n_atoms, M->serial.as<const int>(),
-                           c->g_atomline.as<const long long>(), c->g_textof.as<const int>(), state + 1);
+                           c->g_atomline.as<const long long>(), c->g_textof.as<const int>(), state + 1,
+                           (int *)(state + 2));
     }
     HIP_TRY(hipGetLastError());
     unsigned long long h_state[2] = {0, 0};
@@ -1322,8 +1349,14 @@ extern "C" int32_t jam_molecules_parse_pdb(jam_context *c, const char *const *te
     // ---- residue-name index
     guard.lock();
     const int *order = nullptr;
-    if (h_state[1] != 0) {
-        // serial numbers that descend: the atoms of each text in their order
+    // serial numbers that descend: the atoms of each text in their order
+    if (h_state[1] > 0 && h_state[1] <= ING_RUNS) {
+        HIP_TRY(c->g_sval.reserve(sizeof(int) * na));
+        hipLaunchKernelGGL(jam::k_run_order, dim3(ablocks), dim3(ING_THREADS), 0, s, M->atom_off.as<const int>(), n,
+                           M->serial.as<const int>(), (const int *)(state + 2), (int)h_state[1], c->g_sval.as<int>());
+        HIP_TRY(hipGetLastError());
+        order = c->g_sval.as<const int>();
+    } else if (h_state[1] > 0) {
         HIP_TRY(c->g_skey.reserve(sizeof(unsigned long long) * 2 * na));
         HIP_TRY(c->g_sval.reserve(sizeof(int) * 2 * na));
         unsigned long long *k0 = c->g_skey.as<unsigned long long>(), *k1 = k0 + na;

@@ -19,8 +19,8 @@
 //   k_ing_parse                 thread per atom record: the fixed columns
 //   k_residue_index             the residue-name index: workgroup per molecule,
 //                               a stable counting sort by name (of atoms
-//                               sorted by serial number before, where those
-//                               descend)
+//                               ordered by serial number before, where those
+//                               descend: k_run_order, or radix passes)
 // Numbers are parsed exactly: a decimal field of at most 19 significant
 // digits and a power of ten up to 22 is one correctly rounded division or
 // multiplication of two exact doubles (Clinger's fast path), which is what
@@ -52,6 +52,10 @@ namespace jam {
 // ING_HEADERS of them (in any order) line and offset
 #define ING_HEADERS 256
 #define ING_INFO_WORDS (2 + 2 * ING_HEADERS)
+
+// most atoms at which serial numbers descend for k_run_order
+#define ING_RUNS 64
+#define RUN_CHAINS 4   // bisections side by side
 
 // parse errors (bit flags of the per-atom error word)
 #define ING_EBADFIELD 1     // a numeric field does not parse
@@ -426,15 +430,92 @@ __global__ void __launch_bounds__(ING_THREADS) k_ing_parse(IngText tx, const lon
 // residue-name index
 // ---------------------------------------------------------------------------
 
-// *down != 0 where an atom's serial number is below that of the atom before it
-// in its text.
+// Atoms whose serial number is below that of the atom before them in their
+// text: their number to *n_down, the first ING_RUNS of them (in any order) to
+// down.
 __global__ void __launch_bounds__(ING_THREADS) k_ing_descends(long long n_atoms, const int *serial,
                                                              const long long *atom_line, const int *text_of,
-                                                             unsigned long long *down)
+                                                             unsigned long long *n_down, int *down)
 {
     const long long a = (long long)blockIdx.x * ING_THREADS + threadIdx.x;
     const bool d = a > 0 && a < n_atoms && serial[a] < serial[a - 1] && text_of[atom_line[a]] == text_of[atom_line[a - 1]];
-    if (ballot(d) != 0ull && lane_id() == 0) atomicOr(down, 1ull);
+    const unsigned long long m = ballot(d);
+    if (m == 0ull) return;
+    unsigned long long k = 0;
+    if (lane_id() == 0) k = atomicAdd(n_down, (unsigned long long)__popcll(m));
+    k = __shfl(k, 0, JAM_WAVE) + rank_below(m);
+    if (d && k < ING_RUNS) down[k] = (int)a;
+}
+
+// the molecule that atom a of the batch belongs to: the last that starts at or before it
+__device__ static inline int molecule_of(const int *atom_off, int n_mols, long long a)
+{
+    int lo = 0, hi = n_mols;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (atom_off[mid] <= a) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Molecule-local indices of every molecule's atoms by serial number, ties in
+// input order, at its positions in order, where the serial numbers descend at the few
+// atoms `down` (in any order): an atom's place is the number of atoms before it in
+// each ascending run, by bisection (RUN_CHAINS runs at once). Bound by the chains
+// of a bisection (17 loads for 100,000 atoms), which the other waves hide. With
+// k_visited_names: a text of 100,000 atoms that wraps once 1.08 (radix passes) -> 0.89
+// ms, of 2 M atoms in 21 runs 12.2 -> 11.0 ms; upload of 400,000 atoms in 5 runs
+// 12.6 (sorted on the host) -> 2.1 ms.
+__global__ void __launch_bounds__(ING_THREADS) k_run_order(const int *atom_off, int n_mols, const int *serial,
+                                                          const int *down, int n_down, int *order)
+{
+    __shared__ int first[ING_RUNS];
+    const int t = threadIdx.x;
+    if (t < n_down) {
+        const int v = down[t];
+        int k = 0;
+        for (int q = 0; q < n_down; q++) k += down[q] < v;
+        first[k] = v;
+    }
+    __syncthreads();
+    const long long a = (long long)blockIdx.x * ING_THREADS + t;
+    if (a >= atom_off[n_mols]) return;
+    const int m = molecule_of(atom_off, n_mols, a);
+    const int a0 = atom_off[m], a1 = atom_off[m + 1], s = serial[a];
+    // run r of the molecule: [first[k0 + r - 1], first[k0 + r]), a0 and a1 at its ends
+    int k0 = 0, k1;
+    while (k0 < n_down && first[k0] <= a0) k0++;
+    for (k1 = k0; k1 < n_down && first[k1] < a1;) k1++;
+    int at = a0;
+    for (int r0 = k0; r0 <= k1; r0 += RUN_CHAINS) {
+        int x[RUN_CHAINS], y[RUN_CHAINS];
+        bool upto[RUN_CHAINS];   // an earlier run counts up to s, a later one below s
+#pragma unroll
+        for (int u = 0; u < RUN_CHAINS; u++) {
+            const int r = r0 + u;
+            const int begin = r == k0 ? a0 : r <= k1 ? first[r - 1] : a1, end = r < k1 ? first[r] : a1;
+            upto[u] = begin <= a;
+            x[u] = begin;
+            y[u] = end;
+            at -= begin;
+            if (a >= begin && a < end) x[u] = y[u] = (int)a;
+        }
+        for (bool more = true; more;) {
+            more = false;
+#pragma unroll
+            for (int u = 0; u < RUN_CHAINS; u++) {
+                if (x[u] >= y[u]) continue;
+                const int mid = (x[u] + y[u]) >> 1, v = serial[mid];
+                if (upto[u] ? v <= s : v < s) x[u] = mid + 1;
+                else y[u] = mid;
+                more = true;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < RUN_CHAINS; u++) at += x[u];
+    }
+    order[at] = (int)a - a0;
 }
 
 // Sort key of every atom: its text, then its serial number, which a stable
@@ -468,6 +549,17 @@ __global__ void k_ing_narrow(const long long *in, int n, int *out)
     if (k < n) out[k] = (int)in[k];
 }
 
+// The residue names of every molecule's atoms in the order in which
+// k_residue_index visits them: gathered by the whole device, as one molecule's
+// workgroup alone takes 1.4 ms more for 2 M atoms of 21 interleaved runs.
+__global__ void __launch_bounds__(ING_THREADS) k_visited_names(const int *atom_off, int n_mols, const uint32_t *resname,
+                                                              const int *order, uint32_t *visited)
+{
+    const long long i = (long long)blockIdx.x * ING_THREADS + threadIdx.x;
+    if (i >= atom_off[n_mols]) return;
+    visited[i] = resname[atom_off[molecule_of(atom_off, n_mols, i)] + order[i]];
+}
+
 // The residue-name index of a batch in one launch (ResIndex_create,
 // patches/ResIndex.c.patch:34-119): a workgroup per molecule. The molecule's
 // distinct upper-cased names go through an LDS hash set and a bitonic sort
@@ -478,7 +570,8 @@ __global__ void k_ing_narrow(const long long *in, int n, int *out)
 // name comes from one ballot per bit of the name's number, so the counting
 // sort is stable and its second walk needs no workgroup barrier.
 // `order`, where given, is the order in which a molecule's atoms are visited
-// (its molecule-local indices by serial number, ties in input order); without
+// (its molecule-local indices by serial number, ties in input order), and
+// `visited` their names in that order (else resname); without
 // it they are visited as they come, which is the same thing for serial numbers
 // that never descend. Either way atoms end up by (name, serial, input order).
 //
@@ -500,7 +593,7 @@ __global__ void k_ing_narrow(const long long *in, int n, int *out)
 
 template <int MAXN>
 __global__ void __launch_bounds__(IDX_THREADS) k_residue_index(const int *atom_off, const uint32_t *resname,
-                                                               const int *order, int *perm, uint32_t *keys,
+                                                               const uint32_t *visited, const int *order, int *perm, uint32_t *keys,
                                                                int *starts, int *n_names)
 {
     constexpr int SLOTS = 2 * MAXN;   // open addressing at half load at most
@@ -575,7 +668,7 @@ __global__ void __launch_bounds__(IDX_THREADS) k_residue_index(const int *atom_o
     // the i-th visited atom (molecule-local) and the number of its name
     auto visit = [&](int i, int &atom, int &b) {
         atom = order ? order[a0 + i] : i;
-        const uint32_t key = jam_upper4(resname[a0 + atom]);
+        const uint32_t key = jam_upper4(visited[a0 + i]);
         int lo = 0, hi = n - 1;   // the last name <= key is key itself
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
