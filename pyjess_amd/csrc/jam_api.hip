@@ -142,16 +142,11 @@ struct jam_context {
     int64_t front_cap = 0, done_cap = 0;
     int front_stride = 0, done_stride = 0;
     int join_grid[8] = {};          // resident workgroups of the join kernel's variants
-    int kd_grid[13] = {};           // resident workgroups of the kd kernels
-    // the exact kd pass of each size tier runs on a stream of its own, from
-    // the moment the tier's fast pass has listed its tied sets, beside the
-    // fast passes of the other tiers (all streams at the default priority)
-    hipStream_t kd_side[KD_TIERS] = {};
-    hipEvent_t kd_fast[KD_TIERS] = {}, kd_joined[KD_TIERS] = {};
-    // the largest tier's sets of up to 8 * KD_LDS_SMALL_THREADS entries run
-    // on a stream of their own, beside its larger sets
-    hipStream_t kd_lds = nullptr;
-    hipEvent_t kd_lds_done = nullptr;
+    int kd_grid[KD_GRIDS] = {};   // resident workgroups of the kd kernels
+    // side streams of the kd passes (kd_launches), beside the main stream (all
+    // streams at the default priority)
+    hipStream_t kd_side[KD_SIDES] = {};
+    hipEvent_t kd_fast[KD_SIDES] = {}, kd_joined[KD_SIDES] = {};
     bool kd_pending = false;    // side-stream work of the last kd launch may still run
     unsigned kd_used = 0;       // bit k: the last kd launch uses side stream k
     // sort of the complete matches
@@ -363,13 +358,11 @@ extern "C" int32_t jam_context_create(int32_t device, jam_context **out)
     HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     for (auto &ev : c->ev) HIP_TRY(hipEventCreate(&ev));
     for (auto &ev : c->xev) HIP_TRY(hipEventCreate(&ev));
-    for (int k = 0; k < KD_TIERS; k++) {
+    for (int k = 0; k < KD_SIDES; k++) {
         HIP_TRY(hipStreamCreateWithFlags(&c->kd_side[k], hipStreamNonBlocking));
         HIP_TRY(hipEventCreateWithFlags(&c->kd_fast[k], hipEventDisableTiming));
         HIP_TRY(hipEventCreateWithFlags(&c->kd_joined[k], hipEventDisableTiming));
     }
-    HIP_TRY(hipStreamCreateWithFlags(&c->kd_lds, hipStreamNonBlocking));
-    HIP_TRY(hipEventCreateWithFlags(&c->kd_lds_done, hipEventDisableTiming));
     *out = c.release();
     return JAM_OK;
 }
@@ -398,15 +391,12 @@ extern "C" void jam_context_free(jam_context *ctx)
         if (ev) (void)hipEventDestroy(ev);
     for (auto &ev : ctx->stage_ev)
         if (ev) (void)hipEventDestroy(ev);
-    for (int k = 0; k < KD_TIERS; k++) {
+    for (int k = 0; k < KD_SIDES; k++) {
         if (ctx->kd_side[k]) (void)hipStreamSynchronize(ctx->kd_side[k]);
         if (ctx->kd_fast[k]) (void)hipEventDestroy(ctx->kd_fast[k]);
         if (ctx->kd_joined[k]) (void)hipEventDestroy(ctx->kd_joined[k]);
         if (ctx->kd_side[k]) (void)hipStreamDestroy(ctx->kd_side[k]);
     }
-    if (ctx->kd_lds) (void)hipStreamSynchronize(ctx->kd_lds);
-    if (ctx->kd_lds_done) (void)hipEventDestroy(ctx->kd_lds_done);
-    if (ctx->kd_lds) (void)hipStreamDestroy(ctx->kd_lds);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -1518,7 +1508,7 @@ int32_t grow_sets(jam_context *c, int64_t cap, int n_sets)
 void drain_kd(jam_context *c)
 {
     if (!c->kd_pending) return;
-    for (int k = 0; k < KD_TIERS; k++) (void)hipStreamSynchronize(c->kd_side[k]);
+    for (int k = 0; k < KD_SIDES; k++) (void)hipStreamSynchronize(c->kd_side[k]);
     c->kd_pending = false;
 }
 
@@ -1604,12 +1594,6 @@ int32_t grow_events(jam_context *c, int64_t cap, int stride)
     return JAM_OK;
 }
 
-// clears the kd passes' per-tier counts
-__global__ void k_kd_setup(unsigned int *counts, int n)
-{
-    if ((int)threadIdx.x < n) counts[threadIdx.x] = 0u;
-}
-
 __global__ void k_zero_u64(unsigned long long *v, long long n)
 {
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
@@ -1677,164 +1661,62 @@ void launch_join(jam_context *c, hipStream_t s, const DevMols &dm, const DevTpls
 }
 
 
-// Launches the kd passes over the candidate sets of `st`. Sets of up to
-// KD_LDS_MAX entries are mostly left to the exact QuickSelect pass alone: on
-// 0.001 A coordinates a set of a few hundred entries often has equal values at
-// one of its n-1 split points, and the exact pass costs no more than the sorts
-// of the fast pass (2,000 sets of 800 entries: 0.35 ms against 0.46 ms).
-//
-// One molecule (a few hundred sets, bound by the latency of the longest chain
-// of rounds and by launches): every set of up to KD_BIG entries in one launch
-// of 1,024-thread workgroups, one position per thread -- two of them per CU,
-// so all sets run at once -- and the larger ones beside it on side streams:
-// one of them where the molecule is too small for more than an odd set of
-// that size (KD_ONE_STREAM_ATOMS), three, by size, in larger ones. Sets beyond
-// KD_LDS_MAX get a fast and an exact pass in global scratch, as below (without
-// equal coordinates, one set of 40,000 entries: 40 ms against 55 by the exact
-// pass alone).
-//
-// Several molecules: the sets are bucketed by size tier, and every tier gets
-// a stream of its own. Tiers 0 and 1 (<= 128 entries, mostly without ties)
-// get a fast pass on `s` and the exact pass over the sets that it lists;
-// tiers 2-4 the exact pass alone, two positions per thread above 256 entries
-// (throughput: 0.35 ms for 2,000 sets of 800 entries against 0.51 ms with one
-// position per thread, which is the faster form for a single set); tier 5 the
-// exact pass in LDS up to KD_LDS_MAX entries, and above that a fast and an
-// exact pass in global scratch.
-//
-// The passes of tier k end before kd_joined[k]; every set is written once
-// all are. Grids are upper bounds (the counts stay on the device); every
-// kernel loops over its own list. The caller has cleared *st.kd_err.
-constexpr int64_t KD_ONE_STREAM_ATOMS = 16384;
+// Where kd_launches puts its kernels: side stream k is kd_side[k], KD_MAIN `s`.
+struct KdQueue {
+    jam_context *c;
+    hipStream_t s;
+    int n_sets;
+    hipError_t error = hipSuccess;
+
+    void check(hipError_t e)
+    {
+        if (error == hipSuccess) error = e;
+    }
+    // at most as many workgroups as there are sets and as stay resident
+    template <class... K, class... A>
+    void run(int k, int slot, void (*kernel)(K...), int threads, A... args)
+    {
+        if (c->kd_grid[slot] == 0) c->kd_grid[slot] = resident_grid(kernel, threads, c->device);
+        run_grid(k, std::min(n_sets, c->kd_grid[slot]), kernel, threads, args...);
+    }
+    template <class... K, class... A>
+    void run_grid(int k, int blocks, void (*kernel)(K...), int threads, A... args)
+    {
+        if (error != hipSuccess) return;   // nothing runs out of order
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3((unsigned)threads), 0, k == KD_MAIN ? s : c->kd_side[k],
+                           args...);
+        check(hipGetLastError());
+    }
+    void fork(int k, int from)
+    {
+        if (k == from) check(hipEventRecord(c->kd_fast[k], s));
+        check(hipStreamWaitEvent(c->kd_side[k], c->kd_fast[from], 0));
+    }
+    void joined(int k)
+    {
+        c->kd_used |= 1u << k;
+        check(hipEventRecord(c->kd_joined[k], c->kd_side[k]));
+    }
+};
+
+// Launches the kd passes over the candidate sets of `st` (kd_launches); the
+// caller has cleared *st.kd_err.
 int32_t launch_kd(jam_context *c, const DevMols &dm, const DevTpls &dt, const DevSets &st, hipStream_t s,
                   bool one_molecule, int64_t n_atoms)
 {
-    const int n_sets = st.n_sets;
-    unsigned char *scr = c->kscr.as<unsigned char>();
-    int *bucket = c->kd_bucket.as<int>();
-    int *tied = c->kd_tied.as<int>();
-    unsigned int *nb = c->kd_count.as<unsigned int>();
-    unsigned int *nt = nb + KD_TIERS;
-    const size_t ns = (size_t)n_sets;
-    if (c->kd_grid[0] == 0) {
-        const int d = c->device;
-        c->kd_grid[0] = resident_grid(jam::k_kdwave, JAM_WAVE, d);
-        c->kd_grid[1] = resident_grid(jam::k_kdblock<128>, 128, d);
-        c->kd_grid[2] = resident_grid(jam::k_kdbig, KD_THREADS, d);
-        c->kd_grid[3] = resident_grid(jam::k_kdexact<64>, 64, d);
-        c->kd_grid[4] = resident_grid(jam::k_kdexact<128>, 128, d);
-        c->kd_grid[5] = resident_grid(jam::k_kdexact<256>, 256, d);
-        c->kd_grid[6] = resident_grid(jam::k_kdexact_lds<256, 2>, 256, d);
-        c->kd_grid[7] = resident_grid(jam::k_kdexact_lds<512, 2>, 512, d);
-        c->kd_grid[8] = resident_grid(jam::k_kdexact_lds<KD_BIG, 1>, KD_BIG, d);
-        c->kd_grid[9] = resident_grid(jam::k_kdexact_lds<1024, 2>, 1024, d);
-        c->kd_grid[10] = resident_grid(jam::k_kdexact_lds<1024, 4>, 1024, d);
-        c->kd_grid[11] = resident_grid(jam::k_kdexact_lds<KD_LDS_MAX / 8, 8>, KD_LDS_MAX / 8, d);
-        c->kd_grid[12] = resident_grid(jam::k_kdbig_exact, KD_EXACT_THREADS, d);
-    }
-    auto grid = [&](int k) { return dim3((unsigned)std::min(n_sets, c->kd_grid[k])); };
-    // the LDS exact passes of tier 5 over `lst` (every set where there is none)
-    auto lds2 = [&](hipStream_t x, const int *lst, const unsigned int *lc) {
-        hipLaunchKernelGGL((jam::k_kdexact_lds<1024, 2>), grid(9), dim3(1024), 0, x, dm, dt, st, lst, lc, KD_BIG);
-    };
-    auto lds4 = [&](hipStream_t x, const int *lst, const unsigned int *lc) {
-        hipLaunchKernelGGL((jam::k_kdexact_lds<1024, 4>), grid(10), dim3(1024), 0, x, dm, dt, st, lst, lc,
-                           KD_LDS_MAX / 4);
-    };
-    auto lds8 = [&](hipStream_t x, const int *lst, const unsigned int *lc) {
-        hipLaunchKernelGGL((jam::k_kdexact_lds<KD_LDS_MAX / 8, 8>), grid(11), dim3(KD_LDS_MAX / 8), 0, x, dm, dt, st,
-                           lst, lc, KD_LDS_MAX / 2);
-    };
-    auto big_exact = [&](hipStream_t x, const int *lst, const unsigned int *lc) {
-        hipLaunchKernelGGL(jam::k_kdbig_exact, grid(12), dim3(KD_EXACT_THREADS), 0, x, dm, dt, st, scr, lst, lc,
-                           KD_LDS_MAX);
-    };
     c->kd_pending = true;
     c->kd_used = 0u;
-    // side stream k starts from here on `s`, and is waited for by kd_join
-    auto fork = [&](int k) -> hipError_t {
-        hipError_t e = hipEventRecord(c->kd_fast[k], s);
-        return e == hipSuccess ? hipStreamWaitEvent(c->kd_side[k], c->kd_fast[k], 0) : e;
-    };
-    auto joined = [&](int k) -> hipError_t {
-        c->kd_used |= 1u << k;
-        return hipEventRecord(c->kd_joined[k], c->kd_side[k]);
-    };
-    if (one_molecule) {
-        if (n_atoms > KD_BIG) {
-            const bool spread = n_atoms > KD_ONE_STREAM_ATOMS;
-            HIP_TRY(fork(5));
-            auto side = [&](int k) -> hipStream_t { return c->kd_side[spread ? k : 5]; };
-            for (int k = 3; k < 5 && spread; k++) HIP_TRY(hipStreamWaitEvent(c->kd_side[k], c->kd_fast[5], 0));
-            lds8(side(5), nullptr, nullptr);
-            lds4(side(4), nullptr, nullptr);
-            lds2(side(3), nullptr, nullptr);
-            if (n_atoms > KD_LDS_MAX) {
-                int *lst = tied + 5 * ns;
-                hipLaunchKernelGGL(k_kd_setup, dim3(1), dim3(64), 0, side(5), nt + 5, 1);
-                hipLaunchKernelGGL(jam::k_kdbig, grid(2), dim3(KD_THREADS), 0, side(5), dm, dt, st, scr,
-                                   (const int *)nullptr, (const unsigned int *)nullptr, lst, nt + 5, KD_LDS_MAX);
-                big_exact(side(5), lst, nt + 5);
-            }
-            for (int k = spread ? 3 : 5; k <= 5; k++) HIP_TRY(joined(k));
-        }
-        hipLaunchKernelGGL((jam::k_kdexact_lds<KD_BIG, 1>), grid(8), dim3(KD_BIG), 0, s, dm, dt, st,
-                           (const int *)nullptr, (const unsigned int *)nullptr, 0);
-        HIP_TRY(hipGetLastError());
-        return JAM_OK;
-    }
-    hipLaunchKernelGGL(k_kd_setup, dim3(1), dim3(64), 0, s, nb, 2 * KD_TIERS);
-    hipLaunchKernelGGL(jam::k_kdbucket,
-                       dim3(std::max(1, std::min((n_sets + KD_BUCKET_SPAN - 1) / KD_BUCKET_SPAN, 1024))), dim3(256),
-                       0, s, st, bucket, nb);
-    HIP_TRY(hipGetLastError());
-    // largest tier first: its exact passes, the longest, start earliest
-    for (int k = KD_TIERS - 1; k >= 0; k--) {
-        const int *all = bucket + (size_t)k * ns;
-        int *lst = tied + (size_t)k * ns;
-        const unsigned int *na = nb + k;
-        unsigned int *nl = nt + k;
-        hipStream_t x = c->kd_side[k];
-        if (k == 5) {
-            // the smallest of the tier on kd_lds, beside the larger ones
-            hipLaunchKernelGGL(jam::k_kdbig, grid(2), dim3(KD_THREADS), 0, s, dm, dt, st, scr, all, na, lst, nl,
-                               KD_LDS_MAX);
-            HIP_TRY(fork(k));
-            HIP_TRY(hipStreamWaitEvent(c->kd_lds, c->kd_fast[k], 0));
-            lds2(c->kd_lds, all, na);
-            HIP_TRY(hipEventRecord(c->kd_lds_done, c->kd_lds));
-            lds8(x, all, na);
-            lds4(x, all, na);
-            big_exact(x, lst, nl);
-            HIP_TRY(hipStreamWaitEvent(x, c->kd_lds_done, 0));
-        } else if (k == 4) {
-            HIP_TRY(fork(k));
-            hipLaunchKernelGGL((jam::k_kdexact_lds<512, 2>), grid(7), dim3(512), 0, x, dm, dt, st, all, na, 0);
-        } else if (k == 3) {
-            HIP_TRY(fork(k));
-            hipLaunchKernelGGL((jam::k_kdexact_lds<256, 2>), grid(6), dim3(256), 0, x, dm, dt, st, all, na, 0);
-        } else if (k == 2) {
-            HIP_TRY(fork(k));
-            hipLaunchKernelGGL((jam::k_kdexact<256>), grid(5), dim3(256), 0, x, dm, dt, st, all, na);
-        } else if (k == 1) {
-            hipLaunchKernelGGL((jam::k_kdblock<128>), grid(1), dim3(128), 0, s, dm, dt, st, all, na, lst, nl);
-            HIP_TRY(fork(k));
-            hipLaunchKernelGGL((jam::k_kdexact<128>), grid(4), dim3(128), 0, x, dm, dt, st, lst, nl);
-        } else {
-            hipLaunchKernelGGL(jam::k_kdwave, grid(0), dim3(JAM_WAVE), 0, s, dm, dt, st, all, na, lst, nl);
-            HIP_TRY(fork(k));
-            hipLaunchKernelGGL((jam::k_kdexact<64>), grid(3), dim3(64), 0, x, dm, dt, st, lst, nl);
-        }
-        HIP_TRY(joined(k));
-    }
-    HIP_TRY(hipGetLastError());
+    KdQueue q{c, s, st.n_sets};
+    jam::kd_launches(q, dm, dt, st, c->kscr.as<unsigned char>(), c->kd_bucket.as<int>(), c->kd_tied.as<int>(),
+                     c->kd_count.as<unsigned int>(), one_molecule, n_atoms);
+    HIP_TRY(q.error);
     return JAM_OK;
 }
 
 // `s` waits for the side streams of the last launch_kd
 hipError_t kd_join(jam_context *c, hipStream_t s)
 {
-    for (int k = 0; k < KD_TIERS; k++) {
+    for (int k = 0; k < KD_SIDES; k++) {
         if (!((c->kd_used >> k) & 1u)) continue;
         const hipError_t e = hipStreamWaitEvent(s, c->kd_joined[k], 0);
         if (e != hipSuccess) return e;
@@ -2623,7 +2505,7 @@ extern "C" int32_t jam_kd_order(jam_context *c, const double *xyz, const int64_t
     st.total = (int64_t *)(cnts + CNT_TOTAL);
     st.maxcnt = (int *)(cnts + CNT_MAXCNT);
     st.kd_err = c->kd_count.as<unsigned int>() + 2 * KD_TIERS;
-    hipLaunchKernelGGL(k_kd_setup, dim3(1), dim3(64), 0, s, st.kd_err, 1);
+    hipLaunchKernelGGL(jam::k_kd_setup, dim3(1), dim3(64), 0, s, st.kd_err, 1);
     if ((rc = launch_kd(c, dm, dt, st, s, n_sets == 1, total)) != JAM_OK) {
         drain_kd(c);
         return rc;

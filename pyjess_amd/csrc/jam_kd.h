@@ -623,11 +623,9 @@ __device__ static inline int kd_wave_tree(int n, int d, double c0, double c1, do
     return id;
 }
 
-// largest set of the LDS exact pass (1,024 threads); larger ones run in
-// global scratch. Sets up to 8 * KD_LDS_SMALL_THREADS entries run with fewer
-// threads and half the LDS, three workgroups per CU.
+// largest set of the LDS exact pass (1,024 threads, eight positions each);
+// larger ones run in global scratch
 #define KD_LDS_MAX 8192
-#define KD_LDS_SMALL_THREADS 512
 
 template <int NT, int P>
 struct KdExactLds {
@@ -926,7 +924,7 @@ __global__ void __launch_bounds__(NT, 4) k_kdexact_lds(DevMols ms, DevTpls tp, D
 }
 
 // ---------------------------------------------------------------------------
-// sets larger than KD_BIG: both paths on work arrays in global scratch
+// sets larger than KD_LDS_MAX: both paths on work arrays in global scratch
 // (scr + off * KD_SCRATCH_BYTES_PER_ENTRY), KD_THREADS threads looping over
 // the positions
 // ---------------------------------------------------------------------------
@@ -1408,6 +1406,143 @@ __global__ void __launch_bounds__(KD_EXACT_THREADS) k_kdbig_exact(DevMols ms, De
         else if (threadIdx.x == 0)
             atomicOr(st.kd_err, 1u);
         __syncthreads();
+    }
+}
+
+// ---------------------------------------------------------------------------
+// launches
+// ---------------------------------------------------------------------------
+
+// clears the kd passes' per-tier counts
+__global__ void __launch_bounds__(64) k_kd_setup(unsigned int *counts, int n)
+{
+    if ((int)threadIdx.x < n) counts[threadIdx.x] = 0u;
+}
+
+// The kd passes over the candidate sets of `st`. Sets of up to
+// KD_LDS_MAX entries are mostly left to the exact QuickSelect pass alone: on
+// 0.001 A coordinates a set of a few hundred entries often has equal values at
+// one of its n-1 split points, and the exact pass costs no more than the sorts
+// of the fast pass (2,000 sets of 800 entries: 0.35 ms against 0.46 ms).
+//
+// One molecule (a few hundred sets, bound by the latency of the longest chain
+// of rounds and by launches): every set of up to KD_BIG entries in one launch
+// of 1,024-thread workgroups, one position per thread -- two of them per CU,
+// so all sets run at once -- and the larger ones beside it on side streams:
+// one of them where the molecule is too small for more than an odd set of
+// that size (KD_ONE_STREAM_ATOMS), three, by size, in larger ones. Sets beyond
+// KD_LDS_MAX get a fast and an exact pass in global scratch, as below (without
+// equal coordinates, one set of 40,000 entries: 40 ms against 55 by the exact
+// pass alone).
+//
+// Several molecules: the sets are bucketed by size tier, and every tier gets
+// a stream of its own. Tiers 0 and 1 (<= 128 entries, mostly without ties)
+// get a fast pass on the main stream and the exact pass over the sets that it lists;
+// tiers 2-4 the exact pass alone, two positions per thread above 256 entries
+// (throughput: 0.35 ms for 2,000 sets of 800 entries against 0.51 ms with one
+// position per thread, which is the faster form for a single set); tier 5 the
+// exact pass in LDS up to KD_LDS_MAX entries, and above that a fast and an
+// exact pass in global scratch.
+//
+// q: q.run(k, slot, kernel, threads, args...) launches on side stream k (or
+// KD_MAIN) over a grid of at most n_sets workgroups (slot: the kernel's place
+// among the grids that q keeps), q.run_grid over as many as given; grids are
+// upper bounds, every kernel loops over its own list. q.fork(k, from): side
+// stream k goes on from where the main stream is at fork(from, from);
+// q.joined(k): nothing more on side stream k. Every set is written once all
+// side streams that were joined, and the main stream, are through.
+#define KD_MAIN (-1)
+#define KD_SIDES (KD_TIERS + 1)   // a side stream per tier, and one more for the smallest sets of the largest
+#define KD_GRIDS 13
+constexpr int64_t KD_ONE_STREAM_ATOMS = 16384;
+
+// bucket, tied: KD_TIERS * n_sets each; count: 2 * KD_TIERS
+template <class Q>
+static void kd_launches(Q &q, const DevMols &ms, const DevTpls &tp, const DevSets &st, unsigned char *scr, int *bucket,
+                        int *tied, unsigned int *count, bool one_molecule, int64_t n_atoms)
+{
+    typedef const int *List;
+    typedef const unsigned int *Count;
+    const size_t ns = (size_t)st.n_sets;
+    unsigned int *nb = count, *nt = count + KD_TIERS;
+    // the passes over `list` (every set where there is none) of the sets beyond
+    // KD_BIG entries, by size
+    auto lds2 = [&](int k, List list, Count n) { q.run(k, 9, k_kdexact_lds<1024, 2>, 1024, ms, tp, st, list, n, KD_BIG); };
+    auto lds4 = [&](int k, List list, Count n) {
+        q.run(k, 10, k_kdexact_lds<1024, 4>, 1024, ms, tp, st, list, n, KD_LDS_MAX / 4);
+    };
+    auto lds8 = [&](int k, List list, Count n) {
+        q.run(k, 11, k_kdexact_lds<1024, 8>, 1024, ms, tp, st, list, n, KD_LDS_MAX / 2);
+    };
+    auto big_fast = [&](int k, List list, Count n, int *out, unsigned int *n_out) {
+        q.run(k, 2, k_kdbig, KD_THREADS, ms, tp, st, scr, list, n, out, n_out, KD_LDS_MAX);
+    };
+    auto big_exact = [&](int k, List list, Count n) {
+        q.run(k, 12, k_kdbig_exact, KD_EXACT_THREADS, ms, tp, st, scr, list, n, KD_LDS_MAX);
+    };
+    static_assert(KD_LDS_MAX == 8 * 1024, "the sizes of the LDS passes");
+    if (one_molecule) {
+        if (n_atoms > KD_BIG) {
+            const bool spread = n_atoms > KD_ONE_STREAM_ATOMS;
+            for (int k = 5; k >= (spread ? 3 : 5); k--) q.fork(k, 5);
+            lds8(5, nullptr, nullptr);
+            lds4(spread ? 4 : 5, nullptr, nullptr);
+            lds2(spread ? 3 : 5, nullptr, nullptr);
+            if (n_atoms > KD_LDS_MAX) {
+                int *list = tied + 5 * ns;
+                q.run_grid(5, 1, k_kd_setup, 64, nt + 5, 1);
+                big_fast(5, nullptr, nullptr, list, nt + 5);
+                big_exact(5, list, nt + 5);
+            }
+            for (int k = 5; k >= (spread ? 3 : 5); k--) q.joined(k);
+        }
+        q.run(KD_MAIN, 8, k_kdexact_lds<KD_BIG, 1>, KD_BIG, ms, tp, st, (List)nullptr, (Count)nullptr, 0);
+        return;
+    }
+    q.run_grid(KD_MAIN, 1, k_kd_setup, 64, nb, 2 * KD_TIERS);
+    q.run_grid(KD_MAIN, max(1, min((st.n_sets + KD_BUCKET_SPAN - 1) / KD_BUCKET_SPAN, 1024)), k_kdbucket, 256, st,
+               bucket, nb);
+    // largest tier first: its exact passes, the longest, start earliest
+    for (int k = KD_TIERS - 1; k >= 0; k--) {
+        List all = bucket + (size_t)k * ns;
+        int *list = tied + (size_t)k * ns;
+        Count n_all = nb + k;
+        unsigned int *n_list = nt + k;
+        switch (k) {
+        case 5:
+            big_fast(KD_MAIN, all, n_all, list, n_list);
+            q.fork(5, 5);
+            q.fork(6, 5);
+            lds2(6, all, n_all);
+            q.joined(6);
+            lds8(5, all, n_all);
+            lds4(5, all, n_all);
+            big_exact(5, list, n_list);
+            break;
+        case 4:
+            q.fork(k, k);
+            q.run(k, 7, k_kdexact_lds<512, 2>, 512, ms, tp, st, all, n_all, 0);
+            break;
+        case 3:
+            q.fork(k, k);
+            q.run(k, 6, k_kdexact_lds<256, 2>, 256, ms, tp, st, all, n_all, 0);
+            break;
+        case 2:
+            q.fork(k, k);
+            q.run(k, 5, k_kdexact<256>, 256, ms, tp, st, all, n_all);
+            break;
+        case 1:
+            q.run(KD_MAIN, 1, k_kdblock<128>, 128, ms, tp, st, all, n_all, list, n_list);
+            q.fork(k, k);
+            q.run(k, 4, k_kdexact<128>, 128, ms, tp, st, (List)list, (Count)n_list);
+            break;
+        default:
+            q.run(KD_MAIN, 0, k_kdwave, JAM_WAVE, ms, tp, st, all, n_all, list, n_list);
+            q.fork(k, k);
+            q.run(k, 3, k_kdexact<64>, 64, ms, tp, st, (List)list, (Count)n_list);
+            break;
+        }
+        q.joined(k);
     }
 }
 

@@ -1,10 +1,10 @@
-// Runs the library's kd kernels (pyjess_amd/csrc/jam_kd.h) on the CPU under
-// the HIP emulation of hip/hip_runtime.h, in the order the library launches
-// them (launch_kd in jam_api.hip: bucketing by size tier, then per tier the
-// fast pass and the exact pass over the sets it found tied, or the exact
-// pass over every set of the 513-1024 and 257-512 tiers for one molecule;
-// sets of 1,025-8,192 entries go to the LDS exact pass without a fast pass),
-// and writes each set's kd leaf order. Test infrastructure only.
+// Runs the kd kernels (pyjess_amd/csrc/jam_kd.h) on the CPU under the HIP
+// emulation of hip/hip_runtime.h: bucketing by size tier, then per tier the fast
+// pass and the exact pass over the sets it found tied, or the exact pass over
+// every set of a tier, in template instances from 64 threads up to 1,024, more
+// of them than the library launches (kd_launch_emu.cpp runs the library's own
+// list of launches), and writes each set's kd leaf order. Test infrastructure
+// only.
 //
 //   kd_emu INPUT OUTPUT
 // INPUT: int32 n_sets, int32 one_molecule, int64 off[n_sets + 1],
