@@ -496,6 +496,12 @@ __host__ __device__ constexpr int kd_log2_ceil(int n) { return n <= 1 ? 0 : 1 + 
 // ceil(log2 n) + 1 rounds. Reaching a bound means a broken invariant: the pass
 // stops and reports it instead of looping.
 #define KD_JUMP_BOUND(n) (kd_log2_ceil(n) + 2)
+#ifndef KD_WAVE_ROUNDS
+#define KD_WAVE_ROUNDS JAM_WAVE
+#endif
+#ifndef KD_WAVE_JUMPS
+#define KD_WAVE_JUMPS KD_JUMP_BOUND(JAM_WAVE)
+#endif
 #define KD_ROUND_BOUND(n) ((long long)(n) * (kd_log2_ceil(n) + 2) + 64)
 
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -545,12 +551,15 @@ __device__ static inline int kd_hop(int q, unsigned long long t, int s)
 
 // The QuickSelects of the windows [lw, rw] of a wave, lane = position (rw < 0:
 // no window; lanes of one window agree on lw, rw and K, and are all there),
-// until each has its element K in place. id and v (the key) move along.
-__device__ static inline void kd_wave_select(int &id, double &v, int lw, int rw, int K)
+// until each has its element K in place. id and v (the key) move along. False
+// where a loop bound was reached.
+__device__ static inline bool kd_wave_select(int &id, double &v, int lw, int rw, int K)
 {
     const int lane = lane_id();
+    bool ok = true;
     // every round shortens every open window
-    for (int round = 0; round < JAM_WAVE; round++) {
+    int round = 0;
+    for (; round < KD_WAVE_ROUNDS; round++) {
         const bool open = rw >= 0;
         if (ballot(open) == 0ull) break;
         const int l = open ? lw : lane, r = open ? rw : lane;
@@ -582,11 +591,13 @@ __device__ static inline void kd_wave_select(int &id, double &v, int lw, int rw,
         const int before = lane - l - ones;       // ">" before this lane
         int from = le && before > 0 ? kd_hop(lane, L << (JAM_WAVE - 1 - lane), before) : lane;
         if (lane == r && open) from = pos;
-        for (int jump = 0; jump < KD_JUMP_BOUND(JAM_WAVE); jump++) {
+        int jump = 0;
+        for (; jump < KD_WAVE_JUMPS; jump++) {
             from = __shfl(from, from, JAM_WAVE);
             from = __shfl(from, from, JAM_WAVE);
             if (ballot(open && lane > pos && lane <= r && ((G >> from) & 1ull) == 0ull) == 0ull) break;
         }
+        ok &= jump < KD_WAVE_JUMPS;
         int src = lane < pos ? part : (lane == pos ? r : from);
         src = src == piv ? r : (src == r ? piv : src);
         if (!(open && lane >= l && lane <= r)) src = lane;
@@ -600,12 +611,14 @@ __device__ static inline void kd_wave_select(int &id, double &v, int lw, int rw,
             if (rw >= 0 && lw == rw) rw = -1;
         }
     }
+    return ok && round < KD_WAVE_ROUNDS;
 }
 
 // The whole subtree of n <= 64 elements whose root splits axis d % 3: lane k
 // holds the element at position k (coordinates c0, c1, c2) and returns the
-// lane that held the element which ends there.
-__device__ static inline int kd_wave_tree(int n, int d, double c0, double c1, double c2)
+// lane that held the element which ends there; ok: false where a loop bound
+// was reached.
+__device__ static inline int kd_wave_tree(int n, int d, double c0, double c1, double c2, bool &ok)
 {
     const int lane = lane_id();
     int id = lane, R = 0, H = n;
@@ -614,7 +627,7 @@ __device__ static inline int kd_wave_tree(int n, int d, double c0, double c1, do
         double v = __shfl(ax == 0 ? c0 : (ax == 1 ? c1 : c2), id, JAM_WAVE);
         const bool open = lane < n && H - R >= 2;
         const int K = R + (H - R) / 2;
-        kd_wave_select(id, v, R, open ? H - 1 : -1, K);
+        ok &= kd_wave_select(id, v, R, open ? H - 1 : -1, K);
         if (open) {
             if (lane < K) H = K;
             else R = K;
@@ -825,7 +838,7 @@ __device__ static inline int kd_exact_set(const DevMols &ms, const DevSets &st, 
                 const bool in = p <= r;
                 int e = in ? (int)S.xa[cur][p] : 0;
                 double v = in ? c[e] : 0.0;
-                kd_wave_select(e, v, 0, in ? r - l : -1, K - l);
+                if (!kd_wave_select(e, v, 0, in ? r - l : -1, K - l) && lane == 0) atomicOr(st.kd_err, 1u);
                 if (in) S.xa[cur][p] = (unsigned short)e;
             }
             __syncthreads();
@@ -865,7 +878,9 @@ __device__ static inline int kd_exact_set(const DevMols &ms, const DevSets &st, 
                 for (int q = 0; q < 3; q++) x[q] = ms.xyz[3 * g + q];
             }
         }
-        const int id = kd_wave_tree(m, d, x[0], x[1], x[2]);
+        bool ok = true;
+        const int id = kd_wave_tree(m, d, x[0], x[1], x[2], ok);
+        if (!ok && lane == 0) atomicOr(st.kd_err, 1u);
         e = shfl_int(e, id);
         if (lane < m) S.xa[cur][lo + lane] = (unsigned short)e;
     }

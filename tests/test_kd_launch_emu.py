@@ -81,3 +81,15 @@ def test_batch(tmp_path):
 def test_one_molecule(tmp_path):
     launches = check(build("kd_launch_emu"), selection((9, 65, 513, 1025)), True, tmp_path)
     assert [slot for _, slot, _ in launches if slot >= 0][-1] == 8
+
+
+@pytest.mark.parametrize("bound", ["kd_bound_rounds", "kd_bound_jumps"])
+@pytest.mark.parametrize("one_molecule", [False, True])
+@pytest.mark.parametrize("n", [33, 129])
+def test_a_bound_that_is_reached_is_reported(tmp_path, bound, one_molecule, n):
+    """With bounds too low for any set, the waves that finish small windows (129
+    entries) and whole subtrees (33) end and set the error word."""
+    _, off, q, _ = vectors()
+    i = next(i for i in selection((n,)) if off[i + 1] - off[i] == n)
+    _, kd_err, _ = run(build(bound), [q[off[i]:off[i + 1]].astype(np.float64) / 8.0], one_molecule, tmp_path)
+    assert kd_err != 0
