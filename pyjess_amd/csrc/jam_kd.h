@@ -1497,12 +1497,22 @@ static void kd_launches(Q &q, const DevMols &ms, const DevTpls &tp, const DevSet
     };
     static_assert(KD_LDS_MAX == 8 * 1024, "the sizes of the LDS passes");
     if (one_molecule) {
-        if (n_atoms > KD_BIG) {
-            const bool spread = n_atoms > KD_ONE_STREAM_ATOMS;
+        // the side streams start before the main stream's pass, which is the
+        // longest, and goes first, where sets as large as theirs are odd ones
+        const bool sides = n_atoms > KD_BIG, spread = n_atoms > KD_ONE_STREAM_ATOMS;
+        auto main_pass = [&] {
+            q.run(KD_MAIN, 8, k_kdexact_lds<KD_BIG, 1>, KD_BIG, ms, tp, st, (List)nullptr, (Count)nullptr, 0);
+        };
+        if (sides)
             for (int k = 5; k >= (spread ? 3 : 5); k--) q.fork(k, 5);
+        if (!spread) main_pass();
+        if (sides) {
             lds8(5, nullptr, nullptr);
             lds4(spread ? 4 : 5, nullptr, nullptr);
             lds2(spread ? 3 : 5, nullptr, nullptr);
+        }
+        if (spread) main_pass();
+        if (sides) {
             if (n_atoms > KD_LDS_MAX) {
                 int *list = tied + 5 * ns;
                 q.run_grid(5, 1, k_kd_setup, 64, nt + 5, 1);
@@ -1511,7 +1521,6 @@ static void kd_launches(Q &q, const DevMols &ms, const DevTpls &tp, const DevSet
             }
             for (int k = 5; k >= (spread ? 3 : 5); k--) q.joined(k);
         }
-        q.run(KD_MAIN, 8, k_kdexact_lds<KD_BIG, 1>, KD_BIG, ms, tp, st, (List)nullptr, (Count)nullptr, 0);
         return;
     }
     q.run_grid(KD_MAIN, 1, k_kd_setup, 64, nb, 2 * KD_TIERS);
