@@ -1852,9 +1852,7 @@ int32_t sort_groups(jam_context *c, const DevSets &st, const DevTpls &dt, const 
         hipLaunchKernelGGL(jam::k_group_list, dim3(gs), dim3(256), 0, s, c->sg_seg[0].as<const jam::GroupSeg>(),
                            (long long)n_done, least, list, n_list);
     if (rank_all || most >= (unsigned long long)least) {
-        // passes: key words when every level takes `bits` bits (an upper bound)
-        const int per = 64 / bits, first = (64 - shift) / bits;
-        const int words = 1 + std::max(0, (stride - 1 - first + per - 1) / per);
+        const int words = jam::group_passes(stride, shift, bits);
         const unsigned waves = (unsigned)std::min<int64_t>(8192, (n_done + 3) / 4);
         int cur = 0;
         for (int w = 0; w < words; w++, cur ^= 1)

@@ -1018,6 +1018,14 @@ __global__ void __launch_bounds__(256) k_group_list(const GroupSeg *seg, long lo
     if (listed) list[base + rank_below(m)] = (int)d;
 }
 
+// Passes of k_group_rank: the key words of `stride` levels where every level
+// takes `bits` bits (an upper bound), the first `shift` bits being the row's.
+inline int group_passes(int stride, int shift, int bits)
+{
+    const int per = 64 / bits, first = (64 - shift) / bits;
+    return 1 + (stride - 1 > first ? (stride - 1 - first + per - 1) / per : 0);
+}
+
 // One pass over the key words of the matches at the listed positions (all of
 // them without a list; the positions of a group stay its own from pass to
 // pass): a match's position is its group's start, plus the smaller words, plus
