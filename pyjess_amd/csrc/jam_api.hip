@@ -1609,10 +1609,12 @@ __global__ void k_zero_u64(unsigned long long *v, long long n)
 // group_work_max of them the radix passes are faster (470,000 matches of a
 // 100,000-atom assembly, 28 M in large groups: 0.56 ms against 1.7 ms by radix
 // passes; 6.3 M matches, 550 M in large groups: 3.2 against 2.4 ms). More than
-// GROUP_MATCHES_MAX matches go by radix passes at once: so many come from
-// symmetric templates, whose groups are large, and finding that out costs 0.3
-// ms for 6.3 M matches and 2.5 ms for the 51 M of 16 assemblies x 7,000
-// templates.
+// GROUP_MATCHES_MAX matches go by radix passes at once, although not all of
+// them have large groups: finding out costs 0.3 ms for 6.3 M matches and 2.5 ms
+// for the 51 M of 16 assemblies x 7,000 symmetric templates, in vain where the
+// groups are large; where they are small it would gain 0.3 to 0.5 ms of 3.8 to
+// 5.6 ms (sort and superposition of 5.1 to 6.1 M matches, 8 to 1,024 to a group:
+// 3.4 against 3.8, 4.4 against 4.7, 4.8 against 5.3 ms).
 #ifndef GROUP_RANK_WORK
 #define GROUP_RANK_WORK 8000000ull
 #endif

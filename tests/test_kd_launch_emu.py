@@ -84,9 +84,8 @@ def test_one_molecule(tmp_path):
 
 
 @pytest.mark.parametrize("bound", ["kd_bound_rounds", "kd_bound_jumps"])
-@pytest.mark.parametrize("one_molecule", [False, True])
-@pytest.mark.parametrize("n", [33, 129])
-def test_a_bound_that_is_reached_is_reported(tmp_path, bound, one_molecule, n):
+@pytest.mark.parametrize("n,one_molecule", [(33, False), (129, True)])
+def test_a_bound_that_is_reached_is_reported(tmp_path, bound, n, one_molecule):
     """With bounds too low for any set, the waves that finish small windows (129
     entries) and whole subtrees (33) end and set the error word."""
     _, off, q, _ = vectors()
