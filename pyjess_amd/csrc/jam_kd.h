@@ -552,14 +552,14 @@ __device__ static inline int kd_hop(int q, unsigned long long t, int s)
 // The QuickSelects of the windows [lw, rw] of a wave, lane = position (rw < 0:
 // no window; lanes of one window agree on lw, rw and K, and are all there),
 // until each has its element K in place. id and v (the key) move along. False
-// where a loop bound was reached.
+// where a window is left open, at the bound of the rounds; where a chain of the
+// queue is not followed to its end, at the bound of the jumps, a lane's element
+// is taken twice (kd_wave_whole).
 __device__ static inline bool kd_wave_select(int &id, double &v, int lw, int rw, int K)
 {
     const int lane = lane_id();
-    bool ok = true;
     // every round shortens every open window
-    int round = 0;
-    for (; round < KD_WAVE_ROUNDS; round++) {
+    for (int round = 0; round < KD_WAVE_ROUNDS; round++) {
         const bool open = rw >= 0;
         if (ballot(open) == 0ull) break;
         const int l = open ? lw : lane, r = open ? rw : lane;
@@ -591,13 +591,11 @@ __device__ static inline bool kd_wave_select(int &id, double &v, int lw, int rw,
         const int before = lane - l - ones;       // ">" before this lane
         int from = le && before > 0 ? kd_hop(lane, L << (JAM_WAVE - 1 - lane), before) : lane;
         if (lane == r && open) from = pos;
-        int jump = 0;
-        for (; jump < KD_WAVE_JUMPS; jump++) {
+        for (int jump = 0; jump < KD_WAVE_JUMPS; jump++) {
             from = __shfl(from, from, JAM_WAVE);
             from = __shfl(from, from, JAM_WAVE);
             if (ballot(open && lane > pos && lane <= r && ((G >> from) & 1ull) == 0ull) == 0ull) break;
         }
-        ok &= jump < KD_WAVE_JUMPS;
         int src = lane < pos ? part : (lane == pos ? r : from);
         src = src == piv ? r : (src == r ? piv : src);
         if (!(open && lane >= l && lane <= r)) src = lane;
@@ -611,8 +609,11 @@ __device__ static inline bool kd_wave_select(int &id, double &v, int lw, int rw,
             if (rw >= 0 && lw == rw) rw = -1;
         }
     }
-    return ok && round < KD_WAVE_ROUNDS;
+    return ballot(rw >= 0) == 0ull;
 }
+
+// Whether id, which the selects moved, still names every lane once.
+__device__ static inline bool kd_wave_whole(int id) { return ballot(push_int(1, id) != 1) == 0ull; }
 
 // The whole subtree of n <= 64 elements whose root splits axis d % 3: lane k
 // holds the element at position k (coordinates c0, c1, c2) and returns the
@@ -633,6 +634,7 @@ __device__ static inline int kd_wave_tree(int n, int d, double c0, double c1, do
             else R = K;
         }
     }
+    ok &= kd_wave_whole(id);
     return id;
 }
 
@@ -836,9 +838,11 @@ __device__ static inline int kd_exact_set(const DevMols &ms, const DevSets &st, 
                 const int K = lo + (hi - lo) / 2;
                 const int p = l + lane;
                 const bool in = p <= r;
-                int e = in ? (int)S.xa[cur][p] : 0;
+                int e = in ? (int)S.xa[cur][p] : 0, id = lane;
                 double v = in ? c[e] : 0.0;
-                if (!kd_wave_select(e, v, 0, in ? r - l : -1, K - l) && lane == 0) atomicOr(st.kd_err, 1u);
+                const bool closed = kd_wave_select(id, v, 0, in ? r - l : -1, K - l);
+                if (!(kd_wave_whole(id) && closed) && lane == 0) atomicOr(st.kd_err, 1u);
+                e = shfl_int(e, id);
                 if (in) S.xa[cur][p] = (unsigned short)e;
             }
             __syncthreads();
