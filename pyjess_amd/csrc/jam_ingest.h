@@ -518,28 +518,27 @@ __global__ void __launch_bounds__(ING_THREADS) k_run_order(const int *atom_off, 
     order[at] = (int)a - a0;
 }
 
-// Sort key of every atom: its text, then its serial number, which a stable
+// Sort key of every atom: its molecule, then its serial number, which a stable
 // sort orders as k_residue_index visits atoms whose serial numbers descend
-// somewhere; the value is the atom's index.
-__global__ void __launch_bounds__(ING_THREADS) k_ing_sortkeys(long long n_atoms, const long long *atom_line,
-                                                             const int *text_of, const int *serial,
-                                                             unsigned long long *key, int *val)
+// at many places; the value is the atom's index.
+__global__ void __launch_bounds__(ING_THREADS) k_serial_keys(const int *atom_off, int n_mols, const int *serial,
+                                                            unsigned long long *key, int *val)
 {
     const long long a = (long long)blockIdx.x * ING_THREADS + threadIdx.x;
-    if (a >= n_atoms) return;
-    key[a] = ((unsigned long long)(unsigned int)text_of[atom_line[a]] << 32) | ((unsigned int)serial[a] ^ 0x80000000u);
+    if (a >= atom_off[n_mols]) return;
+    key[a] = ((unsigned long long)(unsigned int)molecule_of(atom_off, n_mols, a) << 32) |
+             ((unsigned int)serial[a] ^ 0x80000000u);
     val[a] = (int)a;
 }
 
-// order[i]: the molecule-local index of the i-th sorted atom (a text's atoms
+// order[i]: the molecule-local index of the i-th sorted atom (a molecule's atoms
 // keep its positions)
-__global__ void __launch_bounds__(ING_THREADS) k_ing_order(long long n_atoms, const int *sorted, const int *atom_off,
-                                                          const long long *atom_line, const int *text_of, int *order)
+__global__ void __launch_bounds__(ING_THREADS) k_sorted_order(const int *atom_off, int n_mols, const int *sorted,
+                                                             int *order)
 {
     const long long i = (long long)blockIdx.x * ING_THREADS + threadIdx.x;
-    if (i >= n_atoms) return;
-    const int a = sorted[i];
-    order[i] = a - atom_off[text_of[atom_line[a]]];
+    if (i >= atom_off[n_mols]) return;
+    order[i] = sorted[i] - atom_off[molecule_of(atom_off, n_mols, i)];
 }
 
 // out[k] = (int)in[k]

@@ -65,13 +65,14 @@ def test_texts(downs):
     assert np.array_equal(perm, np.concatenate([m.index()[0] for m in mols]))
 
 
-def test_upload_time():
-    """A wrap costs an upload little: the order is not sorted on the host."""
-    n = 400000
+@pytest.mark.parametrize("n,down", [(400000, "wrapped"), (100000, "reversed")])
+def test_upload_time(n, down):
+    """Serial numbers that descend cost an upload little: nothing is sorted on
+    the host."""
     times = []
-    for wrap in (n, 99999):
+    for serial in (np.arange(n), np.arange(n) % 99999 if down == "wrapped" else np.arange(n, 0, -1)):
         m = Arrays(np.random.default_rng(1), n, 21, "ascending")
-        m.serial = (np.arange(n) % wrap).astype(np.int32)
+        m.serial = serial.astype(np.int32)
         best = float("inf")
         for _ in range(5):
             t0 = time.perf_counter()
