@@ -487,7 +487,7 @@ __global__ void __launch_bounds__(ING_THREADS) k_run_order(const int *atom_off, 
     int k0 = 0, k1;
     while (k0 < n_down && first[k0] <= a0) k0++;
     for (k1 = k0; k1 < n_down && first[k1] < a1;) k1++;
-    int at = a0;
+    unsigned at = (unsigned)a0;   // (sums of places, which pass the range of an int)
     for (int r0 = k0; r0 <= k1; r0 += RUN_CHAINS) {
         int x[RUN_CHAINS], y[RUN_CHAINS];
         bool upto[RUN_CHAINS];   // an earlier run counts up to s, a later one below s
@@ -498,7 +498,7 @@ __global__ void __launch_bounds__(ING_THREADS) k_run_order(const int *atom_off, 
             upto[u] = begin <= a;
             x[u] = begin;
             y[u] = end;
-            at -= begin;
+            at -= (unsigned)begin;
             if (a >= begin && a < end) x[u] = y[u] = (int)a;
         }
         for (bool more = true; more;) {
@@ -506,14 +506,14 @@ __global__ void __launch_bounds__(ING_THREADS) k_run_order(const int *atom_off, 
 #pragma unroll
             for (int u = 0; u < RUN_CHAINS; u++) {
                 if (x[u] >= y[u]) continue;
-                const int mid = (x[u] + y[u]) >> 1, v = serial[mid];
+                const int mid = x[u] + ((y[u] - x[u]) >> 1), v = serial[mid];
                 if (upto[u] ? v <= s : v < s) x[u] = mid + 1;
                 else y[u] = mid;
                 more = true;
             }
         }
 #pragma unroll
-        for (int u = 0; u < RUN_CHAINS; u++) at += x[u];
+        for (int u = 0; u < RUN_CHAINS; u++) at += (unsigned)x[u];
     }
     order[at] = (int)a - a0;
 }
