@@ -31,7 +31,7 @@
 //          seldom have a tie (up to 128 entries of many molecules, and those
 //          too large for LDS unless a sample of them has one) try the fast path first.
 //
-// Fast path: sets of up to 64 entries in one wave's registers, up to KD_BIG
+// Fast path: sets of up to 64 entries in one wave's registers, up to 128
 // with one position per thread, above KD_LDS_MAX in global scratch. Exact
 // path: up to KD_LDS_MAX entries in LDS, larger ones in global scratch. Every
 // loop of an exact pass whose length depends on the data has a bound that a
@@ -51,10 +51,10 @@ namespace jam {
 #ifndef KD_THREADS
 #define KD_THREADS 256
 #endif
-// threads of the exact pass over a set larger than KD_BIG: its rounds are
+// threads of the exact pass over a set larger than KD_LDS_MAX: its rounds are
 // latency-bound loops over the positions, so more threads per set
 #define KD_EXACT_THREADS 1024
-// global scratch of sets larger than KD_BIG, per set entry (padded to a power
+// global scratch of sets larger than KD_LDS_MAX, per set entry (padded to a power
 // of two for the fast path's sorts: 3 doubles, 9 ints and 1 byte per padded
 // entry, at most 2 * 61 bytes per entry)
 #define KD_SCRATCH_BYTES_PER_ENTRY 128
